@@ -1339,7 +1339,7 @@ int glm53_grouped_linear(const void* x, int64_t act_rows, const int32_t* row_ind
   g.N = N;
   g.out = static_cast<uint16_t*>(y);
   g.out_row_stride = N;
-  HIP_TRY(launch_grouped_gemm(g, GEMM_PLAIN, descriptors, st), "grouped gemm launch");
+  HIP_TRY(launch_grouped_linear(g, descriptors, st), "grouped gemm launch");
   return GLM53_OK;
 }
 

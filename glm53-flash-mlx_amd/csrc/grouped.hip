@@ -843,15 +843,14 @@ __device__ __forceinline__ void load_activation_scales(const ItemSource& src, in
   }
 }
 
+// routes start .. start + len - 1 (len <= 32 GPW) of one expert x column tile ntile
 template <int MODE, bool FIX, int GPW>
-__device__ __forceinline__ void grouped_gemm_body(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile, int64_t d,
-                                                  uint8_t* lds) {
-  constexpr int kRoutes = 32 * GPW;  // routes per descriptor
+__device__ __forceinline__ void grouped_gemm_part(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
+                                                  int32_t expert, int32_t start, int32_t len, uint8_t* lds) {
+  constexpr int kRoutes = 32 * GPW;
   constexpr int kStage = stage_bytes<GPW>();
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  int32_t expert, start, len;
-  if (!item_routes<kRoutes>(src, d, expert, start, len)) return;
   const int64_t K = a.K;
   const int64_t KB = K / kBlock;
   const int pairs = (len + 15) >> 4;
@@ -912,6 +911,14 @@ __device__ __forceinline__ void grouped_gemm_body(const GroupedGemmArgs& a, cons
   if (active) GLM53_LOOP(1);
   else GLM53_LOOP(0);
 #undef GLM53_LOOP
+}
+
+template <int MODE, bool FIX, int GPW>
+__device__ __forceinline__ void grouped_gemm_body(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile, int64_t d,
+                                                  uint8_t* lds) {
+  int32_t expert, start, len;
+  if (!item_routes<32 * GPW>(src, d, expert, start, len)) return;
+  grouped_gemm_part<MODE, FIX, GPW>(a, src, ntile, expert, start, len, lds);
 }
 
 template <int GPW>
@@ -1008,6 +1015,32 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedGemmArgs a) {
   const ItemSource src = item_source(a, used, w, true, ntile, d, fix);
   if (fix) grouped_gemm_body<MODE, true, GPW>(a, src, ntile, d, lds_dyn);
   else grouped_gemm_body<MODE, false, GPW>(a, src, ntile, d, lds_dyn);
+}
+
+// The 32-route shape over a caller's own descriptors (glm53_grouped_linear):
+// a descriptor of up to kGemmTileRows routes runs in 32-route parts (one for
+// the tile plan's descriptors, which hold at most 32, so the 64-route shape
+// would carry half its activation rows empty and stream the weights through
+// shallower direct loads).  Bound by the weight stream: 4,096 routes over
+// 288 experts, [4096 x 4096] and [4096 x 2048] in one chain of building
+// blocks, 2,800 -> 2,612 us for the whole chain against the 64-route shape.
+__global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
+  const int64_t items = a.n_tiles * a.descriptors;
+  const int64_t per_xcd = (items + 7) / 8;
+  const int64_t w = static_cast<int64_t>(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (w >= items) return;
+  int64_t ntile, d;
+  bool fix;
+  const ItemSource src = item_source(a, a.descriptors, w, true, ntile, d, fix);
+  int32_t expert, start, len;
+  if (!item_routes<kGemmTileRows>(src, d, expert, start, len)) return;
+  for (int32_t done = 0; done < len; done += kGemmMinTileRows) {
+    if (done > 0) __syncthreads();  // every wavefront has read the part before out of LDS
+    const int32_t part = len - done < kGemmMinTileRows ? len - done : kGemmMinTileRows;
+    if (fix) grouped_gemm_part<GEMM_PLAIN, true, 1>(a, src, ntile, expert, start + done, part, lds_dyn);
+    else grouped_gemm_part<GEMM_PLAIN, false, 1>(a, src, ntile, expert, start + done, part, lds_dyn);
+  }
 }
 
 // ------------------------------------------ grouped GEMM, wide shape --
@@ -1591,6 +1624,19 @@ hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descr
     else GLM53_GEMM(GEMM_SWIGLU, 2);
   }
 #undef GLM53_GEMM
+  return hipGetLastError();
+}
+
+hipError_t launch_grouped_linear(const GroupedGemmArgs& a, int64_t descriptors, hipStream_t st) {
+  if (descriptors == 0) return hipSuccess;
+  if (a.out_row_stride < a.N || a.out_row_stride >= (int64_t{1} << 22)) return hipErrorInvalidValue;
+  GroupedGemmArgs g = a;
+  g.n_tiles = (a.N + kTileRows - 1) / kTileRows;
+  g.descriptors = descriptors;
+  const unsigned grid = static_cast<unsigned>(8 * ((g.n_tiles * descriptors + 7) / 8));
+  const size_t lds = gemm_lds_bytes<1>(a.K);
+  if (a.K % kBlock != 0 || a.K <= 0 || lds > 160 * 1024) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(grouped_linear_kernel, dim3(grid), dim3(256), lds, st, g);
   return hipGetLastError();
 }
 

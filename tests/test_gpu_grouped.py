@@ -142,6 +142,36 @@ def test_grouped_linear_matches_oracle(M, O, dev):
     assert np.array_equal(to_bits(out), want_out)
 
 
+@pytest.mark.parametrize("tile_rows", [32, 64])
+@pytest.mark.parametrize("n", [128, 144])
+def test_grouped_linear_callers_descriptors_of_up_to_64_routes(M, O, dev, tile_rows, n):
+    """Descriptors of 1 .. 64 routes built by the caller: one of more than 32
+    runs as 32-route parts, every route with the same arithmetic; the last
+    column tile is ragged for n = 144."""
+    import torch
+
+    rng = np.random.default_rng(100 * tile_rows + n)
+    counts = [1, 16, 31, 32, 33, 63, 64, 0, 100]
+    experts, k = len(counts), 256
+    sorted_e = np.repeat(np.arange(experts), counts).astype(np.int32)
+    tiles = [(e, sum(counts[:e]) + d, min(tile_rows, c - d)) for e, c in enumerate(counts)
+             for d in range(0, c, tile_rows)]
+    plan = [torch.tensor(v, dtype=torch.int32, device=dev) for v in zip(*tiles)]
+    codes = rng.integers(0, 127, size=(experts, n, k), dtype=np.int64).astype(np.uint8)
+    scale = (rng.uniform(size=(experts, -(-n // 128), k // 128)) * 0.002).astype(np.float32)
+    x = O.f32_to_bf16(rng.normal(size=(sorted_e.size, k)).astype(np.float32))
+    N = submodule("_native")
+    lib = N.lib()
+    w, s, xd = torch.from_numpy(codes).to(dev), torch.from_numpy(scale).to(dev), from_bits(x, dev)
+    y = torch.zeros((sorted_e.size, n), dtype=torch.bfloat16, device=dev)
+    size = lib.glm53_grouped_linear_workspace_bytes(sorted_e.size, k)
+    ws = N.workspace(size, dev)
+    N.check(lib.glm53_grouped_linear(N.ptr(xd), sorted_e.size, None, sorted_e.size, k, *(N.ptr(t) for t in plan),
+                                     plan[0].numel(), N.ptr(w), N.ptr(s), None, experts, n, N.ptr(y), N.ptr(ws), size,
+                                     N.stream_handle(dev)))
+    assert_parity(to_bits(y), O.grouped_linear(x, sorted_e, codes, scale), O, exact_fraction=0.95)
+
+
 def _place(bits, offset, dev):
     """Device BF16 copy of `bits` starting `offset` elements into its buffer
     (offset 1 leaves the rows 2-byte aligned only)."""
