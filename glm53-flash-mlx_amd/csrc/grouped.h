@@ -131,7 +131,8 @@ constexpr int kHcBranches = 4;
 hipError_t launch_route_plan(const RoutePlanArgs& a, hipStream_t st);
 hipError_t launch_split_activations(const SplitArgs& a, hipStream_t st);
 hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descriptors, hipStream_t st);
-// tile_expert / tile_start / tile_len set by the caller; descriptors of up to kGemmTileRows routes
+// tile_expert / tile_start / tile_len set by the caller; descriptors of up to
+// kGemmTileRows routes; fixup null: the items look for 0x7F / 0xFF themselves
 hipError_t launch_grouped_linear(const GroupedGemmArgs& a, int64_t descriptors, hipStream_t st);
 hipError_t launch_reduce(const ReduceArgs& a, bool direct_order, hipStream_t st);
 hipError_t launch_scan_480(const uint8_t* codes, int64_t n, int32_t* flag, bool clear, hipStream_t st);

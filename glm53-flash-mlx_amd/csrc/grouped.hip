@@ -390,6 +390,10 @@ __device__ __forceinline__ void split_480(uint32_t w, uint32_t& fixed, uint32_t&
   corr = (m * 0x60u) | (w & z);                                // +-32 (code 0x60) where fixed
 }
 
+// Bit 7 of each byte set where the code is 0x7F or 0xFF (the other bits are
+// not cleared): a byte's low 7 bits plus 1 reach 0x80 only from 0x7F.
+__device__ __forceinline__ uint32_t codes_480(uint32_t w) { return (w & 0x7F7F7F7Fu) + 0x01010101u; }
+
 namespace {
 
 constexpr int kTileRows = 128;                     // weight rows per work item
@@ -622,12 +626,15 @@ __device__ __forceinline__ void plain_epilogue(const GroupedGemmArgs& a, const I
 // against all 8 tiles, GPW = 1 pair w / 2 against the tiles of half h =
 // w % 2 (PLAIN: tiles 4 h .. 4 h + 3; SWIGLU: gate tiles 2 h, 2 h + 1 and
 // the matching up tiles).
-template <int MODE, bool FIX, int GPW, int NP>
+// DETECT: found collects, in bit 7 of each byte, whether the weight codes the
+// wavefront staged hold 0x7F / 0xFF (codes_480).
+template <int MODE, bool FIX, int GPW, int NP, bool DETECT>
 __device__ __forceinline__ void grouped_gemm_loop(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
                                                   int32_t start, int32_t len, int64_t KB,
                                                   const uint8_t* const (&gb)[2][2], const uint8_t* const (&ga)[GPW][2],
                                                   uint8_t* lds, uint32_t lds_addr, const uint8_t* lds_se,
-                                                  const float* lds_sw, int wave, int lane) {
+                                                  const float* lds_sw, int wave, int lane, uint32_t& found) {
+  static_assert(!DETECT || GPW == 1, "codes are looked at where the weights stream through registers");
   constexpr int kStage = stage_bytes<GPW>();
   constexpr int kRoutes = 32 * GPW;
   constexpr int NL = GPW == 2 ? 2 * NP : NP;  // activation tiles this wavefront loads per stage
@@ -730,6 +737,12 @@ __device__ __forceinline__ void grouped_gemm_loop(const GroupedGemmArgs& a, cons
       }
     };
     auto store = [&](int slot, const Staged& r) {
+      if constexpr (DETECT) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) found |= codes_480(r.b[i][j]);
+      }
       uint8_t* sb = lds + slot * kStage + 2 * wave * kOperand + 16 * lane;
       *reinterpret_cast<u32x4*>(sb) = r.b[0];
       *reinterpret_cast<u32x4*>(sb + 1024) = r.b[1];
@@ -844,9 +857,9 @@ __device__ __forceinline__ void load_activation_scales(const ItemSource& src, in
 }
 
 // routes start .. start + len - 1 (len <= 32 GPW) of one expert x column tile ntile
-template <int MODE, bool FIX, int GPW>
-__device__ __forceinline__ void grouped_gemm_part(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
-                                                  int32_t expert, int32_t start, int32_t len, uint8_t* lds) {
+template <int MODE, bool FIX, int GPW, bool DETECT>
+__device__ __forceinline__ uint32_t grouped_gemm_part(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
+                                                      int32_t expert, int32_t start, int32_t len, uint8_t* lds) {
   constexpr int kRoutes = 32 * GPW;
   constexpr int kStage = stage_bytes<GPW>();
   const int lane = threadIdx.x & 63;
@@ -906,11 +919,14 @@ __device__ __forceinline__ void grouped_gemm_part(const GroupedGemmArgs& a, cons
   }
   const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
   const bool active = (GPW == 2 ? wave : wave >> 1) < pairs;  // wave-uniform: this wavefront's pair holds routes
-#define GLM53_LOOP(n) \
-  grouped_gemm_loop<MODE, FIX, GPW, n>(a, src, ntile, start, len, KB, gb, ga, lds, lds_addr, lds_se, lds_sw, wave, lane)
+  uint32_t found = 0;
+#define GLM53_LOOP(n)                                                                                            \
+  grouped_gemm_loop<MODE, FIX, GPW, n, DETECT>(a, src, ntile, start, len, KB, gb, ga, lds, lds_addr, lds_se, lds_sw, \
+                                               wave, lane, found)
   if (active) GLM53_LOOP(1);
   else GLM53_LOOP(0);
 #undef GLM53_LOOP
+  return found;
 }
 
 template <int MODE, bool FIX, int GPW>
@@ -918,7 +934,7 @@ __device__ __forceinline__ void grouped_gemm_body(const GroupedGemmArgs& a, cons
                                                   uint8_t* lds) {
   int32_t expert, start, len;
   if (!item_routes<32 * GPW>(src, d, expert, start, len)) return;
-  grouped_gemm_part<MODE, FIX, GPW>(a, src, ntile, expert, start, len, lds);
+  grouped_gemm_part<MODE, FIX, GPW, false>(a, src, ntile, expert, start, len, lds);
 }
 
 template <int GPW>
@@ -1017,6 +1033,22 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedGemmArgs a) {
   else grouped_gemm_body<MODE, false, GPW>(a, src, ntile, d, lds_dyn);
 }
 
+// True in every thread when any thread of the workgroup passes true.  Waits
+// for the workgroup's earlier stores, so that what follows may write the
+// same addresses; `lds` is free to be overwritten once all threads are here.
+__device__ __forceinline__ bool workgroup_any(bool mine, uint8_t* lds) {
+  uint32_t* word = reinterpret_cast<uint32_t*>(lds);
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  if (threadIdx.x == 0) *word = 0;
+  __syncthreads();
+  if (mine) atomicOr(word, 1u);
+  __syncthreads();
+  const bool any = *word != 0;
+  __syncthreads();
+  return any;
+}
+
 // The 32-route shape over a caller's own descriptors (glm53_grouped_linear):
 // a descriptor of up to kGemmTileRows routes runs in 32-route parts (one for
 // the tile plan's descriptors, which hold at most 32, so the 64-route shape
@@ -1024,6 +1056,11 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedGemmArgs a) {
 // shallower direct loads).  Bound by the weight stream: 4,096 routes over
 // 288 experts, [4096 x 4096] and [4096 x 2048] in one chain of building
 // blocks, 2,800 -> 2,612 us for the whole chain against the 64-route shape.
+// Weights that come without a code flag (a.fixup null) are looked at as they
+// stream through the registers, 40 VALU instructions per wavefront and stage
+// beside a stage's 8 MFMAs and loads, and an item that met 0x7F / 0xFF runs
+// again in the FIX form; a scan of the bank beforehand read every expert's
+// bytes once more.
 __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
   const int64_t items = a.n_tiles * a.descriptors;
@@ -1038,8 +1075,13 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) 
   for (int32_t done = 0; done < len; done += kGemmMinTileRows) {
     if (done > 0) __syncthreads();  // every wavefront has read the part before out of LDS
     const int32_t part = len - done < kGemmMinTileRows ? len - done : kGemmMinTileRows;
-    if (fix) grouped_gemm_part<GEMM_PLAIN, true, 1>(a, src, ntile, expert, start + done, part, lds_dyn);
-    else grouped_gemm_part<GEMM_PLAIN, false, 1>(a, src, ntile, expert, start + done, part, lds_dyn);
+    if (!fix) {
+      const uint32_t found =
+          grouped_gemm_part<GEMM_PLAIN, false, 1, true>(a, src, ntile, expert, start + done, part, lds_dyn);
+      if (a.fixup == nullptr) fix = workgroup_any((found & 0x80808080u) != 0, lds_dyn);
+      if (!fix) continue;
+    }
+    grouped_gemm_part<GEMM_PLAIN, true, 1, false>(a, src, ntile, expert, start + done, part, lds_dyn);
   }
 }
 

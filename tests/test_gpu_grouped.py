@@ -143,11 +143,13 @@ def test_grouped_linear_matches_oracle(M, O, dev):
 
 
 @pytest.mark.parametrize("tile_rows", [32, 64])
-@pytest.mark.parametrize("n", [128, 144])
-def test_grouped_linear_callers_descriptors_of_up_to_64_routes(M, O, dev, tile_rows, n):
+@pytest.mark.parametrize("n,codes_480", [(128, False), (144, False), (144, True)])
+def test_grouped_linear_callers_descriptors_of_up_to_64_routes(M, O, dev, tile_rows, n, codes_480):
     """Descriptors of 1 .. 64 routes built by the caller: one of more than 32
     runs as 32-route parts, every route with the same arithmetic; the last
-    column tile is ragged for n = 144."""
+    column tile is ragged for n = 144.  Without a code flag the items look for
+    0x7F / 0xFF themselves: one such code in one expert's first or last row,
+    first or last K block, and none in the others."""
     import torch
 
     rng = np.random.default_rng(100 * tile_rows + n)
@@ -158,6 +160,8 @@ def test_grouped_linear_callers_descriptors_of_up_to_64_routes(M, O, dev, tile_r
              for d in range(0, c, tile_rows)]
     plan = [torch.tensor(v, dtype=torch.int32, device=dev) for v in zip(*tiles)]
     codes = rng.integers(0, 127, size=(experts, n, k), dtype=np.int64).astype(np.uint8)
+    if codes_480:
+        codes[2, 0, 0], codes[4, n - 1, k - 1], codes[6, 5, 127], codes[8, 130, 128] = 0x7F, 0xFF, 0xFF, 0x7F
     scale = (rng.uniform(size=(experts, -(-n // 128), k // 128)) * 0.002).astype(np.float32)
     x = O.f32_to_bf16(rng.normal(size=(sorted_e.size, k)).astype(np.float32))
     N = submodule("_native")
