@@ -19,7 +19,7 @@ ROOT = PKG.parent
 CSRC = PKG / "csrc"
 OUT = PKG / "libglm53_moe.so"
 BUILD = PKG / "_build"
-SOURCES = ["decode.hip", "step.hip", "grouped.hip", "router.hip", "layout.hip", "synth.hip", "api.cpp"]
+SOURCES = ["decode.hip", "step.hip", "grouped.hip", "dense.hip", "router.hip", "layout.hip", "synth.hip", "api.cpp"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
@@ -34,10 +34,10 @@ COMMON = [
     "-Wall",
     "-Wno-unused-function",
 ]
-# Per-source additions.  grouped.hip: MFMA results in ordinary VGPRs (the
+# Per-source additions.  grouped.hip, dense.hip: MFMA results in ordinary VGPRs (the
 # compiler otherwise parks the chained hi/lo results of the narrow GEMM in
 # accumulation registers and copies every element out before folding it).
-EXTRA = {"grouped.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+EXTRA = {name: ["-mllvm", "-amdgpu-mfma-vgpr-form"] for name in ("grouped.hip", "dense.hip")}
 
 
 def _compile(src: str) -> Path:

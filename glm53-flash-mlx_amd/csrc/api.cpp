@@ -14,6 +14,7 @@
 #include <string>
 #include <vector>
 
+#include "dense.h"
 #include "grouped.h"
 #include "kernels.h"
 #include "layout.h"
@@ -385,13 +386,29 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
   const size_t need = glm53_fp8_linear_workspace_bytes(M, N, K);
   if (need > 0 && aligned(weight, 16) && workspace != nullptr && workspace_bytes >= need) {
     SplitBuf b = carve_split(workspace, M, K);
+    HIP_TRY(split(x, M, K, b, st), "split launch");
+    const DenseTile tile = dense_tile(M, K, N);
+    if (tile.cols < 128) {
+      DenseArgs d{};
+      d.a_hi = b.hi;
+      d.a_lo = b.lo;
+      d.a_scale = b.scale;
+      d.weight = weight;
+      d.scale = scale_inv;
+      d.flag = code_flags;  // null: the kernel looks for 0x7F / 0xFF itself
+      d.rows = M;
+      d.K = K;
+      d.N = N;
+      d.out = static_cast<uint16_t*>(y);
+      HIP_TRY(launch_dense_linear(d, tile, st), "dense linear launch");
+      return GLM53_OK;
+    }
     const int32_t* flag = code_flags;
     if (flag == nullptr) {
       int32_t* f = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + split_bytes(M, K));
       HIP_TRY(launch_scan_480(weight, N * K, f, true, st), "scan launch");
       flag = f;
     }
-    HIP_TRY(split(x, M, K, b, st), "split launch");
     GroupedGemmArgs g{};
     g.fixup = flag;
     g.a_hi = b.hi;
@@ -404,9 +421,10 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
     g.scale = scale_inv;
     g.s_cols = K / 128;
     g.N = N;
+    g.tile_rows = tile.rows;
     g.out = static_cast<uint16_t*>(y);
     g.out_row_stride = N;
-    HIP_TRY(launch_grouped_gemm(g, GEMM_PLAIN, cdiv(M, kGemmTileRows), st), "grouped gemm launch");
+    HIP_TRY(launch_grouped_gemm(g, GEMM_PLAIN, cdiv(M, tile.rows), st), "grouped gemm launch");
     return GLM53_OK;
   }
   GenericLinearArgs a{};

@@ -1,0 +1,306 @@
+// Dense block-FP8 linear for few rows: y[m, n] = T(sum_k x[m, k] w[n, k]) on
+// the split activations of grouped.hip, the contraction split over the
+// wavefronts of a workgroup.
+#include "common.h"
+#include "dense.h"
+#include "mfma_fp8.h"
+
+namespace glm53 {
+
+namespace {
+
+constexpr int kDenseWaves = 8;
+constexpr int64_t kDenseMaxK = 1 << 18;  // its weight scales take 8 KB of LDS
+template <int V>
+struct Int {
+  static constexpr int value = V;
+};
+
+// K steps (of kDenseWaves blocks) between two folds: their results wait in
+// LDS, 1 KB per block and 16 x 16 output tile.
+template <int P, int C>
+constexpr int fold_steps() {
+  return P * C <= 2 ? 4 : P * C <= 4 ? 2 : 1;
+}
+// K steps a wavefront keeps in flight in registers
+template <int P, int C>
+constexpr int load_depth() {
+  return P * C <= 2 ? 4 : 2;
+}
+// Operand tiles a wavefront passes through its own LDS buffer at a time
+template <int P, int C>
+constexpr int turn_tiles() {
+  return C > 2 * P ? C : 2 * P;
+}
+
+template <int P, int C>
+size_t dense_lds_bytes(int64_t K) {
+  return static_cast<size_t>(kDenseWaves) * (fold_steps<P, C>() * P * C * 1024 + turn_tiles<P, C>() * kOperand) +
+         sizeof(float) * static_cast<size_t>(K / kBlock);
+}
+
+// Rows row0 .. row0 + 16 P - 1 x columns col0 .. col0 + 16 C - 1.  Wavefront w
+// multiplies K blocks w, w + 8, ...: its operands come from global memory
+// into registers (each byte of the item's rows and columns once per
+// workgroup), load_depth steps ahead, 8 rows of whole 128-byte lines per
+// load, and turn into MFMA order through an LDS buffer of its own, so no
+// barrier is waited at in between.  (Loads in MFMA order, 16 rows per load,
+// ran at a third of this rate: neighbouring lanes in different lines.)
+// A block's MFMA results (hi rows, then lo rows, before the weight scale) go
+// to LDS, and wavefront t < P C adds tile t's results in block order, so
+// every output goes through the operations of the grouped GEMM and has its
+// bits.  Returns codes_480 of the weight bytes (DETECT).
+template <int P, int C, bool FIX, bool DETECT>
+__device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_t row0, int64_t col0, uint8_t* lds) {
+  constexpr int D = FIX ? 1 : load_depth<P, C>(), F = FIX ? 1 : fold_steps<P, C>();
+  constexpr int U = D > F ? D : F;  // steps per loop turn: the registers rotate back, folds fall at its end
+  const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+  const int64_t K = a.K;
+  const int KB = static_cast<int>(K / kBlock);
+  const int steps = (KB + kDenseWaves - 1) / kDenseWaves;
+  constexpr int kFold = kDenseWaves * fold_steps<P, C>() * P * C * 1024;
+  f32x4* lds_c = reinterpret_cast<f32x4*>(lds);                                          // [8 F][P C][64]
+  uint8_t* turn = lds + kFold + wave * turn_tiles<P, C>() * kOperand;                    // this wavefront's
+  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * turn_tiles<P, C>() * kOperand);  // [KB]
+  const OperandSlots slots = operand_slots(lane);
+
+  // rows past the last repeat it, columns past the matrix its last row: valid
+  // bytes whose results are never stored (offsets from wave-uniform bases;
+  // the launcher keeps them below 2^32)
+  uint32_t arow[P][2], srow[P], wrow[C][2];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int64_t last = a.rows - 1;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t m = row0 + 16 * p + 8 * h + (lane >> 3);
+      arow[p][h] = static_cast<uint32_t>((m < last ? m : last) * K + load_piece_offset(lane, h));
+    }
+    const int64_t m = row0 + 16 * p + r;
+    srow[p] = static_cast<uint32_t>((m < last ? m : last) * KB);
+  }
+#pragma unroll
+  for (int c = 0; c < C; ++c)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const int64_t n = col0 + 16 * c + 8 * h + (lane >> 3);
+      wrow[c][h] = static_cast<uint32_t>((n < a.N ? n : a.N - 1) * K + load_piece_offset(lane, h));
+    }
+  struct Step {
+    u32x4 b[C][2], h[P][2], l[P][2];
+    float s[P];
+  };
+  auto load = [&](int s, Step& v) {
+    int kb = kDenseWaves * s + wave;
+    kb = kb < KB ? kb : KB - 1;  // past the end: loaded, never folded
+    const int64_t ko = static_cast<int64_t>(kb) * kBlock;  // wave-uniform
+    const uint8_t *w = a.weight + ko, *hi = a.a_hi + ko, *lo = a.a_lo + ko;
+    const float* se = a.a_scale + kb;
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        v.h[p][h] = *reinterpret_cast<const u32x4*>(hi + arow[p][h]);
+        v.l[p][h] = *reinterpret_cast<const u32x4*>(lo + arow[p][h]);
+      }
+      v.s[p] = se[srow[p]];
+    }
+#pragma unroll
+    for (int c = 0; c < C; ++c)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) v.b[c][h] = *reinterpret_cast<const u32x4*>(w + wrow[c][h]);
+  };
+  auto put = [&](int tile, const u32x4 (&v)[2]) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h) *reinterpret_cast<u32x4*>(turn + tile * kOperand + 1024 * h + 16 * lane) = v[h];
+  };
+  // orders the wavefront's own LDS writes and reads (no other wavefront uses the buffer)
+  auto turned = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };
+  Step v[D];
+#pragma unroll
+  for (int d = 0; d < D; ++d)
+    if (d < steps) load(d, v[d]);
+  const float* sw = a.scale + (col0 / kBlock) * KB;  // the item's columns lie in one scale block
+  for (int kb = threadIdx.x; kb < KB; kb += 64 * kDenseWaves) lds_sw[kb] = sw[kb];
+
+  uint32_t found = 0;
+  float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+  auto multiply = [&](int slot, const Step& v) {  // the step's results into slot (block slot of the fold)
+    i32x8 ah[P], al[P], b[C], bc[1];
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      put(2 * p, v.h[p]);
+      put(2 * p + 1, v.l[p]);
+    }
+    turned();
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      ah[p] = lds_operand(turn + 2 * p * kOperand, slots);
+      al[p] = lds_operand(turn + (2 * p + 1) * kOperand, slots);
+    }
+    turned();
+#pragma unroll
+    for (int c = 0; c < C; ++c) put(c, v.b[c]);
+    turned();
+#pragma unroll
+    for (int c = 0; c < C; ++c) b[c] = lds_operand(turn + c * kOperand, slots);
+    turned();
+    if constexpr (DETECT) {
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) found |= codes_480(static_cast<uint32_t>(b[c][i]));
+      asm volatile("" : "+v"(found));  // here, not after the loop with every operand kept
+    }
+    constexpr f32x4 kZero = {0.0f, 0.0f, 0.0f, 0.0f};
+    if constexpr (FIX) {  // one tile at a time: its corrections take another operand's registers
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        weight_operand<FIX>(b[c], bc[0]);
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+          const int e = static_cast<int>(scale_e8m0(v.s[p]));
+          const f32x4 x = pair_pass<FIX, 0, 127>(ah[p], b[c], bc[0], kZero, e);
+          lds_c[(slot * P * C + p * C + c) * 64 + lane] = pair_pass<FIX, 0, 123>(al[p], b[c], bc[0], x, e);
+        }
+      }
+    } else {
+      f32x4 x[P][C];
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          x[p][c] = pair_pass<FIX, 0, 127>(ah[p], b[c], b[c], kZero, static_cast<int>(scale_e8m0(v.s[p])));
+#pragma unroll
+      for (int p = 0; p < P; ++p)
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+          lds_c[(slot * P * C + p * C + c) * 64 + lane] =
+              pair_pass<FIX, 0, 123>(al[p], b[c], b[c], x[p][c], static_cast<int>(scale_e8m0(v.s[p])));
+    }
+  };
+  // adds the results of the K blocks of steps s0 .. s0 + F - 1, in block order
+  auto fold = [&](int s0) {
+    if (wave >= P * C) return;
+    const int first = kDenseWaves * s0;
+    const int count = KB - first < kDenseWaves * F ? KB - first : kDenseWaves * F;
+    const f32x4* mine = lds_c + wave * 64 + lane;
+    int i = 0;
+    for (; i + 8 <= count; i += 8) {
+      f32x4 x[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) x[u] = mine[(i + u) * P * C * 64];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        const float t = lds_sw[first + i + u];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[u][e], t, acc[e]);
+      }
+    }
+    for (; i < count; ++i) {
+      const f32x4 x = mine[i * P * C * 64];
+      const float t = lds_sw[first + i];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[e], t, acc[e]);
+    }
+  };
+  // R steps from s0 on (every register index static); LAST: none follows, so
+  // nothing past them is loaded
+  auto run = [&](auto R, auto LAST, int s0) {
+#pragma unroll
+    for (int f = 0; f < R.value; ++f) {
+      multiply(kDenseWaves * (f % F) + wave, v[0]);
+      __builtin_amdgcn_sched_barrier(0);  // the next loads take the registers this step leaves
+#pragma unroll
+      for (int d = 0; d + 1 < D; ++d) v[d] = v[d + 1];
+      if (!LAST.value || f + D < R.value) load(s0 + f + D, v[D - 1]);
+      if (f % F == F - 1 || f == R.value - 1) {
+        __syncthreads();
+        fold(s0 + f / F * F);
+        if (!LAST.value || f < R.value - 1) __syncthreads();
+      }
+    }
+  };
+  int s0 = 0;
+  for (; s0 + U < steps; s0 += U) run(Int<U>{}, Int<0>{}, s0);
+  switch (steps - s0) {  // 1 .. U
+    case 1: run(Int<1>{}, Int<1>{}, s0); break;
+    case 2: if constexpr (U > 1) run(Int<2>{}, Int<1>{}, s0); break;
+    case 3: if constexpr (U > 2) run(Int<3>{}, Int<1>{}, s0); break;
+    default: if constexpr (U > 2) run(Int<4>{}, Int<1>{}, s0); break;
+  }
+  // lane holds rows 4 kq .. 4 kq + 3, column r of tile `wave`
+  const int64_t n = col0 + 16 * (wave % C) + r;
+  if (wave < P * C && n < a.N) {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int64_t m = row0 + 16 * (wave / C) + 4 * kq + e;
+      if (m < a.rows) a.out[m * a.N + n] = f32_to_bf16(acc[e]);
+    }
+  }
+  return found;
+}
+
+// Workgroup i runs on XCD i % 8; each XCD takes a contiguous run of items,
+// row groups fastest, so the items that share weight columns meet in one L2.
+template <int P, int C>
+__global__ __launch_bounds__(64 * kDenseWaves) void dense_ksplit_kernel(DenseArgs a) {
+  extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
+  const int64_t row_groups = (a.rows + 16 * P - 1) / (16 * P);
+  const int64_t items = row_groups * ((a.N + 16 * C - 1) / (16 * C));
+  const int64_t per_xcd = (items + 7) / 8;
+  const int64_t i = static_cast<int64_t>(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+  if (i >= items) return;
+  const int64_t row0 = 16 * P * (i % row_groups), col0 = 16 * C * (i / row_groups);
+  bool fix = a.flag != nullptr && *a.flag != 0;
+  if (!fix) {
+    const uint32_t found = dense_ksplit_item<P, C, false, true>(a, row0, col0, lds_dyn);
+    if (a.flag == nullptr) fix = workgroup_any((found & 0x80808080u) != 0, lds_dyn);
+  }
+  if (fix) dense_ksplit_item<P, C, true, false>(a, row0, col0, lds_dyn);
+}
+
+template <int P, int C>
+hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
+  const int64_t items = ((a.rows + 16 * P - 1) / (16 * P)) * ((a.N + 16 * C - 1) / (16 * C));
+  const size_t lds = dense_lds_bytes<P, C>(a.K);
+  if (a.K > kDenseMaxK || lds > 160 * 1024) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((dense_ksplit_kernel<P, C>), dim3(static_cast<unsigned>(8 * ((items + 7) / 8))),
+                     dim3(64 * kDenseWaves), lds, st, a);
+  return hipGetLastError();
+}
+
+}  // namespace
+
+// The smallest tile whose items fit one round of a workgroup per CU: a
+// larger tile brings fewer bytes per output but takes longer per round, and
+// a second round costs more than the larger tile does.  Measured (us, N =
+// 4096, K = 4096, each tile at its last one-round row count and just past
+// it): 16 x 16 7.2 at 16 rows, 12.3 at 32, where 16 x 32 takes 8.4; 32 x 32
+// 10.2 at 64 rows, 18.0 at 96, where 32 x 64 takes 13.4; 32 x 64 13.7 at
+// 128, 24.6 at 200; then the grouped GEMM's 32 x 128 (26.5 at 200 rows, 40.3
+// at 300) and 64 x 128 (28.6 at 300; every row count from 2 on before: 22.2
+// at 16, 28.1 at 128).  The narrow tiles' offsets fit 32 bits.
+DenseTile dense_tile(int64_t rows, int64_t K, int64_t N) {
+  constexpr int64_t kComputeUnits = 256;
+  constexpr DenseTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {32, 128}};
+  const bool fits32 = N * K < (int64_t{1} << 32) && rows * K < (int64_t{1} << 32);
+  for (const DenseTile& t : kTiles) {
+    if (t.cols < 128 && (!fits32 || K > kDenseMaxK)) continue;
+    if (((rows + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) <= kComputeUnits) return t;
+  }
+  return {64, 128};
+}
+
+hipError_t launch_dense_linear(const DenseArgs& a, DenseTile t, hipStream_t st) {
+  if (a.rows <= 0 || a.K <= 0 || a.K % kBlock != 0 || a.N <= 0 || a.N % 16 != 0) return hipErrorInvalidValue;
+  if (a.N * a.K >= (int64_t{1} << 32) || a.rows * a.K >= (int64_t{1} << 32)) return hipErrorInvalidValue;
+  if (t.rows == 16 && t.cols == 16) return launch_ksplit<1, 1>(a, st);
+  if (t.rows == 16 && t.cols == 32) return launch_ksplit<1, 2>(a, st);
+  if (t.rows == 32 && t.cols == 32) return launch_ksplit<2, 2>(a, st);
+  if (t.rows == 32 && t.cols == 64) return launch_ksplit<2, 4>(a, st);
+  return hipErrorInvalidValue;
+}
+
+}  // namespace glm53

@@ -96,6 +96,23 @@ def test_multi_row_mfma_path_matches_oracle(M, O, dev, rows):
     assert_parity(got, O.fp8_linear(x, codes, scale), O, exact_fraction=0.97)
 
 
+@pytest.mark.parametrize("with_480", [False, True])
+@pytest.mark.parametrize("rows,k", [(2, 128), (17, 4224), (250, 1152), (499, 1152), (999, 1152), (1999, 640)])
+def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
+    """Row counts that take each output tile of the several-row linear in turn
+    (16 x 16 twice, 16 x 32, 32 x 32, 32 x 64, 32 x 128 at 272 columns), the last row and
+    column tiles ragged, K of 1, 5, 9 and 33 blocks over the 8 wavefronts.
+    Without a code flag a few 0x7F / 0xFF in one tile must be found."""
+    rng = np.random.default_rng(rows + k)
+    n = 272
+    codes = (rng.integers(0, 0x7F, size=(n, k)) | (rng.integers(0, 2, size=(n, k)) << 7)).astype(np.uint8)
+    if with_480:
+        codes[0, 0], codes[n - 1, k - 1], codes[40, 64] = 0x7F, 0xFF, 0xFF
+    scale = (rng.uniform(size=(-(-n // 128), k // 128)) * 0.002).astype(np.float32)
+    x = O.f32_to_bf16(rng.normal(size=(rows, k)).astype(np.float32))
+    assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
+
+
 @pytest.mark.parametrize("rows", [1, 5, 64])
 def test_both_480_codes_gemv_and_mfma(M, O, dev, rows):
     """Codes over the whole byte range, so 0x7F (+480) and 0xFF (-480) both
