@@ -424,7 +424,9 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
     g.tile_rows = tile.rows;
     g.out = static_cast<uint16_t*>(y);
     g.out_row_stride = N;
-    HIP_TRY(launch_grouped_gemm(g, GEMM_PLAIN, cdiv(M, tile.rows), st), "grouped gemm launch");
+    HIP_TRY(tile.rows == kGemmWideRows ? launch_wide_dense(g, static_cast<int>(tile.cols / 128), st)
+                                       : launch_grouped_gemm(g, GEMM_PLAIN, cdiv(M, tile.rows), st),
+            "grouped gemm launch");
     return GLM53_OK;
   }
   GenericLinearArgs a{};

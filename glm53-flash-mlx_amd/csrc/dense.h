@@ -22,7 +22,8 @@ struct DenseTile {
   int rows, cols;
 };
 // The tile for a [rows, K] x [N, K] product: up to 32 x 64 run by
-// launch_dense_linear, larger ones by the grouped GEMM (tile_rows = rows).
+// launch_dense_linear, larger ones by the grouped GEMM (tile_rows = rows;
+// 128 rows: launch_wide_dense with cols / 128 weight tiles per wavefront).
 DenseTile dense_tile(int64_t rows, int64_t K, int64_t N);
 hipError_t launch_dense_linear(const DenseArgs& a, DenseTile tile, hipStream_t st);
 

@@ -3,6 +3,7 @@
 // wavefronts of a workgroup.
 #include "common.h"
 #include "dense.h"
+#include "grouped.h"
 #include "mfma_fp8.h"
 
 namespace glm53 {
@@ -10,6 +11,7 @@ namespace glm53 {
 namespace {
 
 constexpr int kDenseWaves = 8;
+constexpr int64_t kWideDenseMaxK = 1 << 14;  // 128 x 512 items: 128 K blocks of scales beside their stages
 constexpr int64_t kDenseMaxK = 1 << 18;  // its weight scales take 8 KB of LDS
 template <int V>
 struct Int {
@@ -279,18 +281,30 @@ hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
 // 4096, K = 4096, each tile at its last one-round row count and just past
 // it): 16 x 16 7.2 at 16 rows, 12.3 at 32, where 16 x 32 takes 8.4; 32 x 32
 // 10.2 at 64 rows, 18.0 at 96, where 32 x 64 takes 13.4; 32 x 64 13.7 at
-// 128, 24.6 at 200; then the grouped GEMM's 32 x 128 (26.5 at 200 rows, 40.3
-// at 300) and 64 x 128 (28.6 at 300; every row count from 2 on before: 22.2
-// at 16, 28.1 at 128).  The narrow tiles' offsets fit 32 bits.
+// 128, 24.6 at 200; 32 x 128 (grouped GEMM) 26.8 at 200, 40.5 at 300; 64 x
+// 128 29.2 at 300 rows, 34.8 at 512 (256 items, where 128 x 128 takes 32.2:
+// its two workgroups per CU share the load path from about 224 items on);
+// 128 x 128 (wide shape) 37.6 at 1,024, 66.2 at 1,500; 128 x 256 49.0 at
+// 1,500, 58.0 at 2,048, 118 at 4,096; 128 x 512 74.6 at 2,048 and 97.3 at
+// 4,096, one round of the matrix pipes at 2.8 PFLOP/s counting both passes.
+// (64 x 128 took every row count before: 22.2 at 16 rows, 28.1 at 128, 77.3
+// at 2,048, 156 at 4,096.)  The narrow tiles' offsets fit 32 bits, the wide
+// shape's 31.
 DenseTile dense_tile(int64_t rows, int64_t K, int64_t N) {
-  constexpr int64_t kComputeUnits = 256;
-  constexpr DenseTile kTiles[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}, {32, 128}};
-  const bool fits32 = N * K < (int64_t{1} << 32) && rows * K < (int64_t{1} << 32);
-  for (const DenseTile& t : kTiles) {
-    if (t.cols < 128 && (!fits32 || K > kDenseMaxK)) continue;
-    if (((rows + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) <= kComputeUnits) return t;
+  struct Candidate {
+    DenseTile tile;
+    int64_t items;  // at most
+  };
+  constexpr Candidate kTiles[] = {{{16, 16}, 256},  {{16, 32}, 256},  {{32, 32}, 256},   {{32, 64}, 256},
+                                  {{32, 128}, 256}, {{64, 128}, 224}, {{128, 128}, 256}, {{128, 256}, 256}};
+  const bool narrow = K <= kDenseMaxK && N * K < (int64_t{1} << 32) && rows * K < (int64_t{1} << 32);
+  const bool wide = K <= kWideDenseMaxK && wide_offsets_fit(N, K, rows);
+  for (const Candidate& c : kTiles) {
+    const DenseTile t = c.tile;
+    if (t.cols < 128 ? !narrow : t.rows == 128 && !wide) continue;
+    if (((rows + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) <= c.items) return t;
   }
-  return {64, 128};
+  return wide ? DenseTile{128, 512} : DenseTile{64, 128};
 }
 
 hipError_t launch_dense_linear(const DenseArgs& a, DenseTile t, hipStream_t st) {

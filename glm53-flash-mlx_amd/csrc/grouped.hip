@@ -999,10 +999,12 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) 
 // stage start).  Per stage 8 KB of B and 32 KB of A operand reads for 64
 // MFMAs per wavefront.  The arithmetic per output
 // element is that of the narrower shapes, so every shape gives the same
-// bits.
+// bits.  A PLAIN launch may take T = 1 or 2 weight tiles per wavefront
+// instead of 4 (128 or 256 columns per item): a dense linear whose 512-column
+// items would leave CUs without one.
 namespace {
 constexpr int kWidePairs = kGemmWideRows / 16;            // 8
-constexpr int kWideTilesPerWave = 4;                      // weight tiles per wavefront
+constexpr int kWideTilesPerWave = 4;                      // weight tiles per wavefront (T)
 constexpr int kWideBTiles = 8 * kWideTilesPerWave;        // 32 tiles: 512 rows
 constexpr int kWideBBytes = kWideBTiles * kOperand;       // 64 KB
 constexpr int kWideABytes = 2 * kWidePairs * kOperand;    // 32 KB per A stage
@@ -1010,10 +1012,10 @@ constexpr int kWidePlainRows = kWideBTiles * 16;          // 512
 constexpr int kWideGateRows = kWidePlainRows / 2;         // 256
 }  // namespace
 
-size_t gemm_wide_lds_bytes(int64_t K) {
+size_t gemm_wide_lds_bytes(int64_t K, int tiles) {
   // B stage, 2-stage A ring, activation scale codes [KB][128 routes],
   // weight scales [4][KB]
-  return static_cast<size_t>(kWideBBytes + 2 * kWideABytes) +
+  return static_cast<size_t>(8 * tiles * kOperand + 2 * kWideABytes) +
          (kGemmWideRows + 4 * sizeof(float)) * static_cast<size_t>(K / kBlock);
 }
 
@@ -1046,12 +1048,12 @@ __device__ __forceinline__ const uint8_t* uniform_ptr(const uint8_t* p) {
   return reinterpret_cast<const uint8_t*>((static_cast<uint64_t>(hi) << 32) | lo);
 }
 
-template <int MODE, bool FIX, int NP>
+template <int MODE, bool FIX, int NP, int T>
 __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
                                                 int32_t start, int32_t len, int64_t KB, const WideSources& ls,
                                                 bool loads_pair, uint8_t* lds, uint32_t lds_addr, const uint8_t* lds_se,
                                                 const float* lds_sw, int wave, int lane) {
-  constexpr int T = kWideTilesPerWave;
+  constexpr int kBBytes = 8 * T * kOperand;
   const OperandSlots slots = operand_slots(lane);
   const uint32_t b_own = static_cast<uint32_t>(wave) * T * kOperand;  // this wavefront's tiles in the B stage
   auto issue_b = [&](int64_t kb) {
@@ -1072,7 +1074,7 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
   };
   auto issue_a = [&](int64_t kb, int slot) {
     if (loads_pair) {
-      const uint32_t sa = lds_addr + kWideBBytes + slot * kWideABytes + 2 * wave * kOperand;
+      const uint32_t sa = lds_addr + kBBytes + slot * kWideABytes + 2 * wave * kOperand;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         lds_direct16_at(ls.a_hi + kb * kBlock, ls.aoff[h], sa + 1024 * h);
@@ -1083,7 +1085,7 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
   // weight scale row (of lds_sw) of the wavefront's tile q: PLAIN its
   // 64 rows lie in block (64 w) / 128 of the item; SWIGLU gate tiles in
   // gate block (32 w) / 128, up tiles in the same up block
-  const int sw_lo = MODE == GEMM_PLAIN ? (64 * wave) >> 7 : (32 * wave) >> 7;
+  const int sw_lo = MODE == GEMM_PLAIN ? (16 * T * wave) >> 7 : (32 * wave) >> 7;
   const int sw_hi = MODE == GEMM_PLAIN ? sw_lo : 2 + sw_lo;
 
   float acc[NP][T][4];
@@ -1105,8 +1107,8 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
   i32x8 bq[T];
 #pragma unroll
   for (int q = 0; q < T; ++q) bq[q] = lds_operand(lds + b_own + q * kOperand, slots);
-  i32x8 ahi_next = lds_operand(lds + kWideBBytes, slots);
-  i32x8 alo_next = lds_operand(lds + kWideBBytes + kOperand, slots);
+  i32x8 ahi_next = lds_operand(lds + kBBytes, slots);
+  i32x8 alo_next = lds_operand(lds + kBBytes + kOperand, slots);
   int slot = 0;
   for (int64_t kb = 0; kb < KB; ++kb) {
     // the other slot's stage (kb - 1) was read out by every wavefront before
@@ -1127,14 +1129,14 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
     const float w_lo = lds_sw[sw_lo * KB + kb], w_hi = lds_sw[sw_hi * KB + kb];
     // bytes j: the E8M0 scales of this lane's route in pairs j (lo word) and 4 + j (hi word)
     const uint2 se2 = *reinterpret_cast<const uint2*>(lds_se + kb * kGemmWideRows + (lane & 15) * 8);
-    const uint8_t* st = lds + kWideBBytes + slot * kWideABytes;
+    const uint8_t* st = lds + kBBytes + slot * kWideABytes;
     f32x4 c[T];
     auto fold = [&](int j, int q) {
       const float sw = q < 2 ? w_lo : w_hi;
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[j][q][i] = fmaf(c[q][i], sw, acc[j][q][i]);
     };
-    const uint8_t* st_next = lds + kWideBBytes + (slot ^ 1) * kWideABytes;
+    const uint8_t* st_next = lds + kBBytes + (slot ^ 1) * kWideABytes;
     // A operands a whole pair ahead: pair j + 1's hi and lo rows (after the
     // last pair: the next stage's first) are read as pair j's lo pass
     // starts, so each pair's operands have had a whole pair's MFMAs to
@@ -1210,16 +1212,19 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
   }
 
   // epilogue: lane holds columns 16 tile + l % 16 of routes 16 j + 4 kq + i
-  if (MODE == GEMM_PLAIN) {
-    plain_epilogue<NP, T>(a, src, start, len, 0, 1, ntile * kWidePlainRows + 64 * wave, acc, lane);
+  if constexpr (MODE == GEMM_PLAIN) {
+    plain_epilogue<NP, T>(a, src, start, len, 0, 1, ntile * (128 * T) + 16 * T * wave, acc, lane);
   } else {
     swiglu_epilogue<NP, T / 2>(a, src, start, len, 0, 1, ntile * kWideGateRows + 32 * wave, acc, lane);
   }
 }
 
-template <int MODE, bool FIX>
+template <int MODE, bool FIX, int T>
 __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
                                                 int64_t d, uint8_t* lds) {
+  constexpr int kBBytes = 8 * T * kOperand;
+  constexpr int kBlocks = MODE == GEMM_PLAIN ? T : 4;  // weight scale rows of an item
+  static_assert(MODE == GEMM_PLAIN || T == kWideTilesPerWave, "the SwiGLU item is 256 gate and 256 up rows");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   int32_t expert, start, len;
@@ -1227,7 +1232,7 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
   const int64_t K = a.K;
   const int64_t KB = K / kBlock;
   const int pairs = (len + 15) >> 4;
-  uint8_t* lds_se = lds + kWideBBytes + 2 * kWideABytes;                    // [KB][128]
+  uint8_t* lds_se = lds + kBBytes + 2 * kWideABytes;                    // [KB][128]
   float* lds_sw = reinterpret_cast<float*>(lds_se + kGemmWideRows * KB);    // [4][KB]
   auto token_of = [&](int r) -> int64_t {
     const int64_t route = start + (r < len ? r : len - 1);
@@ -1249,10 +1254,10 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
     ls.wg = src.wg;
     const int64_t rows = a.N;
     const int32_t piece = load_piece_offset(lane, 0);
-    const int64_t rlo = MODE == GEMM_PLAIN ? ntile * kWidePlainRows + 64 * wave : ntile * kWideGateRows + 32 * wave;
+    const int64_t rlo = MODE == GEMM_PLAIN ? ntile * (128 * T) + 16 * T * wave : ntile * kWideGateRows + 32 * wave;
     const int64_t rhi = MODE == GEMM_PLAIN ? rlo + 32 : rlo;
 #pragma unroll
-    for (int q = 0; q < kWideTilesPerWave; ++q)
+    for (int q = 0; q < T; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         int64_t u = (q < 2 ? rlo : rhi) + 16 * (q & 1) + 8 * h;
@@ -1268,15 +1273,15 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
   const uint32_t lds_addr = static_cast<uint32_t>(reinterpret_cast<uintptr_t>(lds));
   // stage 0's direct loads fly while the block scales are gathered
   {
-    const uint32_t b_own = static_cast<uint32_t>(wave) * kWideTilesPerWave * kOperand;
+    const uint32_t b_own = static_cast<uint32_t>(wave) * T * kOperand;
 #pragma unroll
-    for (int q = 0; q < kWideTilesPerWave; ++q)
+    for (int q = 0; q < T; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
         lds_direct16_at((q < 2 ? ls.wlo : ls.whi) + ls.wrow[2 * q + h], ls.woff ^ (16 * h),
                         lds_addr + b_own + q * kOperand + 1024 * h);
     if (loads_pair) {
-      const uint32_t sa = lds_addr + kWideBBytes + 2 * wave * kOperand;
+      const uint32_t sa = lds_addr + kBBytes + 2 * wave * kOperand;
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         lds_direct16_at(ls.a_hi, ls.aoff[h], sa + 1024 * h);
@@ -1288,8 +1293,8 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
   // weight scale rows: PLAIN the item's four 128-row blocks; SWIGLU the two
   // blocks its 256 gate rows span, then the same up blocks
   const int64_t srows = (a.N + 127) / 128;
-  const int64_t b0 = MODE == GEMM_PLAIN ? 4 * ntile : 2 * ntile;
-  for (int64_t i = threadIdx.x; i < 4 * KB; i += 512) {
+  const int64_t b0 = MODE == GEMM_PLAIN ? T * ntile : 2 * ntile;
+  for (int64_t i = threadIdx.x; i < kBlocks * KB; i += 512) {
     const int64_t r = i / KB, k = i - r * KB;
     int64_t blk = b0 + (MODE == GEMM_PLAIN ? r : (r & 1));
     blk = blk < srows ? blk : srows - 1;
@@ -1300,7 +1305,7 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
   __syncthreads();
 
 #define GLM53_WIDE(n) \
-  wide_gemm_loop<MODE, FIX, n>(a, src, ntile, start, len, KB, ls, loads_pair, lds, lds_addr, lds_se, lds_sw, wave, lane)
+  wide_gemm_loop<MODE, FIX, n, T>(a, src, ntile, start, len, KB, ls, loads_pair, lds, lds_addr, lds_se, lds_sw, wave, lane)
   // rows past the descriptor's routes (in its last pair) hold stale
   // activations: their products are never stored
   switch (pairs) {
@@ -1316,7 +1321,7 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
 #undef GLM53_WIDE
 }
 
-template <int MODE>
+template <int MODE, int T>
 __global__ __launch_bounds__(512) void grouped_gemm_wide_kernel(GroupedGemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
   const int64_t used = used_descriptors(a);
@@ -1328,8 +1333,8 @@ __global__ __launch_bounds__(512) void grouped_gemm_wide_kernel(GroupedGemmArgs 
   int64_t ntile, d;
   bool fix;
   const ItemSource src = item_source(a, used, w, false, ntile, d, fix);
-  if (fix) wide_gemm_body<MODE, true>(a, src, ntile, d, lds_dyn);
-  else wide_gemm_body<MODE, false>(a, src, ntile, d, lds_dyn);
+  if (fix) wide_gemm_body<MODE, true, T>(a, src, ntile, d, lds_dyn);
+  else wide_gemm_body<MODE, false, T>(a, src, ntile, d, lds_dyn);
 }
 
 // Sets *flag (pre-cleared by clear_flag_kernel) when any byte of codes is
@@ -1529,12 +1534,12 @@ hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descr
     g.descriptors = descriptors;
     const int64_t items = g.n_tiles * (descriptors + g.x_descriptors);
     const unsigned grid = static_cast<unsigned>(8 * ((items + 7) / 8));
-    const size_t lds = gemm_wide_lds_bytes(a.K);
+    const size_t lds = gemm_wide_lds_bytes(a.K, kWideTilesPerWave);
     if (a.K % kBlock != 0 || a.K <= 0 || lds > 160 * 1024) return hipErrorInvalidValue;
     // its direct loads take 32-bit offsets into each matrix and activation plane
     if (!wide_offsets_fit(a.N, a.K, a.routes > a.x_routes ? a.routes : a.x_routes)) return hipErrorInvalidValue;
-    if (mode == GEMM_PLAIN) hipLaunchKernelGGL(grouped_gemm_wide_kernel<GEMM_PLAIN>, dim3(grid), dim3(512), lds, st, g);
-    else hipLaunchKernelGGL(grouped_gemm_wide_kernel<GEMM_SWIGLU>, dim3(grid), dim3(512), lds, st, g);
+    if (mode == GEMM_PLAIN) hipLaunchKernelGGL((grouped_gemm_wide_kernel<GEMM_PLAIN, kWideTilesPerWave>), dim3(grid), dim3(512), lds, st, g);
+    else hipLaunchKernelGGL((grouped_gemm_wide_kernel<GEMM_SWIGLU, kWideTilesPerWave>), dim3(grid), dim3(512), lds, st, g);
     return hipGetLastError();
   }
   GroupedGemmArgs g = a;
@@ -1556,6 +1561,25 @@ hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descr
     else GLM53_GEMM(GEMM_SWIGLU, 2);
   }
 #undef GLM53_GEMM
+  return hipGetLastError();
+}
+
+hipError_t launch_wide_dense(const GroupedGemmArgs& a, int tiles, hipStream_t st) {
+  if (a.out_row_stride < a.N || a.out_row_stride >= (int64_t{1} << 22)) return hipErrorInvalidValue;
+  GroupedGemmArgs g = a;
+  g.n_tiles = (a.N + 128 * tiles - 1) / (128 * tiles);
+  g.descriptors = (a.routes + kGemmWideRows - 1) / kGemmWideRows;
+  const unsigned grid = static_cast<unsigned>(8 * ((g.n_tiles * g.descriptors + 7) / 8));
+  const size_t lds = gemm_wide_lds_bytes(a.K, tiles);
+  if (a.K % kBlock != 0 || a.K <= 0 || lds > 160 * 1024) return hipErrorInvalidValue;
+  if (!wide_offsets_fit(a.N, a.K, a.routes)) return hipErrorInvalidValue;
+#define GLM53_WIDE_DENSE(t) \
+  hipLaunchKernelGGL((grouped_gemm_wide_kernel<GEMM_PLAIN, t>), dim3(grid), dim3(512), lds, st, g)
+  if (tiles == 1) GLM53_WIDE_DENSE(1);
+  else if (tiles == 2) GLM53_WIDE_DENSE(2);
+  else if (tiles == kWideTilesPerWave) GLM53_WIDE_DENSE(kWideTilesPerWave);
+  else return hipErrorInvalidValue;
+#undef GLM53_WIDE_DENSE
   return hipGetLastError();
 }
 

@@ -97,11 +97,13 @@ def test_multi_row_mfma_path_matches_oracle(M, O, dev, rows):
 
 
 @pytest.mark.parametrize("with_480", [False, True])
-@pytest.mark.parametrize("rows,k", [(2, 128), (17, 4224), (250, 1152), (499, 1152), (999, 1152), (1999, 640)])
+@pytest.mark.parametrize("rows,k", [(2, 128), (17, 4224), (250, 1152), (499, 1152), (999, 1152), (1999, 640),
+                                    (2800, 256), (4801, 384), (11000, 128), (16500, 256)])
 def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
     """Row counts that take each output tile of the several-row linear in turn
-    (16 x 16 twice, 16 x 32, 32 x 32, 32 x 64, 32 x 128 at 272 columns), the last row and
-    column tiles ragged, K of 1, 5, 9 and 33 blocks over the 8 wavefronts.
+    (16 x 16 twice, 16 x 32, 32 x 32, 32 x 64, 32 x 128, 64 x 128, 128 x 128, 128 x 256
+    and 128 x 512 at 272 columns), the last row and
+    column tiles ragged, K of 1 to 33 blocks.
     Without a code flag a few 0x7F / 0xFF in one tile must be found."""
     rng = np.random.default_rng(rows + k)
     n = 272
