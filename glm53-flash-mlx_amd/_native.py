@@ -129,6 +129,8 @@ _SIGNATURES = {
     "glm53_prefill_plan_destroy": (None, [P]),
     "glm53_prefill_moe": (ctypes.c_int, [P, P, P, P, P, I64, P, P, I32, P, P]),
     "glm53_prefill_moe_hc": (ctypes.c_int, [P, P, P, P, P, I64, P, P, I32, P, P, P, P, P]),
+    "glm53_prefill_workspace_bytes": (SZ, [I64, I64, I64, I64, I64, I64]),
+    "glm53_prefill_moe_workspace": (ctypes.c_int, [I64, I64, I64, I64, I64, F32, P, P, P, P, I64, I32, P, P, SZ, P]),
     "glm53_prefill_plan_status": (ctypes.c_int, [P, P]),
     "glm53_prefill_plan_scratch": (ctypes.c_int, [P, I32, P, P]),
     "glm53_prefill_plan_counters": (ctypes.c_int, [P, P]),

@@ -1453,10 +1453,12 @@ struct glm53_prefill_plan {
   uint64_t host_syncs = 0;
 };
 
-int glm53_prefill_plan_create(int64_t hidden, int64_t intermediate, int64_t shared_intermediate, int64_t experts,
-                              int64_t top_k, int64_t max_tokens, float swiglu_limit, glm53_prefill_plan** out) {
-  CHECK_ARG(out != nullptr, "out is null");
-  *out = nullptr;
+namespace {
+
+// Checks a prefill's dimensions and fills `p` with them and, once
+// p->arena is set (bind_prefill_arena), with its buffers.
+int init_prefill(glm53_prefill_plan* p, int64_t hidden, int64_t intermediate, int64_t shared_intermediate,
+                 int64_t experts, int64_t top_k, int64_t max_tokens, float swiglu_limit) {
   CHECK_ARG(hidden > 0 && hidden % 128 == 0 && intermediate > 0 && intermediate % 128 == 0,
             "grouped path requires block-aligned projection dimensions; got hidden=%lld, intermediate=%lld",
             (long long)hidden, (long long)intermediate);
@@ -1464,7 +1466,6 @@ int glm53_prefill_plan_create(int64_t hidden, int64_t intermediate, int64_t shar
   CHECK_ARG(experts > 0 && experts <= kPlanMaxExperts, "experts must be in [1, %d]", kPlanMaxExperts);
   CHECK_ARG(top_k > 0 && top_k <= kMaxTopK && top_k <= experts, "top_k must be in [1, %d]", kMaxTopK);
   CHECK_ARG(max_tokens > 0 && max_tokens * top_k < (int64_t(1) << 31), "invalid max_tokens");
-  auto* p = new glm53_prefill_plan();
   p->H = hidden;
   p->I = intermediate;
   p->Is = shared_intermediate;
@@ -1472,7 +1473,14 @@ int glm53_prefill_plan_create(int64_t hidden, int64_t intermediate, int64_t shar
   p->k = top_k;
   p->max_tokens = max_tokens;
   p->limit = swiglu_limit;
-  const int64_t T = max_tokens, R = T * top_k;
+  return GLM53_OK;
+}
+
+// The arena of an initialised prefill: its size in p->arena_bytes and, when
+// p->arena is set, its buffers.
+void bind_prefill_arena(glm53_prefill_plan* p) {
+  const int64_t hidden = p->H, intermediate = p->I, shared_intermediate = p->Is, experts = p->E;
+  const int64_t T = p->max_tokens, R = T * p->k;
   // the separate shared hidden rows (hs) and their split (sq) serve only a
   // shared expert of another width than the routed one: one of the routed
   // width runs merged into the routed buffers (below)
@@ -1501,17 +1509,7 @@ int glm53_prefill_plan_create(int64_t hidden, int64_t intermediate, int64_t shar
   size_t o_h = take(2 * RH * intermediate), o_down = take(2 * R * hidden), o_hs = take(2 * T * Ism);
   size_t o_so = take(2 * T * hidden), o_flags = take(32);
   p->arena_bytes = off;
-  hipError_t e = hipMalloc(&p->arena, off);
-  if (e != hipSuccess) {
-    delete p;
-    return hip_fail(e, "prefill plan hipMalloc");
-  }
-  e = hipMemset(p->arena, 0, off);
-  if (e != hipSuccess) {
-    (void)hipFree(p->arena);
-    delete p;
-    return hip_fail(e, "prefill plan hipMemset");
-  }
+  if (p->arena == nullptr) return;
   uint8_t* b = static_cast<uint8_t*>(p->arena);
   p->router_partial = reinterpret_cast<float*>(b + o_xf);
   p->logits = reinterpret_cast<float*>(b + o_logits);
@@ -1537,6 +1535,31 @@ int glm53_prefill_plan_create(int64_t hidden, int64_t intermediate, int64_t shar
   p->hs = separate_shared ? reinterpret_cast<uint16_t*>(b + o_hs) : nullptr;
   p->shared_out = reinterpret_cast<uint16_t*>(b + o_so);
   p->flags = reinterpret_cast<int32_t*>(b + o_flags);
+}
+
+}  // namespace
+
+int glm53_prefill_plan_create(int64_t hidden, int64_t intermediate, int64_t shared_intermediate, int64_t experts,
+                              int64_t top_k, int64_t max_tokens, float swiglu_limit, glm53_prefill_plan** out) {
+  CHECK_ARG(out != nullptr, "out is null");
+  *out = nullptr;
+  glm53_prefill_plan dims{};
+  if (int rc = init_prefill(&dims, hidden, intermediate, shared_intermediate, experts, top_k, max_tokens, swiglu_limit))
+    return rc;
+  auto* p = new glm53_prefill_plan(dims);
+  bind_prefill_arena(p);
+  hipError_t e = hipMalloc(&p->arena, p->arena_bytes);
+  if (e != hipSuccess) {
+    delete p;
+    return hip_fail(e, "prefill plan hipMalloc");
+  }
+  e = hipMemset(p->arena, 0, p->arena_bytes);
+  if (e != hipSuccess) {
+    (void)hipFree(p->arena);
+    delete p;
+    return hip_fail(e, "prefill plan hipMemset");
+  }
+  bind_prefill_arena(p);
   *out = p;
   return GLM53_OK;
 }
@@ -1798,6 +1821,34 @@ int glm53_prefill_moe_hc(glm53_prefill_plan* p, const glm53_bank* bank, const gl
   CHECK_ARG(tokens == 0 || (residual && post && comb && out_hc), "null pointer argument");
   return prefill_run(p, bank, shared, router, x, tokens, expert_ids, scores, reduction, nullptr, residual, post, comb,
                      out_hc, stream);
+}
+
+size_t glm53_prefill_workspace_bytes(int64_t hidden, int64_t intermediate, int64_t shared_intermediate,
+                                     int64_t experts, int64_t top_k, int64_t tokens) {
+  glm53_prefill_plan p{};
+  if (tokens <= 0 || init_prefill(&p, hidden, intermediate, shared_intermediate, experts, top_k, tokens, 0.0f)) return 0;
+  bind_prefill_arena(&p);
+  return p.arena_bytes;
+}
+
+int glm53_prefill_moe_workspace(int64_t hidden, int64_t intermediate, int64_t shared_intermediate, int64_t experts,
+                                int64_t top_k, float swiglu_limit, const glm53_bank* bank,
+                                const glm53_shared_expert* shared, const glm53_router* router, const void* x,
+                                int64_t tokens, int32_t reduction, void* out, void* workspace, size_t workspace_bytes,
+                                void* stream) {
+  CHECK_ARG(router != nullptr, "router is null");
+  CHECK_ARG(tokens >= 0, "tokens < 0");
+  if (tokens == 0) return GLM53_OK;
+  CHECK_ARG(out != nullptr, "null pointer argument");
+  glm53_prefill_plan p{};
+  if (int rc = init_prefill(&p, hidden, intermediate, shared_intermediate, experts, top_k, tokens, swiglu_limit))
+    return rc;
+  p.arena = workspace;
+  bind_prefill_arena(&p);
+  CHECK_ARG(workspace != nullptr && workspace_bytes >= p.arena_bytes && aligned(workspace, 256),
+            "prefill workspace must be 256-byte aligned and hold %zu bytes", p.arena_bytes);
+  return prefill_run(&p, bank, shared, router, x, tokens, nullptr, nullptr, reduction, out, nullptr, nullptr, nullptr,
+                     nullptr, stream);
 }
 
 int glm53_prefill_plan_status(glm53_prefill_plan* plan, uint32_t* invalid_routes) {

@@ -20,7 +20,7 @@ import torch
 
 from . import _native as N
 from .abi import GROUPED_MIN_ROUTES
-from .fp8 import BLOCK_SIZE
+from .fp8 import BLOCK_SIZE, BlockFP8Linear, ClampedMLP, _scale_shape
 from .packed import PackedFP8MoE, _c_shared
 from .router import Float32Gate
 
@@ -28,6 +28,15 @@ GROUPED_TILE_ROWS = 32
 PLAN_MAX_EXPERTS = 1024  # the route plan's expert bound (kPlanMaxExperts)
 GROUPED_OUTPUT_COLS = 16
 GROUPED_K_TILE = 128
+_DIRECT_PLAN_ROUTES = 4096  # native_direct's scratch stays near 100 MB at H = 4096
+
+
+def _hooked(module) -> bool:
+    """Whether calling `module` would run more than its forward."""
+    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
+                or module._backward_pre_hooks or "forward" in module.__dict__
+                or torch.nn.modules.module._global_forward_hooks
+                or torch.nn.modules.module._global_forward_pre_hooks)
 
 
 def _route_plan(expert_ids: torch.Tensor, scores: torch.Tensor | None, top_k: int, expert_count: int,
@@ -300,6 +309,72 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
         plan.run(self.bank, _c_shared(self.shared_experts), router, flat, tokens, ids, sc, reduction, out, x.device)
         return out.reshape(x.shape)
 
+    def _few_routes_on_device(self, x, tokens: int) -> bool:
+        """Whether a call below min_routes can run as one grouped prefill in
+        the Direct order, which gives the Direct loop's bytes (every route and
+        the shared expert on the same MFMA tree, the same accumulation order):
+        the plan's widths, a plain Float32Gate over the bank's experts, a
+        shared expert whose forward is the plan's (plain block-FP8
+        projections without bias, the layer's limit, no hooks), and buffers
+        that the native call can take by their addresses.  Anything else,
+        traced calls, and batches of over 4,096 routes stay with the loop."""
+        bank, cfg, gate, shared = self.bank, self.config, self.gate, self.shared_experts
+        limit = float(cfg.swiglu_limit)
+        if type(self) is not SortedGroupedFP8MoE or type(gate) is not Float32Gate or _hooked(gate):
+            return False
+        if x.dtype != torch.bfloat16 or x.shape[-1] != bank.hidden_size or torch.compiler.is_compiling():
+            return False
+        if gate.top_k != cfg.num_experts_per_tok or tokens * gate.top_k > _DIRECT_PLAN_ROUTES:
+            return False
+        if bank.hidden_size % BLOCK_SIZE or bank.intermediate_size % BLOCK_SIZE or bank.expert_count > PLAN_MAX_EXPERTS:
+            return False
+        if self._expert_views[0].limit != limit or self._expert_views[0].gate_proj._bank is not bank:
+            return False
+        weights = [bank.gate_up_weight, bank.down_weight]
+        tables = [bank.gate_up_scale_inv, bank.down_scale_inv, gate.weight, gate.e_score_correction_bias]
+        shapes = [(gate.weight, (bank.expert_count, bank.hidden_size)),
+                  (gate.e_score_correction_bias, (bank.expert_count,))]
+        if shared is not None:
+            if type(shared) is not ClampedMLP or _hooked(shared) or shared.limit != limit:
+                return False
+            width = shared.gate_proj.weight.shape[0]
+            if width % BLOCK_SIZE:
+                return False
+            for proj, shape in ((shared.gate_proj, (width, bank.hidden_size)),
+                                (shared.up_proj, (width, bank.hidden_size)),
+                                (shared.down_proj, (bank.hidden_size, width))):
+                if type(proj) is not BlockFP8Linear or _hooked(proj) or proj.bias is not None:
+                    return False
+                weights.append(proj.weight)
+                tables.append(proj.weight_scale_inv)
+                shapes += [(proj.weight, shape), (proj.weight_scale_inv, _scale_shape(*shape))]
+        return (all(t.shape == shape for t, shape in shapes)
+                and all(t.dtype == torch.uint8 and t.data_ptr() % 16 == 0 for t in weights)
+                and all(t.dtype == torch.float32 for t in tables)
+                and all(t.is_contiguous() and t.device == x.device for t in weights + tables))
+
+    def native_direct(self, x):
+        """The native call behind glm53::moe_direct: the grouped prefill in
+        the Direct order for a batch below min_routes, its scratch from
+        torch's allocator for this call alone (nothing is kept between calls,
+        so streams and threads stay independent)."""
+        flat = x.reshape(-1, x.shape[-1]).contiguous()
+        tokens = flat.shape[0]
+        bank, shared, cfg = self.bank, self.shared_experts, self.config
+        width = 0 if shared is None else int(shared.gate_proj.weight.shape[0])
+        dims = (bank.hidden_size, bank.intermediate_size, width, bank.expert_count, cfg.num_experts_per_tok)
+        out = torch.empty_like(flat)
+        lib = N.lib()
+        ws_bytes = lib.glm53_prefill_workspace_bytes(*dims, tokens)
+        ws = N.workspace(ws_bytes, x.device)
+        b, r = bank.as_c_struct(), self.gate.as_c_struct()
+        s = shared.as_c_struct() if shared is not None else None
+        N.check(lib.glm53_prefill_moe_workspace(*dims, float(cfg.swiglu_limit), ctypes.byref(b),
+                                                ctypes.byref(s) if s else None, ctypes.byref(r), N.ptr(flat), tokens,
+                                                N.REDUCE_DIRECT, N.ptr(out), N.ptr(ws), ws_bytes,
+                                                N.stream_handle(x.device)))
+        return out.reshape(x.shape)
+
     def _last_plan(self, device) -> PrefillPlan:
         return self._prefill_plans[(device.index, torch.cuda.current_stream(device).cuda_stream)]
 
@@ -316,8 +391,13 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
         return result
 
     def forward(self, x):
-        routes = x.reshape(-1, x.shape[-1]).shape[0] * self.config.num_experts_per_tok
-        if routes < self.min_routes:
+        tokens = x.reshape(-1, x.shape[-1]).shape[0]
+        if tokens * self.config.num_experts_per_tok < self.min_routes:
+            # Two and more tokens in the Direct order on the device: 8 tokens
+            # over 288 experts (H = 4096, I = 1536) 10 ms through the loop's
+            # ~600 launches and its readback of the ids, 217 us in one prefill.
+            if tokens > 1 and x.is_cuda and self._few_routes_on_device(x, tokens):
+                return torch.ops.glm53.moe_direct(x.detach(), self._op_key)
             return super().forward(x)
         if isinstance(self.gate, Float32Gate):
             N.require_device(x)

@@ -13,9 +13,11 @@ and FakeTensor / meta propagation gets the output shapes without a device.
 * ``glm53::moe_decode(x, owner, expert_ids?, scores?)`` -- one token through
   a ``PackedFP8MoE`` (router + routed + shared, or caller routing);
 * ``glm53::moe_prefill(x, owner, expert_ids?, scores?)`` -- the grouped
-  prefill of a ``SortedGroupedFP8MoE``.
+  prefill of a ``SortedGroupedFP8MoE``;
+* ``glm53::moe_direct(x, owner)`` -- a batch below a ``SortedGroupedFP8MoE``'s
+  min_routes as one prefill in the Direct order.
 
-The two MoE ops take the module by an integer key (``register_owner``): the
+The MoE ops take the module by an integer key (``register_owner``): the
 module keeps its weights, its per-(device, stream) native plans and its
 cached 0x7F/0xFF code flags, as an ``nn.Module`` does for its parameters,
 and the op reads them from there.  Outputs are always new tensors.
@@ -94,4 +96,14 @@ def moe_prefill(x: torch.Tensor, owner: int, expert_ids: Optional[torch.Tensor],
 
 @moe_prefill.register_fake
 def _(x, owner, expert_ids, scores):
+    return torch.empty_like(x)
+
+
+@torch.library.custom_op("glm53::moe_direct", mutates_args=())
+def moe_direct(x: torch.Tensor, owner: int) -> torch.Tensor:
+    return _owner(owner).native_direct(x)
+
+
+@moe_direct.register_fake
+def _(x, owner):
     return torch.empty_like(x)

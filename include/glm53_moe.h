@@ -472,6 +472,20 @@ int glm53_prefill_moe_hc(glm53_prefill_plan* plan, const glm53_bank* bank,
                          const float* scores, int32_t reduction, const void* residual,
                          const float* post, const float* comb, void* out_hc, void* stream);
 
+/* glm53_prefill_moe without a plan (no reference counterpart): the router's
+ * routes, scratch in `workspace` (device, 256-byte aligned, of
+ * glm53_prefill_workspace_bytes bytes, 0 for dimensions a plan would refuse;
+ * its contents need no initialisation and are free again once the work
+ * enqueued here is done).  Nothing is kept between calls, so calls on any
+ * threads and streams, each with its own workspace, are independent. */
+size_t glm53_prefill_workspace_bytes(int64_t hidden, int64_t intermediate, int64_t shared_intermediate,
+                                     int64_t experts, int64_t top_k, int64_t tokens);
+int glm53_prefill_moe_workspace(int64_t hidden, int64_t intermediate, int64_t shared_intermediate, int64_t experts,
+                                int64_t top_k, float swiglu_limit, const glm53_bank* bank,
+                                const glm53_shared_expert* shared, const glm53_router* router, const void* x,
+                                int64_t tokens, int32_t reduction, void* out, void* workspace, size_t workspace_bytes,
+                                void* stream);
+
 /* Synchronous: invalid route count of the last glm53_prefill_moe. */
 int glm53_prefill_plan_status(glm53_prefill_plan* plan, uint32_t* invalid_routes);
 

@@ -691,6 +691,51 @@ def test_direct_order_prefill_equals_direct_bit_for_bit(M, dev, config2_layer, t
     assert torch.equal(got.view(torch.int16), want.view(torch.int16)), (tokens, singletons)
 
 
+class _Gate:
+    def __init__(self, gate):
+        self.gate = gate
+
+    def __call__(self, x):
+        return self.gate(x)
+
+
+@pytest.mark.parametrize("shared_experts,reduction", [(1, "grouped"), (2, "direct"), (0, "grouped")])
+def test_few_tokens_equal_the_direct_loop_bit_for_bit(M, dev, shared_experts, reduction):
+    """Below min_routes a SortedGroupedFP8MoE runs the batch as one prefill in
+    the Direct order whatever its reduction: the Direct loop's bytes, from a
+    strided input too.  A gate, an input dtype or a shared expert that the
+    prefill does not stand for keeps the loop (same bytes, or its error)."""
+    import torch
+
+    syn = submodule("synthetic")
+    cfg = syn.layer_config(hidden=512, intermediate=256, experts=40, top_k=8, limit=7.0, shared=shared_experts)
+    bank, shared, gate = syn.synth_layer(cfg, seed=77, device=dev)
+    loop = M.PackedFP8MoE(bank, cfg, gate, shared)  # T > 1: the Direct loop
+    moe = M.SortedGroupedFP8MoE(bank, cfg, gate, shared, reduction=reduction)
+    for tokens in (2, 3, 9, 31):
+        x = syn.normal_bf16((tokens, 1024), syn.key(77, tokens), device=dev)[None, :, ::2]
+        assert moe._few_routes_on_device(x, tokens)
+        got, want = moe(x), loop(x)
+        assert got.shape == x.shape and not got.requires_grad
+        assert torch.equal(got.view(torch.int16), want.view(torch.int16)), tokens
+    assert not moe._prefill_plans
+    other = M.SortedGroupedFP8MoE(bank, cfg, _Gate(gate), shared, reduction=reduction)
+    assert not other._few_routes_on_device(x, 31)
+    assert torch.equal(other(x).view(torch.int16), want.view(torch.int16))
+    with pytest.raises(ValueError):
+        moe(x.float())
+    with pytest.raises(ValueError):
+        moe(x[..., :256])
+    if shared is not None:
+        hook = shared.register_forward_hook(lambda module, args, out: out * 0)
+        assert not moe._few_routes_on_device(x, 31)
+        assert torch.equal(moe(x).view(torch.int16), loop(x).view(torch.int16))
+        hook.remove()
+        shared.limit = 3.0
+        assert not moe._few_routes_on_device(x, 31)
+        assert torch.equal(moe(x).view(torch.int16), loop(x).view(torch.int16))
+
+
 def test_custom_ops_compile_without_graph_breaks(M, dev):
     """The MoE modules call the glm53 custom ops: torch.compile with
     fullgraph=True (no graph break allowed) traces decode and prefill, and
