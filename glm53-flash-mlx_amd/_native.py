@@ -178,15 +178,18 @@ def check(status: int) -> None:
     raise RuntimeError(message)
 
 
-def stream_handle(device: torch.device | None = None) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def stream_handle(device: torch.device | None = None) -> int:
+    """The hipStream_t of torch's current stream on `device` (the current
+    device when None or without an index)."""
+    index = device.index if device is not None else None
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
 
 
 def require_device(*tensors: torch.Tensor) -> None:
-    if not torch.cuda.is_available():
-        raise RuntimeError("the glm53 MI355X MoE path requires a ROCm GPU; no CPU fallback exists")
     for t in tensors:
         if t is not None and not t.is_cuda:
+            if not torch.cuda.is_available():
+                raise RuntimeError("the glm53 MI355X MoE path requires a ROCm GPU; no CPU fallback exists")
             raise ValueError("expected a tensor on the ROCm device, got one on the CPU")
 
 

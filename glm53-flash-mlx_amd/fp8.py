@@ -16,7 +16,7 @@ import math
 import torch
 
 from . import _native as N
-from . import ops as _ops  # noqa: F401  (registers the glm53 custom ops)
+from . import ops as _ops  # registers the glm53 custom ops
 
 BLOCK_SIZE = 128
 DECODE_TOP_K = 8
@@ -47,6 +47,8 @@ def block_fp8_linear(x: torch.Tensor, weight: torch.Tensor, scale_inv: torch.Ten
     expected = _scale_shape(out_features, in_features)
     if tuple(scale_inv.shape) != expected:
         raise ValueError(f"scale shape {tuple(scale_inv.shape)} != block128 shape {expected}")
+    if _ops.direct(x, weight, scale_inv, code_flags):
+        return native_block_fp8_linear(x, weight, scale_inv, code_flags)
     return torch.ops.glm53.block_fp8_linear(x, weight, scale_inv, code_flags)
 
 
@@ -54,17 +56,18 @@ def native_block_fp8_linear(x, weight, scale_inv, code_flags):
     """The native call behind the glm53::block_fp8_linear op (arguments
     validated by ``block_fp8_linear``)."""
     out_features, in_features = weight.shape
-    flat = x.reshape(-1, in_features).contiguous()
-    weight = weight.contiguous()
-    scale_inv = scale_inv.contiguous()
+    flat = x if x.dim() == 2 else x.reshape(-1, in_features)
+    flat, weight, scale_inv = flat.contiguous(), weight.contiguous(), scale_inv.contiguous()
     rows = flat.shape[0]
     y = torch.empty((rows, out_features), dtype=torch.bfloat16, device=x.device)
     lib = N.lib()
-    ws_bytes = lib.glm53_fp8_linear_workspace_bytes(rows, out_features, in_features)
+    ws_bytes = lib.glm53_fp8_linear_workspace_bytes(rows, out_features, in_features) if rows > 1 else 0
     ws = N.workspace(ws_bytes, x.device)
-    N.check(lib.glm53_fp8_linear(N.ptr(flat), rows, in_features, N.ptr(weight), out_features, N.ptr(scale_inv),
-                                 N.ptr(code_flags), N.ptr(y), N.ptr(ws), ws_bytes, N.stream_handle(x.device)))
-    return y.reshape(*x.shape[:-1], out_features)
+    N.check(lib.glm53_fp8_linear(flat.data_ptr(), rows, in_features, weight.data_ptr(), out_features,
+                                 scale_inv.data_ptr(), None if code_flags is None else code_flags.data_ptr(),
+                                 y.data_ptr(), None if ws is None else ws.data_ptr(), ws_bytes,
+                                 N.stream_handle(x.device)))
+    return y if x.dim() == 2 else y.reshape(*x.shape[:-1], out_features)
 
 
 def swiglu(gate: torch.Tensor, up: torch.Tensor, limit: float) -> torch.Tensor:

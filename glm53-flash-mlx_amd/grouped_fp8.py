@@ -19,6 +19,7 @@ import math
 import torch
 
 from . import _native as N
+from . import ops
 from .abi import GROUPED_MIN_ROUTES
 from .fp8 import BLOCK_SIZE, BlockFP8Linear, ClampedMLP, _scale_shape
 from .packed import PackedFP8MoE, _c_shared
@@ -385,7 +386,10 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
         N.require_device(x, indices, scores)
         if indices.shape[-1] != self.config.num_experts_per_tok:
             raise ValueError("indices do not match num_experts_per_tok")
-        result = torch.ops.glm53.moe_prefill(x, self._op_key, indices, scores)
+        if ops.direct(x, indices, scores):
+            result = self.native_prefill(x, indices, scores)
+        else:
+            result = torch.ops.glm53.moe_prefill(x, self._op_key, indices, scores)
         if check and self._last_plan(x.device).invalid_routes() != 0:
             raise ValueError(f"expert ids must lie in [0, {self.bank.expert_count})")
         return result
@@ -397,10 +401,14 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
             # over 288 experts (H = 4096, I = 1536) 10 ms through the loop's
             # ~600 launches and its readback of the ids, 217 us in one prefill.
             if tokens > 1 and x.is_cuda and self._few_routes_on_device(x, tokens):
+                if ops.direct(x):
+                    return self.native_direct(x)
                 return torch.ops.glm53.moe_direct(x.detach(), self._op_key)
             return super().forward(x)
         if isinstance(self.gate, Float32Gate):
             N.require_device(x)
+            if ops.direct(x):
+                return self.native_prefill(x)
             return torch.ops.glm53.moe_prefill(x, self._op_key, None, None)
         indices, scores = self.gate(x)
         return self.grouped_from_routes(x, indices, scores)

@@ -42,6 +42,31 @@ def register_owner(module) -> int:
     return key
 
 
+_PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter, torch.nn.Buffer)
+
+
+def direct(*tensors) -> bool:
+    """True when dispatching an op on `tensors` could only reach its device
+    kernel, so that an eager call may run the native call itself: the custom
+    op's Python layers cost ~12 us a call, more than a one-row linear's
+    kernel (4.5 us) and its launch together (call of a 4096 x 4096
+    BlockFP8Linear: 20 us through the op, 11 us direct).  Anything that
+    acts between the call and the kernel goes through the op: tracing and
+    compilation, dispatch and function modes, functorch transforms, forward-
+    and reverse-mode differentiation, a recording profiler, tensor
+    subclasses."""
+    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
+            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
+            or torch._C._functorch.peek_interpreter_stack() is not None
+            or torch.autograd.forward_ad._current_level >= 0 or torch.autograd._profiler_enabled()):
+        return False
+    grad = torch.is_grad_enabled()
+    for t in tensors:
+        if t is not None and (type(t) not in _PLAIN_TENSORS or (grad and t.requires_grad)):
+            return False
+    return True
+
+
 def _owner(key: int):
     ref = _OWNERS.get(int(key))
     module = ref() if ref is not None else None

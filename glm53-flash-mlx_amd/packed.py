@@ -716,6 +716,8 @@ class PackedFP8MoE(DirectFP8MoE):
             raise ValueError(f"decode expects {DECODE_TOP_K} expert ids and scores")
         if x.numel() != self.bank.hidden_size:
             raise ValueError(f"decode expects one token of width {self.bank.hidden_size}")
+        if ops.direct(x, expert_ids, scores):
+            return self.native_decode(x, expert_ids, scores)
         return torch.ops.glm53.moe_decode(x, self._op_key, expert_ids, scores)
 
     def forward(self, x):
@@ -724,6 +726,8 @@ class PackedFP8MoE(DirectFP8MoE):
             return super().forward(x)
         if isinstance(self.gate, Float32Gate) and self.gate.top_k == DECODE_TOP_K:
             N.require_device(x)
+            if ops.direct(x):
+                return self.native_decode(x)
             return torch.ops.glm53.moe_decode(x, self._op_key, None, None)
         indices, scores = self.gate(x)
         if indices.shape[-1] != DECODE_TOP_K:

@@ -21,7 +21,7 @@ from __future__ import annotations
 import torch
 
 from . import _native as N
-from . import ops as _ops  # noqa: F401  (registers the glm53 custom ops)
+from . import ops as _ops  # registers the glm53 custom ops
 
 
 class Float32Gate(torch.nn.Module):
@@ -58,6 +58,9 @@ class Float32Gate(torch.nn.Module):
         hidden = self.weight.shape[1]
         if x.shape[-1] != hidden:
             raise ValueError(f"input width {x.shape[-1]} != router width {hidden}")
+        if _ops.direct(x, self.weight, self.e_score_correction_bias):
+            return native_router_topk(x, self.weight, self.e_score_correction_bias, self.top_k,
+                                      self.routed_scaling_factor, self.norm_topk_prob, self.n_group, self.topk_group)
         return torch.ops.glm53.router_topk(x, self.weight, self.e_score_correction_bias, self.top_k,
                                            self.routed_scaling_factor, self.norm_topk_prob, self.n_group,
                                            self.topk_group)

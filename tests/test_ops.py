@@ -42,3 +42,44 @@ def test_unknown_owner_raises():
     ops = submodule("ops")
     with pytest.raises(RuntimeError, match="no longer exists"):
         ops._owner(10 ** 9)
+
+
+def test_direct_calls_only_where_the_op_would_reach_its_kernel_alone():
+    """ops.direct lets an eager call skip the op; anything that acts between
+    the call and the kernel goes through it."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.autograd import forward_ad
+    from torch.overrides import TorchFunctionMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    ops = submodule("ops")
+
+    class Dispatch(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Function(TorchFunctionMode):
+        def __torch_function__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Subclass(torch.Tensor):
+        pass
+
+    x = torch.zeros(4)
+    assert ops.direct(x, None, torch.nn.Parameter(x, requires_grad=False))
+    leaf = torch.zeros(4, requires_grad=True)
+    assert not ops.direct(x, leaf)
+    with torch.no_grad():
+        assert ops.direct(x, leaf)
+    assert not ops.direct(x.as_subclass(Subclass))
+    for mode in (Dispatch(), Function(), FakeTensorMode(), forward_ad.dual_level(),
+                 torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU])):
+        with mode:
+            assert not ops.direct(x), mode
+    seen = []
+    torch.vmap(lambda v: seen.append(ops.direct(v)) or v)(torch.zeros(2, 3))
+    torch.jit.trace(lambda v: seen.append(ops.direct(v)) or v + 1, (x,), check_trace=False)
+    torch.compile(lambda v: v + 1 if ops.direct(v) else v - 1, backend="eager")(x)
+    assert seen and not any(seen)
+    assert torch.equal(torch.compile(lambda v: v + 1 if ops.direct(v) else v - 1, backend="eager")(x), x - 1)
+    assert ops.direct(x)
