@@ -90,6 +90,47 @@ hipError_t split(const void* x, int64_t rows, int64_t cols, const SplitBuf& b, h
   return launch_split_activations(a, st);
 }
 
+// One dense problem, plain or SwiGLU, on split activations, in the shape that
+// dense_tile names.  `flags`: device int32 [1] (SwiGLU: [2]) for the weights
+// that come without a code flag where the shape does not look for the codes
+// itself.
+int dense(const DenseArgs& d, bool swiglu, int32_t* flags, hipStream_t st) {
+  const DenseTile tile = dense_tile(d.rows, d.K, d.N, swiglu);
+  if (dense_ksplit(tile, swiglu)) {
+    HIP_TRY(launch_dense_linear(d, tile, swiglu, st), "dense linear launch");
+    return GLM53_OK;
+  }
+  auto flag_of = [&](const int32_t* flag, const uint8_t* weight, int32_t* space) -> const int32_t* {
+    if (flag != nullptr) return flag;
+    return launch_scan_480(weight, d.N * d.K, space, true, st) == hipSuccess ? space : nullptr;
+  };
+  GroupedGemmArgs g{};
+  g.fixup = flag_of(d.flag, d.weight, flags);
+  if (swiglu) g.fixup_up = flag_of(d.flag_up, d.weight_up, flags + 1);
+  if (g.fixup == nullptr || (swiglu && g.fixup_up == nullptr)) return hip_fail(hipGetLastError(), "scan launch");
+  g.a_hi = d.a_hi;
+  g.a_lo = d.a_lo;
+  g.a_scale = d.a_scale;
+  g.K = d.K;
+  g.routes = d.rows;
+  g.experts = 1;
+  g.weight = d.weight;
+  g.weight_up = d.weight_up;
+  g.scale = d.scale;
+  g.scale_up = d.scale_up;
+  g.s_cols = d.K / 128;
+  g.N = d.N;
+  g.limit = d.limit;
+  g.tile_rows = tile.rows;
+  g.out = d.out;
+  g.out_row_stride = d.N;
+  const int mode = swiglu ? GEMM_SWIGLU : GEMM_PLAIN;
+  HIP_TRY(tile.rows == kGemmWideRows ? launch_wide_dense(g, mode, tile.cols / (swiglu ? 64 : 128), st)
+                                     : launch_grouped_gemm(g, mode, cdiv(d.rows, tile.rows), st),
+          "grouped gemm launch");
+  return GLM53_OK;
+}
+
 int check_linear(const glm53_linear& l, int64_t out, int64_t in, const char* name) {
   CHECK_ARG(l.weight != nullptr && l.scale_inv != nullptr, "%s: null weight or scale", name);
   CHECK_ARG(l.out_features == out && l.in_features == in, "%s: shape [%lld, %lld] != expected [%lld, %lld]", name,
@@ -387,47 +428,18 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
   if (need > 0 && aligned(weight, 16) && workspace != nullptr && workspace_bytes >= need) {
     SplitBuf b = carve_split(workspace, M, K);
     HIP_TRY(split(x, M, K, b, st), "split launch");
-    const DenseTile tile = dense_tile(M, K, N);
-    if (tile.cols < 128) {
-      DenseArgs d{};
-      d.a_hi = b.hi;
-      d.a_lo = b.lo;
-      d.a_scale = b.scale;
-      d.weight = weight;
-      d.scale = scale_inv;
-      d.flag = code_flags;  // null: the kernel looks for 0x7F / 0xFF itself
-      d.rows = M;
-      d.K = K;
-      d.N = N;
-      d.out = static_cast<uint16_t*>(y);
-      HIP_TRY(launch_dense_linear(d, tile, st), "dense linear launch");
-      return GLM53_OK;
-    }
-    const int32_t* flag = code_flags;
-    if (flag == nullptr) {
-      int32_t* f = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + split_bytes(M, K));
-      HIP_TRY(launch_scan_480(weight, N * K, f, true, st), "scan launch");
-      flag = f;
-    }
-    GroupedGemmArgs g{};
-    g.fixup = flag;
-    g.a_hi = b.hi;
-    g.a_lo = b.lo;
-    g.a_scale = b.scale;
-    g.K = K;
-    g.routes = M;
-    g.experts = 1;
-    g.weight = weight;
-    g.scale = scale_inv;
-    g.s_cols = K / 128;
-    g.N = N;
-    g.tile_rows = tile.rows;
-    g.out = static_cast<uint16_t*>(y);
-    g.out_row_stride = N;
-    HIP_TRY(tile.rows == kGemmWideRows ? launch_wide_dense(g, static_cast<int>(tile.cols / 128), st)
-                                       : launch_grouped_gemm(g, GEMM_PLAIN, cdiv(M, tile.rows), st),
-            "grouped gemm launch");
-    return GLM53_OK;
+    DenseArgs d{};
+    d.a_hi = b.hi;
+    d.a_lo = b.lo;
+    d.a_scale = b.scale;
+    d.weight = weight;
+    d.scale = scale_inv;
+    d.flag = code_flags;
+    d.rows = M;
+    d.K = K;
+    d.N = N;
+    d.out = static_cast<uint16_t*>(y);
+    return dense(d, false, reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + split_bytes(M, K)), st);
   }
   GenericLinearArgs a{};
   a.x = static_cast<const uint16_t*>(x);
@@ -446,6 +458,84 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
   CHECK_ARG(K <= 16384, "generic path supports K <= 16384");
   HIP_TRY(launch_linear_generic(a, st), "generic linear launch");
   return GLM53_OK;
+}
+
+// --------------------------------------------------------------- MLP ------
+
+namespace {
+struct MlpSpace {
+  SplitBuf xq;
+  uint16_t* h;
+  SplitBuf hq;
+  int32_t* flags;
+  size_t bytes;
+};
+MlpSpace mlp_space(void* base, int64_t M, int64_t H, int64_t I) {
+  uint8_t* p = static_cast<uint8_t*>(base);
+  MlpSpace s;
+  s.xq = carve_split(p, M, H);
+  p += split_bytes(M, H);
+  s.h = reinterpret_cast<uint16_t*>(p);
+  p += round_up(2 * static_cast<size_t>(M * I));
+  s.hq = carve_split(p, M, I);
+  p += split_bytes(M, I);
+  s.flags = reinterpret_cast<int32_t*>(p);
+  s.bytes = static_cast<size_t>(p - static_cast<uint8_t*>(base)) + 256;
+  return s;
+}
+}  // namespace
+
+size_t glm53_mlp_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate) {
+  if (M <= 1 || hidden <= 0 || intermediate <= 0 || hidden % 128 != 0 || intermediate % 128 != 0) return 0;
+  return mlp_space(nullptr, M, hidden, intermediate).bytes;
+}
+
+int glm53_mlp(const glm53_shared_expert* mlp, float limit, const void* x, int64_t M, void* y, void* workspace,
+              size_t workspace_bytes, void* stream) {
+  CHECK_ARG(mlp != nullptr, "mlp is null");
+  const int64_t H = mlp->gate.in_features, I = mlp->gate.out_features;
+  if (int rc = check_linear(mlp->gate, I, H, "gate")) return rc;
+  if (int rc = check_linear(mlp->up, I, H, "up")) return rc;
+  if (int rc = check_linear(mlp->down, H, I, "down")) return rc;
+  const size_t need = glm53_mlp_workspace_bytes(M, H, I);
+  CHECK_ARG(need > 0, "mlp needs two or more rows and widths that are multiples of 128; got M=%lld, H=%lld, I=%lld",
+            (long long)M, (long long)H, (long long)I);
+  CHECK_ARG(x && y && workspace && workspace_bytes >= need && aligned(workspace, 256),
+            "mlp needs x, y and a 256-byte aligned workspace of %zu bytes", need);
+  CHECK_ARG(aligned(mlp->gate.weight, 16) && aligned(mlp->up.weight, 16) && aligned(mlp->down.weight, 16),
+            "mlp weights must be 16-byte aligned");
+  hipStream_t st = S(stream);
+  const MlpSpace s = mlp_space(workspace, M, H, I);
+  HIP_TRY(split(x, M, H, s.xq, st), "split launch");
+  DenseArgs g{};
+  g.a_hi = s.xq.hi;
+  g.a_lo = s.xq.lo;
+  g.a_scale = s.xq.scale;
+  g.weight = mlp->gate.weight;
+  g.scale = mlp->gate.scale_inv;
+  g.flag = mlp->gate.code_flags;
+  g.weight_up = mlp->up.weight;
+  g.scale_up = mlp->up.scale_inv;
+  g.flag_up = mlp->up.code_flags;
+  g.limit = limit;
+  g.rows = M;
+  g.K = H;
+  g.N = I;
+  g.out = s.h;
+  if (int rc = dense(g, true, s.flags, st)) return rc;
+  HIP_TRY(split(s.h, M, I, s.hq, st), "split launch");
+  DenseArgs d{};
+  d.a_hi = s.hq.hi;
+  d.a_lo = s.hq.lo;
+  d.a_scale = s.hq.scale;
+  d.weight = mlp->down.weight;
+  d.scale = mlp->down.scale_inv;
+  d.flag = mlp->down.code_flags;
+  d.rows = M;
+  d.K = I;
+  d.N = H;
+  d.out = static_cast<uint16_t*>(y);
+  return dense(d, false, s.flags + 2, st);
 }
 
 // ------------------------------------------------------------ router ------

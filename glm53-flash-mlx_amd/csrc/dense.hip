@@ -38,10 +38,12 @@ constexpr int turn_tiles() {
 template <int P, int C>
 size_t dense_lds_bytes(int64_t K) {
   return static_cast<size_t>(kDenseWaves) * (fold_steps<P, C>() * P * C * 1024 + turn_tiles<P, C>() * kOperand) +
-         sizeof(float) * static_cast<size_t>(K / kBlock);
+         2 * sizeof(float) * static_cast<size_t>(K / kBlock);
 }
 
-// Rows row0 .. row0 + 16 P - 1 x columns col0 .. col0 + 16 C - 1.  Wavefront w
+// Rows row0 .. row0 + 16 P - 1 x weight tiles 0 .. C - 1: columns col0 .. col0
+// + 16 C - 1, or (SWIGLU) gate rows col0 .. col0 + 8 C - 1 in the first half
+// of the tiles and the matching up rows in the second.  Wavefront w
 // multiplies K blocks w, w + 8, ...: its operands come from global memory
 // into registers (each byte of the item's rows and columns once per
 // workgroup), load_depth steps ahead, 8 rows of whole 128-byte lines per
@@ -52,9 +54,10 @@ size_t dense_lds_bytes(int64_t K) {
 // to LDS, and wavefront t < P C adds tile t's results in block order, so
 // every output goes through the operations of the grouped GEMM and has its
 // bits.  Returns codes_480 of the weight bytes (DETECT).
-template <int P, int C, bool FIX, bool DETECT>
+template <int P, int C, bool SWIGLU, bool FIX, bool DETECT>
 __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_t row0, int64_t col0, uint8_t* lds) {
   constexpr int D = FIX ? 1 : load_depth<P, C>(), F = FIX ? 1 : fold_steps<P, C>();
+  constexpr int H = SWIGLU ? C / 2 : C;  // tiles of one matrix
   constexpr int U = D > F ? D : F;  // steps per loop turn: the registers rotate back, folds fall at its end
   const int lane = threadIdx.x & 63, r = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
@@ -64,7 +67,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   constexpr int kFold = kDenseWaves * fold_steps<P, C>() * P * C * 1024;
   f32x4* lds_c = reinterpret_cast<f32x4*>(lds);                                          // [8 F][P C][64]
   uint8_t* turn = lds + kFold + wave * turn_tiles<P, C>() * kOperand;                    // this wavefront's
-  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * turn_tiles<P, C>() * kOperand);  // [KB]
+  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * turn_tiles<P, C>() * kOperand);  // [2][KB]
   const OperandSlots slots = operand_slots(lane);
 
   // rows past the last repeat it, columns past the matrix its last row: valid
@@ -86,7 +89,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   for (int c = 0; c < C; ++c)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
-      const int64_t n = col0 + 16 * c + 8 * h + (lane >> 3);
+      const int64_t n = col0 + 16 * (c % H) + 8 * h + (lane >> 3);
       wrow[c][h] = static_cast<uint32_t>((n < a.N ? n : a.N - 1) * K + load_piece_offset(lane, h));
     }
   struct Step {
@@ -97,7 +100,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
     int kb = kDenseWaves * s + wave;
     kb = kb < KB ? kb : KB - 1;  // past the end: loaded, never folded
     const int64_t ko = static_cast<int64_t>(kb) * kBlock;  // wave-uniform
-    const uint8_t *w = a.weight + ko, *hi = a.a_hi + ko, *lo = a.a_lo + ko;
+    const uint8_t *w = a.weight + ko, *up = SWIGLU ? a.weight_up + ko : w, *hi = a.a_hi + ko, *lo = a.a_lo + ko;
     const float* se = a.a_scale + kb;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
@@ -111,7 +114,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
 #pragma unroll
     for (int c = 0; c < C; ++c)
 #pragma unroll
-      for (int h = 0; h < 2; ++h) v.b[c][h] = *reinterpret_cast<const u32x4*>(w + wrow[c][h]);
+      for (int h = 0; h < 2; ++h) v.b[c][h] = *reinterpret_cast<const u32x4*>((c < H ? w : up) + wrow[c][h]);
   };
   auto put = [&](int tile, const u32x4 (&v)[2]) {
 #pragma unroll
@@ -123,8 +126,11 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
 #pragma unroll
   for (int d = 0; d < D; ++d)
     if (d < steps) load(d, v[d]);
-  const float* sw = a.scale + (col0 / kBlock) * KB;  // the item's columns lie in one scale block
-  for (int kb = threadIdx.x; kb < KB; kb += 64 * kDenseWaves) lds_sw[kb] = sw[kb];
+  const int64_t scale_row = (col0 / kBlock) * KB;  // the item's columns lie in one scale block
+  for (int kb = threadIdx.x; kb < KB; kb += 64 * kDenseWaves) {
+    lds_sw[kb] = a.scale[scale_row + kb];
+    if constexpr (SWIGLU) lds_sw[KB + kb] = a.scale_up[scale_row + kb];
+  }
 
   uint32_t found = 0;
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -188,6 +194,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
     const int first = kDenseWaves * s0;
     const int count = KB - first < kDenseWaves * F ? KB - first : kDenseWaves * F;
     const f32x4* mine = lds_c + wave * 64 + lane;
+    const float* my_sw = lds_sw + (wave % C < H ? 0 : KB);
     int i = 0;
     for (; i + 8 <= count; i += 8) {
       f32x4 x[8];
@@ -195,14 +202,14 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
       for (int u = 0; u < 8; ++u) x[u] = mine[(i + u) * P * C * 64];
 #pragma unroll
       for (int u = 0; u < 8; ++u) {
-        const float t = lds_sw[first + i + u];
+        const float t = my_sw[first + i + u];
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[u][e], t, acc[e]);
       }
     }
     for (; i < count; ++i) {
       const f32x4 x = mine[i * P * C * 64];
-      const float t = lds_sw[first + i];
+      const float t = my_sw[first + i];
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[e] = fmaf(x[e], t, acc[e]);
     }
@@ -234,11 +241,34 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   }
   // lane holds rows 4 kq .. 4 kq + 3, column r of tile `wave`
   const int64_t n = col0 + 16 * (wave % C) + r;
-  if (wave < P * C && n < a.N) {
+  uint32_t y[2];
+  if constexpr (SWIGLU) {
+    f32x4* turned_up = lds_c + (wave % C < H ? wave + H : wave) * 64 + lane;  // the matching up tile's results
+    __syncthreads();  // every fold has read its results
+    if (wave < P * C && wave % C >= H) *turned_up = (f32x4){acc[0], acc[1], acc[2], acc[3]};
+    __syncthreads();
+    if (wave >= P * C || wave % C >= H) return found;
+    const f32x4 up = *turned_up;
+    SwigluCheck check;
+#pragma unroll
+    for (int q = 0; q < 2; ++q)
+      y[q] = swiglu_mlx_straight2(acc[2 * q], up[2 * q], acc[2 * q + 1], up[2 * q + 1], a.limit, check);
+    if (__builtin_amdgcn_ballot_w64(!swiglu_straight_ok(check, a.limit)) != 0) {
+#pragma unroll
+      for (int q = 0; q < 2; ++q)
+        y[q] = swiglu_mlx(acc[2 * q], up[2 * q], a.limit) |
+               static_cast<uint32_t>(swiglu_mlx(acc[2 * q + 1], up[2 * q + 1], a.limit)) << 16;
+    }
+  } else {
+    if (wave >= P * C) return found;
+#pragma unroll
+    for (int q = 0; q < 2; ++q) y[q] = f32x2_to_bf16x2(acc[2 * q], acc[2 * q + 1]);
+  }
+  if (n < a.N) {
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       const int64_t m = row0 + 16 * (wave / C) + 4 * kq + e;
-      if (m < a.rows) a.out[m * a.N + n] = f32_to_bf16(acc[e]);
+      if (m < a.rows) a.out[m * a.N + n] = static_cast<uint16_t>(e & 1 ? y[e >> 1] >> 16 : y[e >> 1]);
     }
   }
   return found;
@@ -246,29 +276,32 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
 
 // Workgroup i runs on XCD i % 8; each XCD takes a contiguous run of items,
 // row groups fastest, so the items that share weight columns meet in one L2.
-template <int P, int C>
+template <int P, int C, bool SWIGLU>
 __global__ __launch_bounds__(64 * kDenseWaves) void dense_ksplit_kernel(DenseArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
+  constexpr int kCols = SWIGLU ? 8 * C : 16 * C;
   const int64_t row_groups = (a.rows + 16 * P - 1) / (16 * P);
-  const int64_t items = row_groups * ((a.N + 16 * C - 1) / (16 * C));
+  const int64_t items = row_groups * ((a.N + kCols - 1) / kCols);
   const int64_t per_xcd = (items + 7) / 8;
   const int64_t i = static_cast<int64_t>(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
   if (i >= items) return;
-  const int64_t row0 = 16 * P * (i % row_groups), col0 = 16 * C * (i / row_groups);
-  bool fix = a.flag != nullptr && *a.flag != 0;
+  const int64_t row0 = 16 * P * (i % row_groups), col0 = kCols * (i / row_groups);
+  const bool look = a.flag == nullptr || (SWIGLU && a.flag_up == nullptr);
+  bool fix = (a.flag != nullptr && *a.flag != 0) || (SWIGLU && a.flag_up != nullptr && *a.flag_up != 0);
   if (!fix) {
-    const uint32_t found = dense_ksplit_item<P, C, false, true>(a, row0, col0, lds_dyn);
-    if (a.flag == nullptr) fix = workgroup_any((found & 0x80808080u) != 0, lds_dyn);
+    const uint32_t found = dense_ksplit_item<P, C, SWIGLU, false, true>(a, row0, col0, lds_dyn);
+    if (look) fix = workgroup_any((found & 0x80808080u) != 0, lds_dyn);
   }
-  if (fix) dense_ksplit_item<P, C, true, false>(a, row0, col0, lds_dyn);
+  if (fix) dense_ksplit_item<P, C, SWIGLU, true, false>(a, row0, col0, lds_dyn);
 }
 
-template <int P, int C>
+template <int P, int C, bool SWIGLU>
 hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
-  const int64_t items = ((a.rows + 16 * P - 1) / (16 * P)) * ((a.N + 16 * C - 1) / (16 * C));
+  constexpr int kCols = SWIGLU ? 8 * C : 16 * C;
+  const int64_t items = ((a.rows + 16 * P - 1) / (16 * P)) * ((a.N + kCols - 1) / kCols);
   const size_t lds = dense_lds_bytes<P, C>(a.K);
   if (a.K > kDenseMaxK || lds > 160 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((dense_ksplit_kernel<P, C>), dim3(static_cast<unsigned>(8 * ((items + 7) / 8))),
+  hipLaunchKernelGGL((dense_ksplit_kernel<P, C, SWIGLU>), dim3(static_cast<unsigned>(8 * ((items + 7) / 8))),
                      dim3(64 * kDenseWaves), lds, st, a);
   return hipGetLastError();
 }
@@ -290,30 +323,35 @@ hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
 // (64 x 128 took every row count before: 22.2 at 16 rows, 28.1 at 128, 77.3
 // at 2,048, 156 at 4,096.)  The narrow tiles' offsets fit 32 bits, the wide
 // shape's 31.
-DenseTile dense_tile(int64_t rows, int64_t K, int64_t N) {
+// A SwiGLU tile holds half as many output columns in the same time (gate and
+// up tile side by side), so 16 x 16 has no SwiGLU form of its own.
+DenseTile dense_tile(int64_t rows, int64_t K, int64_t N, bool swiglu) {
   struct Candidate {
-    DenseTile tile;
-    int64_t items;  // at most
+    DenseTile tile;  // weight columns
+    int64_t items;   // at most
   };
   constexpr Candidate kTiles[] = {{{16, 16}, 256},  {{16, 32}, 256},  {{32, 32}, 256},   {{32, 64}, 256},
                                   {{32, 128}, 256}, {{64, 128}, 224}, {{128, 128}, 256}, {{128, 256}, 256}};
   const bool narrow = K <= kDenseMaxK && N * K < (int64_t{1} << 32) && rows * K < (int64_t{1} << 32);
   const bool wide = K <= kWideDenseMaxK && wide_offsets_fit(N, K, rows);
+  auto of = [&](DenseTile t) { return DenseTile{t.rows, swiglu ? t.cols / 2 : t.cols}; };
   for (const Candidate& c : kTiles) {
-    const DenseTile t = c.tile;
-    if (t.cols < 128 ? !narrow : t.rows == 128 && !wide) continue;
+    if (c.tile.cols < 128 ? !narrow : c.tile.rows == 128 && !wide) continue;
+    if (swiglu && (c.tile.cols == 16 || (c.tile.rows == 128 && c.tile.cols == 128))) continue;
+    const DenseTile t = of(c.tile);
     if (((rows + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) <= c.items) return t;
   }
-  return wide ? DenseTile{128, 512} : DenseTile{64, 128};
+  return of(wide ? DenseTile{128, 512} : DenseTile{64, 128});
 }
 
-hipError_t launch_dense_linear(const DenseArgs& a, DenseTile t, hipStream_t st) {
+hipError_t launch_dense_linear(const DenseArgs& a, DenseTile t, bool swiglu, hipStream_t st) {
   if (a.rows <= 0 || a.K <= 0 || a.K % kBlock != 0 || a.N <= 0 || a.N % 16 != 0) return hipErrorInvalidValue;
   if (a.N * a.K >= (int64_t{1} << 32) || a.rows * a.K >= (int64_t{1} << 32)) return hipErrorInvalidValue;
-  if (t.rows == 16 && t.cols == 16) return launch_ksplit<1, 1>(a, st);
-  if (t.rows == 16 && t.cols == 32) return launch_ksplit<1, 2>(a, st);
-  if (t.rows == 32 && t.cols == 32) return launch_ksplit<2, 2>(a, st);
-  if (t.rows == 32 && t.cols == 64) return launch_ksplit<2, 4>(a, st);
+  const int cols = swiglu ? 2 * t.cols : t.cols;
+  if (t.rows == 16 && cols == 16 && !swiglu) return launch_ksplit<1, 1, false>(a, st);
+  if (t.rows == 16 && cols == 32) return swiglu ? launch_ksplit<1, 2, true>(a, st) : launch_ksplit<1, 2, false>(a, st);
+  if (t.rows == 32 && cols == 32) return swiglu ? launch_ksplit<2, 2, true>(a, st) : launch_ksplit<2, 2, false>(a, st);
+  if (t.rows == 32 && cols == 64) return swiglu ? launch_ksplit<2, 4, true>(a, st) : launch_ksplit<2, 4, false>(a, st);
   return hipErrorInvalidValue;
 }
 

@@ -135,8 +135,8 @@ hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descr
 // kGemmTileRows routes; fixup null: the items look for 0x7F / 0xFF themselves
 hipError_t launch_grouped_linear(const GroupedGemmArgs& a, int64_t descriptors, hipStream_t st);
 // A dense problem (implicit descriptors, expert 0) on the wide shape with
-// `tiles` weight tiles per wavefront: 128 rows x 128 tiles columns per item
-hipError_t launch_wide_dense(const GroupedGemmArgs& a, int tiles, hipStream_t st);
+// `tiles` weight tiles per wavefront: 128 rows x 128 tiles weight rows per item
+hipError_t launch_wide_dense(const GroupedGemmArgs& a, int mode, int tiles, hipStream_t st);
 hipError_t launch_reduce(const ReduceArgs& a, bool direct_order, hipStream_t st);
 hipError_t launch_scan_480(const uint8_t* codes, int64_t n, int32_t* flag, bool clear, hipStream_t st);
 

@@ -999,8 +999,8 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) 
 // stage start).  Per stage 8 KB of B and 32 KB of A operand reads for 64
 // MFMAs per wavefront.  The arithmetic per output
 // element is that of the narrower shapes, so every shape gives the same
-// bits.  A PLAIN launch may take T = 1 or 2 weight tiles per wavefront
-// instead of 4 (128 or 256 columns per item): a dense linear whose 512-column
+// bits.  A dense launch may take T = 2 (PLAIN: or 1) weight tiles per
+// wavefront instead of 4 (256 or 128 weight rows per item) where 512-row
 // items would leave CUs without one.
 namespace {
 constexpr int kWidePairs = kGemmWideRows / 16;            // 8
@@ -1054,6 +1054,7 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
                                                 bool loads_pair, uint8_t* lds, uint32_t lds_addr, const uint8_t* lds_se,
                                                 const float* lds_sw, int wave, int lane) {
   constexpr int kBBytes = 8 * T * kOperand;
+  constexpr int kHalf = T > 1 ? T / 2 : 1;  // tiles of the lo rows (SWIGLU: gate), the others of the hi rows (up)
   const OperandSlots slots = operand_slots(lane);
   const uint32_t b_own = static_cast<uint32_t>(wave) * T * kOperand;  // this wavefront's tiles in the B stage
   auto issue_b = [&](int64_t kb) {
@@ -1063,11 +1064,11 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
     for (int q = 0; q < T; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        lds_direct16_at((q < 2 ? mlo : mhi) + ls.wrow[2 * q + h], ls.woff ^ (16 * h),
+        lds_direct16_at((q < kHalf ? mlo : mhi) + ls.wrow[2 * q + h], ls.woff ^ (16 * h),
                         lds_addr + b_own + q * kOperand + 1024 * h);
   };
   auto issue_b_tile = [&](int64_t kb, int q) {
-    const uint8_t* m = (q < 2 ? ls.wlo : ls.whi) + (kb << (7 + ls.wg));
+    const uint8_t* m = (q < kHalf ? ls.wlo : ls.whi) + (kb << (7 + ls.wg));
 #pragma unroll
     for (int h = 0; h < 2; ++h)
       lds_direct16_at(m + ls.wrow[2 * q + h], ls.woff ^ (16 * h), lds_addr + b_own + q * kOperand + 1024 * h);
@@ -1085,8 +1086,8 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
   // weight scale row (of lds_sw) of the wavefront's tile q: PLAIN its
   // 64 rows lie in block (64 w) / 128 of the item; SWIGLU gate tiles in
   // gate block (32 w) / 128, up tiles in the same up block
-  const int sw_lo = MODE == GEMM_PLAIN ? (16 * T * wave) >> 7 : (32 * wave) >> 7;
-  const int sw_hi = MODE == GEMM_PLAIN ? sw_lo : 2 + sw_lo;
+  const int sw_lo = MODE == GEMM_PLAIN ? (16 * T * wave) >> 7 : (8 * T * wave) >> 7;
+  const int sw_hi = MODE == GEMM_PLAIN ? sw_lo : T / 2 + sw_lo;
 
   float acc[NP][T][4];
 #pragma unroll
@@ -1132,7 +1133,7 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
     const uint8_t* st = lds + kBBytes + slot * kWideABytes;
     f32x4 c[T];
     auto fold = [&](int j, int q) {
-      const float sw = q < 2 ? w_lo : w_hi;
+      const float sw = q < kHalf ? w_lo : w_hi;
 #pragma unroll
       for (int i = 0; i < 4; ++i) acc[j][q][i] = fmaf(c[q][i], sw, acc[j][q][i]);
     };
@@ -1215,7 +1216,7 @@ __device__ __forceinline__ void wide_gemm_loop(const GroupedGemmArgs& a, const I
   if constexpr (MODE == GEMM_PLAIN) {
     plain_epilogue<NP, T>(a, src, start, len, 0, 1, ntile * (128 * T) + 16 * T * wave, acc, lane);
   } else {
-    swiglu_epilogue<NP, T / 2>(a, src, start, len, 0, 1, ntile * kWideGateRows + 32 * wave, acc, lane);
+    swiglu_epilogue<NP, T / 2>(a, src, start, len, 0, 1, ntile * (64 * T) + 8 * T * wave, acc, lane);
   }
 }
 
@@ -1223,8 +1224,8 @@ template <int MODE, bool FIX, int T>
 __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const ItemSource src, int64_t ntile,
                                                 int64_t d, uint8_t* lds) {
   constexpr int kBBytes = 8 * T * kOperand;
-  constexpr int kBlocks = MODE == GEMM_PLAIN ? T : 4;  // weight scale rows of an item
-  static_assert(MODE == GEMM_PLAIN || T == kWideTilesPerWave, "the SwiGLU item is 256 gate and 256 up rows");
+  constexpr int kHalf = T > 1 ? T / 2 : 1;  // tiles of the lo rows (SWIGLU: gate), the others of the hi rows (up)
+  static_assert(MODE == GEMM_PLAIN || T % 2 == 0, "a SwiGLU item holds whole gate and up scale blocks");
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
   int32_t expert, start, len;
@@ -1254,13 +1255,13 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
     ls.wg = src.wg;
     const int64_t rows = a.N;
     const int32_t piece = load_piece_offset(lane, 0);
-    const int64_t rlo = MODE == GEMM_PLAIN ? ntile * (128 * T) + 16 * T * wave : ntile * kWideGateRows + 32 * wave;
-    const int64_t rhi = MODE == GEMM_PLAIN ? rlo + 32 : rlo;
+    const int64_t rlo = MODE == GEMM_PLAIN ? ntile * (128 * T) + 16 * T * wave : ntile * (64 * T) + 8 * T * wave;
+    const int64_t rhi = MODE == GEMM_PLAIN ? rlo + 16 * kHalf : rlo;
 #pragma unroll
     for (int q = 0; q < T; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        int64_t u = (q < 2 ? rlo : rhi) + 16 * (q & 1) + 8 * h;
+        int64_t u = (q < kHalf ? rlo : rhi) + 16 * (q % kHalf) + 8 * h;
         u = u < rows - 8 ? u : rows - 8;
         ls.wrow[2 * q + h] = group_row_base(u, K, ls.wg);
       }
@@ -1278,7 +1279,7 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
     for (int q = 0; q < T; ++q)
 #pragma unroll
       for (int h = 0; h < 2; ++h)
-        lds_direct16_at((q < 2 ? ls.wlo : ls.whi) + ls.wrow[2 * q + h], ls.woff ^ (16 * h),
+        lds_direct16_at((q < kHalf ? ls.wlo : ls.whi) + ls.wrow[2 * q + h], ls.woff ^ (16 * h),
                         lds_addr + b_own + q * kOperand + 1024 * h);
     if (loads_pair) {
       const uint32_t sa = lds_addr + kBBytes + 2 * wave * kOperand;
@@ -1293,12 +1294,12 @@ __device__ __forceinline__ void wide_gemm_body(const GroupedGemmArgs& a, const I
   // weight scale rows: PLAIN the item's four 128-row blocks; SWIGLU the two
   // blocks its 256 gate rows span, then the same up blocks
   const int64_t srows = (a.N + 127) / 128;
-  const int64_t b0 = MODE == GEMM_PLAIN ? T * ntile : 2 * ntile;
-  for (int64_t i = threadIdx.x; i < kBlocks * KB; i += 512) {
+  const int64_t b0 = MODE == GEMM_PLAIN ? T * ntile : kHalf * ntile;
+  for (int64_t i = threadIdx.x; i < T * KB; i += 512) {
     const int64_t r = i / KB, k = i - r * KB;
-    int64_t blk = b0 + (MODE == GEMM_PLAIN ? r : (r & 1));
+    int64_t blk = b0 + (MODE == GEMM_PLAIN ? r : r % kHalf);
     blk = blk < srows ? blk : srows - 1;
-    const float* sc = (MODE == GEMM_SWIGLU && r >= 2) ? src.scale_up : src.scale;
+    const float* sc = (MODE == GEMM_SWIGLU && r >= kHalf) ? src.scale_up : src.scale;
     lds_sw[i] = sc[static_cast<int64_t>(expert) * a.s_expert_stride + blk * a.s_cols + k];
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wavefront's stage-0 loads landed
@@ -1564,20 +1565,22 @@ hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descr
   return hipGetLastError();
 }
 
-hipError_t launch_wide_dense(const GroupedGemmArgs& a, int tiles, hipStream_t st) {
+hipError_t launch_wide_dense(const GroupedGemmArgs& a, int mode, int tiles, hipStream_t st) {
   if (a.out_row_stride < a.N || a.out_row_stride >= (int64_t{1} << 22)) return hipErrorInvalidValue;
+  const int64_t cols = mode == GEMM_PLAIN ? 128 * tiles : 64 * tiles;
   GroupedGemmArgs g = a;
-  g.n_tiles = (a.N + 128 * tiles - 1) / (128 * tiles);
+  g.n_tiles = (a.N + cols - 1) / cols;
   g.descriptors = (a.routes + kGemmWideRows - 1) / kGemmWideRows;
   const unsigned grid = static_cast<unsigned>(8 * ((g.n_tiles * g.descriptors + 7) / 8));
   const size_t lds = gemm_wide_lds_bytes(a.K, tiles);
   if (a.K % kBlock != 0 || a.K <= 0 || lds > 160 * 1024) return hipErrorInvalidValue;
   if (!wide_offsets_fit(a.N, a.K, a.routes)) return hipErrorInvalidValue;
-#define GLM53_WIDE_DENSE(t) \
-  hipLaunchKernelGGL((grouped_gemm_wide_kernel<GEMM_PLAIN, t>), dim3(grid), dim3(512), lds, st, g)
-  if (tiles == 1) GLM53_WIDE_DENSE(1);
-  else if (tiles == 2) GLM53_WIDE_DENSE(2);
-  else if (tiles == kWideTilesPerWave) GLM53_WIDE_DENSE(kWideTilesPerWave);
+#define GLM53_WIDE_DENSE(m, t) hipLaunchKernelGGL((grouped_gemm_wide_kernel<m, t>), dim3(grid), dim3(512), lds, st, g)
+  if (mode == GEMM_PLAIN && tiles == 1) GLM53_WIDE_DENSE(GEMM_PLAIN, 1);
+  else if (mode == GEMM_PLAIN && tiles == 2) GLM53_WIDE_DENSE(GEMM_PLAIN, 2);
+  else if (mode == GEMM_PLAIN && tiles == kWideTilesPerWave) GLM53_WIDE_DENSE(GEMM_PLAIN, kWideTilesPerWave);
+  else if (mode == GEMM_SWIGLU && tiles == 2) GLM53_WIDE_DENSE(GEMM_SWIGLU, 2);
+  else if (mode == GEMM_SWIGLU && tiles == kWideTilesPerWave) GLM53_WIDE_DENSE(GEMM_SWIGLU, kWideTilesPerWave);
   else return hipErrorInvalidValue;
 #undef GLM53_WIDE_DENSE
   return hipGetLastError();

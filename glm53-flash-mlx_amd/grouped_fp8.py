@@ -21,7 +21,7 @@ import torch
 from . import _native as N
 from . import ops
 from .abi import GROUPED_MIN_ROUTES
-from .fp8 import BLOCK_SIZE, BlockFP8Linear, ClampedMLP, _scale_shape
+from .fp8 import BLOCK_SIZE, BlockFP8Linear, ClampedMLP, _hooked, _scale_shape
 from .packed import PackedFP8MoE, _c_shared
 from .router import Float32Gate
 
@@ -30,14 +30,6 @@ PLAN_MAX_EXPERTS = 1024  # the route plan's expert bound (kPlanMaxExperts)
 GROUPED_OUTPUT_COLS = 16
 GROUPED_K_TILE = 128
 _DIRECT_PLAN_ROUTES = 4096  # native_direct's scratch stays near 100 MB at H = 4096
-
-
-def _hooked(module) -> bool:
-    """Whether calling `module` would run more than its forward."""
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
-                or module._backward_pre_hooks or "forward" in module.__dict__
-                or torch.nn.modules.module._global_forward_hooks
-                or torch.nn.modules.module._global_forward_pre_hooks)
 
 
 def _route_plan(expert_ids: torch.Tensor, scores: torch.Tensor | None, top_k: int, expert_count: int,

@@ -181,6 +181,17 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
                      const float* scale_inv, const int32_t* code_flags, void* y, void* workspace,
                      size_t workspace_bytes, void* stream);
 
+/* ClampedMLP (patch.py:114-129) over two or more rows in one call: y = down(T(
+ * T(g' * sigmoid(g')) * u')), g' = min(T(gate(x)), L), u' = clip(T(up(x)), -L,
+ * L) -- the bits of glm53_fp8_linear, glm53_activate_gate_up and
+ * glm53_fp8_linear composed, with x split once and the SwiGLU formed in the
+ * gate/up product's epilogue.  x bf16 [M, H], y bf16 [M, H]; H and I
+ * multiples of 128, weights 16-byte aligned; workspace (device, 256-byte
+ * aligned) of glm53_mlp_workspace_bytes bytes, 0 for shapes not taken. */
+size_t glm53_mlp_workspace_bytes(int64_t M, int64_t hidden, int64_t intermediate);
+int glm53_mlp(const glm53_shared_expert* mlp, float limit, const void* x, int64_t M, void* y, void* workspace,
+              size_t workspace_bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Router -- replaces patch.py:131-142 `Float32Gate.__call__` (with the
  * selection half of mlx-vlm dsv32.group_expert_select, group-limited when

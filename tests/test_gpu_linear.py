@@ -115,6 +115,39 @@ def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
     assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
 
 
+@pytest.mark.parametrize("with_480", [False, True])
+@pytest.mark.parametrize("rows", [2, 33, 150, 300, 700, 1300, 6000, 12000])
+def test_mlp_in_one_call_equals_its_parts(M, dev, rows, with_480):
+    """ClampedMLP over two or more rows runs as one native call: the bytes of
+    gate_proj, up_proj, swiglu and down_proj called in turn (a hook on one of
+    them keeps the parts), in every tile of the SwiGLU form and of the down
+    product, rows and columns ragged, codes 0x7F / 0xFF in one matrix each."""
+    import torch
+
+    hidden, inter = 256, 640
+    gen = torch.Generator().manual_seed(rows)
+    for marked in ("gate_proj", "up_proj", "down_proj") if with_480 else ("none",):
+        mlp = M.ClampedMLP(hidden, inter, 2.0, device=dev)
+        for name in ("gate_proj", "up_proj", "down_proj"):
+            proj = getattr(mlp, name)
+            codes = torch.randint(0, 0x7F, tuple(proj.weight.shape), generator=gen, dtype=torch.uint8)
+            codes |= torch.randint(0, 2, tuple(codes.shape), generator=gen, dtype=torch.uint8) << 7
+            if name == marked:
+                codes[-1, -1], codes[3, 200] = 0xFF, 0x7F
+            proj.weight.copy_(codes)
+            proj.weight_scale_inv.copy_(torch.rand(tuple(proj.weight_scale_inv.shape), generator=gen) * 0.002)
+        x = torch.randn((1, rows, 2 * hidden), generator=gen).to(dev, torch.bfloat16)[..., ::2]
+        assert mlp._one_call(x)
+        y = mlp(x)
+        hook = mlp.up_proj.register_forward_hook(lambda module, args, out: None)
+        assert not mlp._one_call(x)
+        assert torch.equal(y.view(torch.int16), mlp(x).view(torch.int16)), (rows, marked)
+        hook.remove()
+    assert not mlp._one_call(x[:, :1]) and not mlp._one_call(x.float())
+    with pytest.raises(ValueError):
+        mlp(x[..., :128])
+
+
 @pytest.mark.parametrize("rows", [1, 5, 64])
 def test_both_480_codes_gemv_and_mfma(M, O, dev, rows):
     """Codes over the whole byte range, so 0x7F (+480) and 0xFF (-480) both
