@@ -218,6 +218,39 @@ def test_reductions_at_any_width_and_alignment_match_oracle(M, O, dev, hidden, o
     assert np.array_equal(to_bits(out), want)
 
 
+@pytest.mark.parametrize("k,hidden", [(1, 64), (5, 72), (8, 2056), (8, 63), (16, 64)])
+def test_direct_reduction_order_with_equal_and_missing_experts(O, dev, k, hidden):
+    """Ascending expert id, equal ids in slot order, a route without a sorted
+    position NaN: top_k 8 (its own form) and others, 8 columns and 1 column
+    per thread, against the accumulation written out in BF16 steps."""
+    import torch
+
+    N = submodule("_native")
+    rng = np.random.default_rng(10 * k + hidden)
+    tokens = 6
+    route = O.f32_to_bf16(rng.normal(size=(tokens * k, hidden)).astype(np.float32))
+    ids = rng.integers(0, 6, size=(tokens, k)).astype(np.int32)
+    ids[0] = np.arange(k)[::-1]
+    scores = rng.uniform(size=(tokens, k)).astype(np.float32)
+    inverse = rng.permutation(tokens * k).astype(np.int32)
+    inverse[-1] = -1
+    out = torch.empty((tokens, hidden), dtype=torch.bfloat16, device=dev)
+    put = lambda a: torch.from_numpy(np.ascontiguousarray(a.reshape(-1))).to(dev)  # noqa: E731
+    route_d, inv_d, ids_d, scores_d = from_bits(route, dev), put(inverse), put(ids), put(scores)
+    N.check(N.lib().glm53_direct_order_reduce(N.ptr(route_d), N.ptr(inv_d), N.ptr(ids_d), N.ptr(scores_d), tokens, k,
+                                              hidden, None, N.ptr(out), N.stream_handle(dev)))
+    rnd = lambda v: O.bf16_to_f32(O.f32_to_bf16(v.astype(np.float32)))  # noqa: E731
+    rows = O.bf16_to_f32(route)
+    want = np.zeros((tokens, hidden), np.float32)
+    for t in range(tokens):
+        for slot in np.argsort(ids[t], kind="stable"):
+            pos = inverse[t * k + slot]
+            row = rows[pos] if pos >= 0 else np.full(hidden, np.nan, np.float32)
+            want[t] = rnd(want[t] + rnd(row * scores[t, slot]))
+    got = out.float().cpu().numpy()
+    assert np.array_equal(got[:-1], want[:-1]) and np.isnan(got[-1]).all()
+
+
 def test_grouped_linear_unaligned_activations_split_alike(M, O, dev):
     """Activation rows that are only 2-byte aligned take the two-column split;
     the GEMM output equals the aligned run bit for bit."""
