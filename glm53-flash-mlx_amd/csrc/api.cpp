@@ -78,7 +78,7 @@ SplitBuf carve_split(void* base, int64_t rows, int64_t cols) {
   return b;
 }
 
-hipError_t split(const void* x, int64_t rows, int64_t cols, const SplitBuf& b, hipStream_t st) {
+SplitArgs split_args(const void* x, int64_t rows, int64_t cols, const SplitBuf& b) {
   SplitArgs a{};
   a.x = static_cast<const uint16_t*>(x);
   a.x_row_stride = cols;
@@ -87,7 +87,11 @@ hipError_t split(const void* x, int64_t rows, int64_t cols, const SplitBuf& b, h
   a.hi = b.hi;
   a.lo = b.lo;
   a.scale = b.scale;
-  return launch_split_activations(a, st);
+  return a;
+}
+
+hipError_t split(const void* x, int64_t rows, int64_t cols, const SplitBuf& b, hipStream_t st) {
+  return launch_split_activations(split_args(x, rows, cols, b), st);
 }
 
 // One dense problem, plain or SwiGLU, on split activations, in the shape that
@@ -1330,7 +1334,7 @@ int route_plan_impl(const int32_t* expert_ids, const float* scores, int64_t rout
                     int64_t tile_rows, int32_t* sorted_route, int32_t* inverse, int32_t* sorted_expert,
                     int32_t* sorted_token, float* sorted_score, uint32_t* route_offsets, uint32_t* tile_offsets,
                     int32_t* tile_expert, int32_t* tile_start, int32_t* tile_len, int64_t capacity, uint32_t* status,
-                    void* workspace, hipStream_t st) {
+                    void* workspace, hipStream_t st, const SplitArgs* with_split = nullptr) {
   RoutePlanArgs a{};
   a.expert_ids = expert_ids;
   a.scores = scores;
@@ -1354,7 +1358,7 @@ int route_plan_impl(const int32_t* expert_ids, const float* scores, int64_t rout
   a.tile_start = tile_start;
   a.tile_len = tile_len;
   a.status = status;
-  HIP_TRY(launch_route_plan(a, st), "route plan launch");
+  HIP_TRY(launch_route_plan(a, with_split, st), "route plan launch");
   return GLM53_OK;
 }
 
@@ -1730,8 +1734,8 @@ static int prefill_run(glm53_prefill_plan* p, const glm53_bank* bank, const glm5
       shared_down_flag = p->flags + 3;
     }
   }
-  // 1. activations -> exact hi/lo E4M3 split
-  HIP_TRY(split(x, T, H, p->xq, st), "split x");
+  // 1. activations -> exact hi/lo E4M3 split (launched with the route plan)
+  const SplitArgs x_split = split_args(x, T, H, p->xq);
   // 2. expert-sorted route plan: 128-route descriptors (the wide GEMM shape)
   // when experts average at least 48 routes, 64-route ones from 32 (fewer
   // re-reads of each weight tile), 32-route ones (a deeper load ring per
@@ -1742,7 +1746,7 @@ static int prefill_run(glm53_prefill_plan* p, const glm53_bank* bank, const glm5
   const int64_t cap = cdiv(R, tile) + E;
   if ((rc = route_plan_impl(ids, sc, R, k, E, tile, p->sorted_route, p->inverse, p->sorted_expert,
                             p->sorted_token, p->sorted_score, p->route_offsets, p->tile_offsets, p->tile_expert,
-                            p->tile_start, p->tile_len, cap, p->status, p->plan_ws, st)))
+                            p->tile_start, p->tile_len, cap, p->status, p->plan_ws, st, &x_split)))
     return rc;
   // 3. grouped gate/up + SwiGLU (token rows gathered through sorted_token);
   // with a shared expert of the routed width, its dense gate/up (all T

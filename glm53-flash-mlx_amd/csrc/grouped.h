@@ -7,6 +7,7 @@
 namespace glm53 {
 
 constexpr int kPlanMaxExperts = 1024;
+constexpr int64_t kPlanOneLaunchRoutes = 2048;  // route plans up to here run as one workgroup
 constexpr int kGroupedTileRows = 32;   // routes per descriptor of the reference (grouped_fp8.py:20)
 constexpr int kGemmTileRows = 64;      // routes per descriptor of the MFMA grouped GEMM (many routes per expert)
 constexpr int kGemmMinTileRows = 32;   // its narrow form (one group per wavefront, deeper ring)
@@ -128,7 +129,8 @@ struct ReduceArgs {
 };
 constexpr int kHcBranches = 4;
 
-hipError_t launch_route_plan(const RoutePlanArgs& a, hipStream_t st);
+// split: an activation split of the same call to run beside the plan, or null
+hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hipStream_t st);
 hipError_t launch_split_activations(const SplitArgs& a, hipStream_t st);
 hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descriptors, hipStream_t st);
 // tile_expert / tile_start / tile_len set by the caller; descriptors of up to

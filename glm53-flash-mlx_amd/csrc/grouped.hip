@@ -81,6 +81,45 @@ __device__ void block_scan2_inclusive(unsigned* a, unsigned* b, int n) {
   __syncthreads();
 }
 
+// Offsets, status and descriptors from the inclusive scans in LDS (one
+// workgroup of 1024 threads).
+__device__ __forceinline__ void write_plan_tables(const RoutePlanArgs& a, const unsigned* route_cum,
+                                                  const unsigned* tile_cum, unsigned invalid_total) {
+  const int t = threadIdx.x;
+  if (t < a.experts) {
+    a.route_offsets[t + 1] = route_cum[t];
+    a.tile_offsets[t + 1] = tile_cum[t];
+  }
+  if (t == 0) {
+    a.route_offsets[0] = 0;
+    a.tile_offsets[0] = 0;
+    a.status[0] = invalid_total;                       // invalid route count
+    a.status[1] = tile_cum[a.experts - 1];             // valid descriptors
+  }
+  // descriptors: owner by binary search over the inclusive tile scan
+  const unsigned total_tiles = tile_cum[a.experts - 1];
+  for (int64_t d = t; d < a.capacity; d += 1024) {
+    if (d >= total_tiles) {
+      a.tile_expert[d] = 0;
+      a.tile_start[d] = static_cast<int32_t>(a.routes);
+      a.tile_len[d] = 0;
+      continue;
+    }
+    int lo = 0, hi = a.experts - 1;
+    while (lo < hi) {  // first e with tile_cum[e] > d
+      int mid = (lo + hi) >> 1;
+      if (tile_cum[mid] > d) hi = mid; else lo = mid + 1;
+    }
+    const unsigned first_tile = lo == 0 ? 0 : tile_cum[lo - 1];
+    const unsigned first_route = lo == 0 ? 0 : route_cum[lo - 1];
+    const unsigned start = first_route + (static_cast<unsigned>(d) - first_tile) * a.tile_rows;
+    const unsigned end = route_cum[lo];
+    a.tile_expert[d] = lo;
+    a.tile_start[d] = static_cast<int32_t>(start);
+    a.tile_len[d] = static_cast<int32_t>(end - start < static_cast<unsigned>(a.tile_rows) ? end - start : a.tile_rows);
+  }
+}
+
 __global__ __launch_bounds__(1024) void route_scan_kernel(RoutePlanArgs a) {
   __shared__ unsigned route_cum[kPlanMaxExperts];
   __shared__ unsigned tile_cum[kPlanMaxExperts];
@@ -123,38 +162,7 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(RoutePlanArgs a) {
   for (int64_t b = t; b < a.blocks; b += 1024) atomicAdd(&invalid_total, a.block_invalid[b]);
   __syncthreads();
   block_scan2_inclusive(route_cum, tile_cum, a.experts);
-  if (t < a.experts) {
-    a.route_offsets[t + 1] = route_cum[t];
-    a.tile_offsets[t + 1] = tile_cum[t];
-  }
-  if (t == 0) {
-    a.route_offsets[0] = 0;
-    a.tile_offsets[0] = 0;
-    a.status[0] = invalid_total;                       // invalid route count
-    a.status[1] = tile_cum[a.experts - 1];             // valid descriptors
-  }
-  // descriptors: owner by binary search over the inclusive tile scan
-  const unsigned total_tiles = tile_cum[a.experts - 1];
-  for (int64_t d = t; d < a.capacity; d += 1024) {
-    if (d >= total_tiles) {
-      a.tile_expert[d] = 0;
-      a.tile_start[d] = static_cast<int32_t>(a.routes);
-      a.tile_len[d] = 0;
-      continue;
-    }
-    int lo = 0, hi = a.experts - 1;
-    while (lo < hi) {  // first e with tile_cum[e] > d
-      int mid = (lo + hi) >> 1;
-      if (tile_cum[mid] > d) hi = mid; else lo = mid + 1;
-    }
-    const unsigned first_tile = lo == 0 ? 0 : tile_cum[lo - 1];
-    const unsigned first_route = lo == 0 ? 0 : route_cum[lo - 1];
-    const unsigned start = first_route + (static_cast<unsigned>(d) - first_tile) * a.tile_rows;
-    const unsigned end = route_cum[lo];
-    a.tile_expert[d] = lo;
-    a.tile_start[d] = static_cast<int32_t>(start);
-    a.tile_len[d] = static_cast<int32_t>(end - start < static_cast<unsigned>(a.tile_rows) ? end - start : a.tile_rows);
-  }
+  write_plan_tables(a, route_cum, tile_cum, invalid_total);
 }
 
 __global__ __launch_bounds__(256) void route_scatter_kernel(RoutePlanArgs a) {
@@ -262,13 +270,11 @@ __device__ __forceinline__ void store_bf16_run(uint16_t* p, const float* v) {
 // a reduction over one 16-lane DPP row) when the rows are 16-byte aligned,
 // V = 2 (one block per wavefront) otherwise.
 template <int V>
-__global__ __launch_bounds__(256) void split_activations_kernel(SplitArgs a) {
+__device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int lane) {
   constexpr int kLanesPerBlock = kBlock / V;
   constexpr int kBlocksPerWave = 64 / kLanesPerBlock;
-  const int lane = threadIdx.x & 63;
   const int64_t blocks_per_row = a.cols / kBlock;
   const int64_t groups = (blocks_per_row + kBlocksPerWave - 1) / kBlocksPerWave;
-  const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
   if (unit >= a.rows * groups) return;
   const int64_t row = unit / groups;
   const int64_t blk = (unit % groups) * kBlocksPerWave + lane / kLanesPerBlock;
@@ -335,6 +341,109 @@ __global__ __launch_bounds__(256) void split_activations_kernel(SplitArgs a) {
     *reinterpret_cast<uint16_t*>(a.lo + off) = static_cast<uint16_t>(lo[0]);
   }
   if (lane % kLanesPerBlock == 0) a.scale[row * blocks_per_row + blk] = s;
+}
+
+template <int V>
+__global__ __launch_bounds__(256) void split_activations_kernel(SplitArgs a) {
+  split_unit<V>(a, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+}
+
+// The whole route plan of up to kPlanOneLaunchRoutes routes in one workgroup
+// of 16 wavefronts; wavefront w ranks the routes of its own run of B
+// batches of 64, held in registers from one round of loads.  A lane's peers
+// (same id in its batch) come from one ballot per id bit, so a batch costs
+// ~12 ballots and one LDS counter round trip instead of a loop over the
+// routes before it; the wavefront's counters per expert then turn into its
+// bases by one pass over the 16 rows.  Bound by latency: 5.4 us at 512
+// routes and 8.4 at 2,048 over 288 experts, where the three launches take
+// 11.7 and 12.3; at 3,072 and 4,096 (11.7 and 13.7 with four batches against
+// 13.3 and 13.0) one workgroup's batches cost what the launches do, so
+// larger plans keep those.
+constexpr int kPlanWaves = 16;
+template <int B>
+__device__ __forceinline__ void route_plan_one(const RoutePlanArgs& a, int id_bits, unsigned* hist,
+                                               unsigned* route_cum, unsigned* tile_cum, unsigned* invalid_total) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, E = a.experts;
+  unsigned* mine = hist + w * E;
+  int32_t id[B];
+  unsigned rank[B];
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const int64_t i = (static_cast<int64_t>(w) * B + b) * 64 + lane;
+    id[b] = i < a.routes ? a.expert_ids[i] : -1;
+  }
+  for (int e = lane; e < E; e += 64) mine[e] = 0;
+  if (t == 0) *invalid_total = 0;
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const int64_t i = (static_cast<int64_t>(w) * B + b) * 64 + lane;
+    const bool valid = id[b] >= 0 && id[b] < E;
+    const unsigned long long bad = __ballot(i < a.routes && !valid);
+    if (lane == 0 && bad != 0) atomicAdd(invalid_total, static_cast<unsigned>(__popcll(bad)));
+    unsigned long long peers = __ballot(valid);
+    for (int bit = 0; bit < id_bits; ++bit) {
+      const bool one = (id[b] >> bit) & 1;
+      const unsigned long long ones = __ballot(one);
+      peers &= one ? ones : ~ones;
+    }
+    const unsigned before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers), 0u));
+    rank[b] = valid ? mine[id[b]] + before : 0u;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every peer has read the counter
+    if (valid && before == 0) mine[id[b]] = rank[b] + static_cast<unsigned>(__popcll(peers));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next batch reads it
+  }
+  __syncthreads();
+  if (t < E) {
+    unsigned c[kPlanWaves], run = 0;
+#pragma unroll
+    for (int j = 0; j < kPlanWaves; ++j) c[j] = hist[j * E + t];
+#pragma unroll
+    for (int j = 0; j < kPlanWaves; ++j) {
+      hist[j * E + t] = run;
+      run += c[j];
+    }
+    route_cum[t] = run;
+    tile_cum[t] = (run + a.tile_rows - 1) / a.tile_rows;
+  }
+  __syncthreads();
+  block_scan2_inclusive(route_cum, tile_cum, E);
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const int64_t i = (static_cast<int64_t>(w) * B + b) * 64 + lane;
+    const int32_t e = id[b];
+    if (i >= a.routes) continue;
+    if (e < 0 || e >= E) {
+      a.inverse[i] = -1;
+      continue;
+    }
+    const int64_t pos = static_cast<int64_t>((e == 0 ? 0u : route_cum[e - 1]) + mine[e] + rank[b]);
+    a.sorted_route[pos] = static_cast<int32_t>(i);
+    a.inverse[i] = static_cast<int32_t>(pos);
+    a.sorted_expert[pos] = e;
+    a.sorted_token[pos] = static_cast<int32_t>(static_cast<uint32_t>(i) / static_cast<uint32_t>(a.top_k));
+    if (a.scores != nullptr) a.sorted_score[pos] = a.scores[i];
+  }
+  write_plan_tables(a, route_cum, tile_cum, *invalid_total);
+}
+
+// Workgroup 0: the plan.  The others: the activation split of the same call
+// (V as in split_activations_kernel; s.rows = 0: none), which needs nothing
+// of the plan and would otherwise be a launch of its own.
+template <int V>
+__global__ __launch_bounds__(1024) void route_plan_one_kernel(RoutePlanArgs a, int id_bits, SplitArgs s) {
+  extern __shared__ unsigned plan_hist[];  // [kPlanWaves][experts]
+  __shared__ unsigned route_cum[kPlanMaxExperts];
+  __shared__ unsigned tile_cum[kPlanMaxExperts];
+  __shared__ unsigned invalid_total;
+  if (blockIdx.x > 0) {
+    split_unit<V>(s, static_cast<int64_t>(blockIdx.x - 1) * kPlanWaves + (threadIdx.x >> 6), threadIdx.x & 63);
+    return;
+  }
+  static_assert(kPlanOneLaunchRoutes <= 2 * 64 * kPlanWaves, "two batches per wavefront at most");
+  if (a.routes <= 64 * kPlanWaves) route_plan_one<1>(a, id_bits, plan_hist, route_cum, tile_cum, &invalid_total);
+  else route_plan_one<2>(a, id_bits, plan_hist, route_cum, tile_cum, &invalid_total);
 }
 
 // --------------------------------------------------------- grouped GEMM --
@@ -1515,25 +1624,43 @@ __global__ __launch_bounds__(256) void direct_order_reduce_kernel(ReduceArgs a) 
 
 // ------------------------------------------------------------- launchers --
 
-hipError_t launch_route_plan(const RoutePlanArgs& a, hipStream_t st) {
-  if (a.blocks > 0) {
-    hipLaunchKernelGGL(route_count_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(256), 0, st, a);
+namespace {
+bool split_wide(const SplitArgs& a) { return a.x_row_stride % 8 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0; }
+int64_t split_units(const SplitArgs& a) {  // wavefronts
+  const int64_t blocks_per_row = a.cols / kBlock;
+  return a.rows * (split_wide(a) ? (blocks_per_row + 3) / 4 : blocks_per_row);
+}
+}  // namespace
+
+hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hipStream_t st) {
+  if (a.routes <= kPlanOneLaunchRoutes) {
+    SplitArgs s{};
+    if (split != nullptr) s = *split;
+    if (s.cols % kBlock != 0) return hipErrorInvalidValue;
+    int id_bits = 0;
+    while ((1 << id_bits) < a.experts) ++id_bits;
+    const int64_t split_blocks = s.rows > 0 ? (split_units(s) + kPlanWaves - 1) / kPlanWaves : 0;
+    const dim3 grid(static_cast<unsigned>(1 + split_blocks));
+    const size_t lds = sizeof(unsigned) * static_cast<size_t>(kPlanWaves * a.experts);
+    if (split_wide(s)) hipLaunchKernelGGL(route_plan_one_kernel<8>, grid, dim3(64 * kPlanWaves), lds, st, a, id_bits, s);
+    else hipLaunchKernelGGL(route_plan_one_kernel<2>, grid, dim3(64 * kPlanWaves), lds, st, a, id_bits, s);
+    return hipGetLastError();
   }
+  if (split != nullptr) {
+    const hipError_t e = launch_split_activations(*split, st);
+    if (e != hipSuccess) return e;
+  }
+  hipLaunchKernelGGL(route_count_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(256), 0, st, a);
   hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), 0, st, a);
-  if (a.blocks > 0) {
-    hipLaunchKernelGGL(route_scatter_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(256), 0, st, a);
-  }
+  hipLaunchKernelGGL(route_scatter_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
 hipError_t launch_split_activations(const SplitArgs& a, hipStream_t st) {
   if (a.rows == 0) return hipSuccess;
   if (a.cols % kBlock != 0) return hipErrorInvalidValue;
-  const bool wide = a.x_row_stride % 8 == 0 && reinterpret_cast<uintptr_t>(a.x) % 16 == 0;
-  const int64_t blocks_per_row = a.cols / kBlock;
-  const int64_t units = a.rows * (wide ? (blocks_per_row + 3) / 4 : blocks_per_row);  // wavefronts
-  const dim3 grid(static_cast<unsigned>((units + 3) / 4));
-  if (wide) hipLaunchKernelGGL(split_activations_kernel<8>, grid, dim3(256), 0, st, a);
+  const dim3 grid(static_cast<unsigned>((split_units(a) + 3) / 4));
+  if (split_wide(a)) hipLaunchKernelGGL(split_activations_kernel<8>, grid, dim3(256), 0, st, a);
   else hipLaunchKernelGGL(split_activations_kernel<2>, grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
