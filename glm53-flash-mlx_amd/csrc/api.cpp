@@ -253,7 +253,7 @@ int route_tokens(const glm53_router* r, const void* x, int64_t T, float* space, 
     g.expert_groups = shape.expert_groups;
     g.k_chunk = shape.k_chunk;
     g.splits = shape.splits;
-    HIP_TRY(launch_router_logits(g, r->weight, st), "router logits launch");
+    HIP_TRY(launch_router_logits(g, shape.few_tokens, r->weight, st), "router logits launch");
     return topk(g.partial, r, T, ids, scores, st, static_cast<int>(shape.splits), T * E);
   }
   RouterArgs a{};

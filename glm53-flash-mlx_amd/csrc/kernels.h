@@ -208,10 +208,11 @@ struct RouterGemmArgs {
 constexpr int kMaxRouterSplits = 16;
 struct RouterGemmShape {
   int64_t token_groups, expert_groups, k_chunk, splits;  // splits <= kMaxRouterSplits
+  bool few_tokens;  // 32 x 32 tiles
 };
 bool router_gemm_supported(int64_t hidden, int64_t experts, const void* x, const void* weight);
 RouterGemmShape router_gemm_shape(int64_t tokens, int64_t hidden, int64_t experts);
-hipError_t launch_router_logits(const RouterGemmArgs& a, const float* weight, hipStream_t st);
+hipError_t launch_router_logits(const RouterGemmArgs& a, bool few_tokens, const float* weight, hipStream_t st);
 hipError_t launch_linear_generic(const GenericLinearArgs& a, hipStream_t st);
 hipError_t launch_swiglu(const SwigluArgs& a, hipStream_t st);
 hipError_t launch_swiglu_stages(const SwigluArgs& a, uint16_t* sigma, uint16_t* silu, hipStream_t st);

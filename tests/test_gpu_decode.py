@@ -138,7 +138,8 @@ def test_router_matches_oracle(O, config2_layer, dev, tokens):
 
 @pytest.mark.parametrize("tokens,hidden,experts", [(333, 4096, 288), (1024, 4096, 288), (2048, 4096, 288),
                                                    (100, 1024, 200), (77, 512, 512), (40, 256, 320), (50, 384, 64),
-                                                   (5, 200, 16), (3, 201, 16)])
+                                                   (2, 4096, 288), (31, 128, 33), (33, 640, 97), (256, 4096, 288),
+                                                   (384, 4096, 288), (5, 200, 16), (3, 201, 16)])
 def test_router_many_tokens_matches_oracle(M, O, dev, tokens, hidden, experts):
     """Many-token router: for any token count (2048 included) the
     hand-written BF16 MFMA tile kernel over the exact three-way BF16 split of
