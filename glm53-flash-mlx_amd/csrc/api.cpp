@@ -94,12 +94,18 @@ hipError_t split(const void* x, int64_t rows, int64_t cols, const SplitBuf& b, h
   return launch_split_activations(split_args(x, rows, cols, b), st);
 }
 
-// One dense problem, plain or SwiGLU, on split activations, in the shape that
-// dense_tile names.  `flags`: device int32 [1] (SwiGLU: [2]) for the weights
-// that come without a code flag where the shape does not look for the codes
-// itself.
-int dense(const DenseArgs& d, bool swiglu, int32_t* flags, hipStream_t st) {
+// One dense problem, plain or SwiGLU, in the shape that dense_tile names: x
+// bf16 [d.rows, d.K] is split into `space` (d's planes) and multiplied.
+// `flags`: device int32 [1] (SwiGLU: [2]) for the weights that come without a
+// code flag where the shape does not look for the codes itself.
+int dense(DenseArgs d, const void* x, const SplitBuf& space, bool swiglu, int32_t* flags, hipStream_t st) {
   const DenseTile tile = dense_tile(d.rows, d.K, d.N, swiglu);
+  SplitArgs sp = split_args(x, d.rows, d.K, space);
+  sp.operand_order = dense_ksplit(tile, swiglu);
+  HIP_TRY(launch_split_activations(sp, st), "split launch");
+  d.a_hi = space.hi;
+  d.a_lo = space.lo;
+  d.a_scale = space.scale;
   if (dense_ksplit(tile, swiglu)) {
     HIP_TRY(launch_dense_linear(d, tile, swiglu, st), "dense linear launch");
     return GLM53_OK;
@@ -431,11 +437,7 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
   const size_t need = glm53_fp8_linear_workspace_bytes(M, N, K);
   if (need > 0 && aligned(weight, 16) && workspace != nullptr && workspace_bytes >= need) {
     SplitBuf b = carve_split(workspace, M, K);
-    HIP_TRY(split(x, M, K, b, st), "split launch");
     DenseArgs d{};
-    d.a_hi = b.hi;
-    d.a_lo = b.lo;
-    d.a_scale = b.scale;
     d.weight = weight;
     d.scale = scale_inv;
     d.flag = code_flags;
@@ -443,7 +445,7 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
     d.K = K;
     d.N = N;
     d.out = static_cast<uint16_t*>(y);
-    return dense(d, false, reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + split_bytes(M, K)), st);
+    return dense(d, x, b, false, reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + split_bytes(M, K)), st);
   }
   GenericLinearArgs a{};
   a.x = static_cast<const uint16_t*>(x);
@@ -510,11 +512,7 @@ int glm53_mlp(const glm53_shared_expert* mlp, float limit, const void* x, int64_
             "mlp weights must be 16-byte aligned");
   hipStream_t st = S(stream);
   const MlpSpace s = mlp_space(workspace, M, H, I);
-  HIP_TRY(split(x, M, H, s.xq, st), "split launch");
   DenseArgs g{};
-  g.a_hi = s.xq.hi;
-  g.a_lo = s.xq.lo;
-  g.a_scale = s.xq.scale;
   g.weight = mlp->gate.weight;
   g.scale = mlp->gate.scale_inv;
   g.flag = mlp->gate.code_flags;
@@ -526,12 +524,8 @@ int glm53_mlp(const glm53_shared_expert* mlp, float limit, const void* x, int64_
   g.K = H;
   g.N = I;
   g.out = s.h;
-  if (int rc = dense(g, true, s.flags, st)) return rc;
-  HIP_TRY(split(s.h, M, I, s.hq, st), "split launch");
+  if (int rc = dense(g, x, s.xq, true, s.flags, st)) return rc;
   DenseArgs d{};
-  d.a_hi = s.hq.hi;
-  d.a_lo = s.hq.lo;
-  d.a_scale = s.hq.scale;
   d.weight = mlp->down.weight;
   d.scale = mlp->down.scale_inv;
   d.flag = mlp->down.code_flags;
@@ -539,7 +533,7 @@ int glm53_mlp(const glm53_shared_expert* mlp, float limit, const void* x, int64_
   d.K = I;
   d.N = H;
   d.out = static_cast<uint16_t*>(y);
-  return dense(d, false, s.flags + 2, st);
+  return dense(d, s.h, s.hq, false, s.flags + 2, st);
 }
 
 // ------------------------------------------------------------ router ------

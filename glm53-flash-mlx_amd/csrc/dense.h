@@ -7,7 +7,7 @@
 namespace glm53 {
 
 struct DenseArgs {
-  const uint8_t* a_hi;     // [rows, K] split activations
+  const uint8_t* a_hi;     // [rows, K] split activations; for launch_dense_linear in MFMA operand order
   const uint8_t* a_lo;
   const float* a_scale;    // [rows, K / 128]
   const uint8_t* weight;   // [N, K], 16-byte aligned

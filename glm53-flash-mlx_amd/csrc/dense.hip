@@ -29,15 +29,9 @@ template <int P, int C>
 constexpr int load_depth() {
   return P * C <= 2 ? 4 : 2;
 }
-// Operand tiles a wavefront passes through its own LDS buffer at a time
-template <int P, int C>
-constexpr int turn_tiles() {
-  return C > 2 * P ? C : 2 * P;
-}
-
 template <int P, int C>
 size_t dense_lds_bytes(int64_t K) {
-  return static_cast<size_t>(kDenseWaves) * (fold_steps<P, C>() * P * C * 1024 + turn_tiles<P, C>() * kOperand) +
+  return static_cast<size_t>(kDenseWaves) * (fold_steps<P, C>() * P * C * 1024 + C * kOperand) +
          2 * sizeof(float) * static_cast<size_t>(K / kBlock);
 }
 
@@ -46,10 +40,14 @@ size_t dense_lds_bytes(int64_t K) {
 // of the tiles and the matching up rows in the second.  Wavefront w
 // multiplies K blocks w, w + 8, ...: its operands come from global memory
 // into registers (each byte of the item's rows and columns once per
-// workgroup), load_depth steps ahead, 8 rows of whole 128-byte lines per
-// load, and turn into MFMA order through an LDS buffer of its own, so no
-// barrier is waited at in between.  (Loads in MFMA order, 16 rows per load,
-// ran at a third of this rate: neighbouring lanes in different lines.)
+// workgroup), load_depth steps ahead, so no barrier is waited at in between.
+// The activations lie in operand order and are multiplied as loaded; the
+// weight rows come 8 whole 128-byte lines per load and turn into operand
+// order through an LDS buffer of the wavefront's own.  (Loading row-major
+// bytes in operand order, 16 rows per load, ran at a third of this rate,
+// neighbouring lanes in different lines; turning the activations through LDS
+// too cost 300 x 1536 x 4096 13.9 us instead of 12.4, 16 x 4096 x 4096 7.2
+// instead of 6.6.)
 // A block's MFMA results (hi rows, then lo rows, before the weight scale) go
 // to LDS, and wavefront t < P C adds tile t's results in block order, so
 // every output goes through the operations of the grouped GEMM and has its
@@ -66,22 +64,25 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   const int steps = (KB + kDenseWaves - 1) / kDenseWaves;
   constexpr int kFold = kDenseWaves * fold_steps<P, C>() * P * C * 1024;
   f32x4* lds_c = reinterpret_cast<f32x4*>(lds);                                          // [8 F][P C][64]
-  uint8_t* turn = lds + kFold + wave * turn_tiles<P, C>() * kOperand;                    // this wavefront's
-  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * turn_tiles<P, C>() * kOperand);  // [2][KB]
+  uint8_t* turn = lds + kFold + wave * C * kOperand;                    // this wavefront's
+  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * C * kOperand);  // [2][KB]
   const OperandSlots slots = operand_slots(lane);
 
   // rows past the last repeat it, columns past the matrix its last row: valid
   // bytes whose results are never stored (offsets from wave-uniform bases;
   // the launcher keeps them below 2^32)
-  uint32_t arow[P][2], srow[P], wrow[C][2];
+  uint32_t aoff[P], srow[P], wrow[C][2];
+  int64_t apair[P];  // the pair's bytes in the planes
+  int arows[P];      // and rows
 #pragma unroll
   for (int p = 0; p < P; ++p) {
     const int64_t last = a.rows - 1;
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int64_t m = row0 + 16 * p + 8 * h + (lane >> 3);
-      arow[p][h] = static_cast<uint32_t>((m < last ? m : last) * K + load_piece_offset(lane, h));
-    }
+    int64_t pair = row0 / 16 + p;
+    pair = pair < last / 16 ? pair : last / 16;
+    const int64_t left = a.rows - 16 * pair;
+    arows[p] = left < 16 ? static_cast<int>(left) : 16;
+    apair[p] = 16 * pair * K;
+    aoff[p] = static_cast<uint32_t>(16 * ((r < arows[p] ? r : arows[p] - 1) + arows[p] * kq));
     const int64_t m = row0 + 16 * p + r;
     srow[p] = static_cast<uint32_t>((m < last ? m : last) * KB);
   }
@@ -100,14 +101,15 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
     int kb = kDenseWaves * s + wave;
     kb = kb < KB ? kb : KB - 1;  // past the end: loaded, never folded
     const int64_t ko = static_cast<int64_t>(kb) * kBlock;  // wave-uniform
-    const uint8_t *w = a.weight + ko, *up = SWIGLU ? a.weight_up + ko : w, *hi = a.a_hi + ko, *lo = a.a_lo + ko;
+    const uint8_t *w = a.weight + ko, *up = SWIGLU ? a.weight_up + ko : w;
     const float* se = a.a_scale + kb;
 #pragma unroll
     for (int p = 0; p < P; ++p) {
+      const int64_t block = apair[p] + ko * arows[p];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        v.h[p][h] = *reinterpret_cast<const u32x4*>(hi + arow[p][h]);
-        v.l[p][h] = *reinterpret_cast<const u32x4*>(lo + arow[p][h]);
+        v.h[p][h] = *reinterpret_cast<const u32x4*>(a.a_hi + block + 64 * h * arows[p] + aoff[p]);
+        v.l[p][h] = *reinterpret_cast<const u32x4*>(a.a_lo + block + 64 * h * arows[p] + aoff[p]);
       }
       v.s[p] = se[srow[p]];
     }
@@ -115,6 +117,10 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
     for (int c = 0; c < C; ++c)
 #pragma unroll
       for (int h = 0; h < 2; ++h) v.b[c][h] = *reinterpret_cast<const u32x4*>((c < H ? w : up) + wrow[c][h]);
+  };
+  auto vec = [](const u32x4 (&v)[2]) {
+    return (i32x8){(int)v[0][0], (int)v[0][1], (int)v[0][2], (int)v[0][3],
+                   (int)v[1][0], (int)v[1][1], (int)v[1][2], (int)v[1][3]};
   };
   auto put = [&](int tile, const u32x4 (&v)[2]) {
 #pragma unroll
@@ -135,19 +141,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   uint32_t found = 0;
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   auto multiply = [&](int slot, const Step& v) {  // the step's results into slot (block slot of the fold)
-    i32x8 ah[P], al[P], b[C], bc[1];
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      put(2 * p, v.h[p]);
-      put(2 * p + 1, v.l[p]);
-    }
-    turned();
-#pragma unroll
-    for (int p = 0; p < P; ++p) {
-      ah[p] = lds_operand(turn + 2 * p * kOperand, slots);
-      al[p] = lds_operand(turn + (2 * p + 1) * kOperand, slots);
-    }
-    turned();
+    i32x8 b[C], bc[1];
 #pragma unroll
     for (int c = 0; c < C; ++c) put(c, v.b[c]);
     turned();
@@ -169,8 +163,8 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
 #pragma unroll
         for (int p = 0; p < P; ++p) {
           const int e = static_cast<int>(scale_e8m0(v.s[p]));
-          const f32x4 x = pair_pass<FIX, 0, 127>(ah[p], b[c], bc[0], kZero, e);
-          lds_c[(slot * P * C + p * C + c) * 64 + lane] = pair_pass<FIX, 0, 123>(al[p], b[c], bc[0], x, e);
+          const f32x4 x = pair_pass<FIX, 0, 127>(vec(v.h[p]), b[c], bc[0], kZero, e);
+          lds_c[(slot * P * C + p * C + c) * 64 + lane] = pair_pass<FIX, 0, 123>(vec(v.l[p]), b[c], bc[0], x, e);
         }
       }
     } else {
@@ -179,13 +173,13 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
       for (int p = 0; p < P; ++p)
 #pragma unroll
         for (int c = 0; c < C; ++c)
-          x[p][c] = pair_pass<FIX, 0, 127>(ah[p], b[c], b[c], kZero, static_cast<int>(scale_e8m0(v.s[p])));
+          x[p][c] = pair_pass<FIX, 0, 127>(vec(v.h[p]), b[c], b[c], kZero, static_cast<int>(scale_e8m0(v.s[p])));
 #pragma unroll
       for (int p = 0; p < P; ++p)
 #pragma unroll
         for (int c = 0; c < C; ++c)
           lds_c[(slot * P * C + p * C + c) * 64 + lane] =
-              pair_pass<FIX, 0, 123>(al[p], b[c], b[c], x[p][c], static_cast<int>(scale_e8m0(v.s[p])));
+              pair_pass<FIX, 0, 123>(vec(v.l[p]), b[c], b[c], x[p][c], static_cast<int>(scale_e8m0(v.s[p])));
     }
   };
   // adds the results of the K blocks of steps s0 .. s0 + F - 1, in block order
@@ -312,9 +306,9 @@ hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
 // larger tile brings fewer bytes per output but takes longer per round, and
 // a second round costs more than the larger tile does.  Measured (us, N =
 // 4096, K = 4096, each tile at its last one-round row count and just past
-// it): 16 x 16 7.2 at 16 rows, 12.3 at 32, where 16 x 32 takes 8.4; 32 x 32
-// 10.2 at 64 rows, 18.0 at 96, where 32 x 64 takes 13.4; 32 x 64 13.7 at
-// 128, 24.6 at 200; 32 x 128 (grouped GEMM) 26.8 at 200, 40.5 at 300; 64 x
+// it): 16 x 16 6.6 at 16 rows, 12 at 32, where 16 x 32 takes 7.6; 32 x 32
+// 10.0 at 64 rows, 17.2 at 96, where 32 x 64 takes 12.7; 32 x 64 13.0 at
+// 128, 22.7 at 200; 32 x 128 (grouped GEMM) 26.8 at 200, 40.5 at 300; 64 x
 // 128 29.2 at 300 rows, 34.8 at 512 (256 items, where 128 x 128 takes 32.2:
 // its two workgroups per CU share the load path from about 224 items on);
 // 128 x 128 (wide shape) 37.6 at 1,024, 66.2 at 1,500; 128 x 256 49.0 at

@@ -55,8 +55,21 @@ struct SplitArgs {
   int64_t rows, cols;         // cols % 128 == 0
   uint8_t* hi;                // [rows, cols] E4M3
   uint8_t* lo;                // [rows, cols] E4M3 (residual * 16)
+  bool operand_order;         // hi and lo in MFMA operand order (operand_order_offset) instead of row-major
   float* scale;               // [rows, cols / 128] power of two
 };
+
+// Byte offset of element (row, col) of a split plane in MFMA operand order:
+// rows in pairs of 16 (the last one maybe fewer), a pair's 128-column blocks
+// one after the other, each block's two 64-byte halves h as [k quarter][row]
+// [16 bytes], so that an operand's lane (row l % 16, quarter l / 16) reads
+// its two 16-byte pieces where the lanes before it leave off.  The plane
+// keeps its rows x cols bytes.
+__host__ __device__ inline int64_t operand_order_offset(int64_t row, int64_t col, int64_t rows, int64_t cols) {
+  const int64_t pair = row >> 4, left = rows - 16 * pair, n = left < 16 ? left : 16;
+  const int64_t c = col & 127;
+  return 16 * pair * cols + (col >> 7) * 128 * n + ((c >> 4) & 1) * 64 * n + ((row & 15) + n * (c >> 5)) * 16 + (c & 15);
+}
 
 struct GroupedGemmArgs {
   const uint8_t* a_hi;

@@ -265,11 +265,57 @@ __device__ __forceinline__ void store_bf16_run(uint16_t* p, const float* v) {
   }
 }
 
+// A block's scale s = 2^ceil(log2(amax / 448)): amax / s lies in (224, 448].
+__device__ __forceinline__ float split_scale(float amax) {
+  float s = 1.0f;
+  if (amax > 0.0f && isfinite(amax)) {
+    int e = ilogbf(amax / 448.0f);
+    if (e < -126) e = -126;
+    s = ldexpf(1.0f, e);
+    if (amax / s > 448.0f) s = ldexpf(1.0f, e + 1);
+  }
+  return s;
+}
+
+// V values of a block, times inv = 1 / s, as hi and lo codes packed four to a word.
+template <int V>
+__device__ __forceinline__ void split_encode(const Bf16Run<V>& x, float inv, uint32_t (&hi)[(V + 3) / 4],
+                                             uint32_t (&lo)[(V + 3) / 4]) {
+  float q[V];
+  bool in_range = true;
+#pragma unroll
+  for (int i = 0; i < V; ++i) {
+    q[i] = x.get(i) * inv;
+    in_range = in_range && fabsf(q[i]) <= 448.0f;
+  }
+#pragma unroll
+  for (int w = 0; w < (V + 3) / 4; ++w) hi[w] = lo[w] = 0;
+  if (in_range) {
+    // Every |q| <= 448 is on the E4M3 range, where the hardware conversion
+    // (OCP E4M3, round to nearest even) is encode_e4m3; the residual
+    // |q - hi| <= 16 makes 16 (q - hi) lie within +-256.
+#pragma unroll
+    for (int w = 0; w < (V + 3) / 4; ++w) {
+      encode_pair_e4m3<false>(q[4 * w], q[4 * w + 1], hi[w], lo[w]);
+      if constexpr (V >= 4) encode_pair_e4m3<true>(q[4 * w + 2], q[4 * w + 3], hi[w], lo[w]);
+    }
+  } else {  // a non-finite or saturating value in this lane
+#pragma unroll
+    for (int i = 0; i < V; ++i) {
+      const uint32_t h = encode_e4m3(q[i]);
+      const uint32_t l = encode_e4m3((q[i] - e4m3_value(h)) * 16.0f);
+      hi[i >> 2] |= h << (8 * (i & 3));
+      lo[i >> 2] |= l << (8 * (i & 3));
+    }
+  }
+}
+
 // Wavefront = one row x (V / 2) consecutive 128-column blocks; lane l holds
 // V columns of block l / (128 / V).  V = 8 (16-byte loads, each block's amax
 // a reduction over one 16-lane DPP row) when the rows are 16-byte aligned,
-// V = 2 (one block per wavefront) otherwise.
-template <int V>
+// V = 2 (one block per wavefront) otherwise, into row-major planes or (V = 2
+// only) planes in operand order.
+template <int V, bool OPERAND>
 __device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int lane) {
   constexpr int kLanesPerBlock = kBlock / V;
   constexpr int kBlocksPerWave = 64 / kLanesPerBlock;
@@ -295,57 +341,66 @@ __device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int
     amax = fmaxf(amax, dpp_f32<0x141>(amax));  // row_half_mirror
     amax = fmaxf(amax, dpp_f32<0x140>(amax));  // row_mirror: the block's amax in all 16 lanes
   }
-  // s = 2^ceil(log2(amax / 448)): amax / s lies in (224, 448].
-  float s = 1.0f;
-  if (amax > 0.0f && isfinite(amax)) {
-    int e = ilogbf(amax / 448.0f);
-    if (e < -126) e = -126;
-    s = ldexpf(1.0f, e);
-    if (amax / s > 448.0f) s = ldexpf(1.0f, e + 1);
-  }
-  const float inv = 1.0f / s;
-  float q[V];
-  bool in_range = true;
-#pragma unroll
-  for (int i = 0; i < V; ++i) {
-    q[i] = x.get(i) * inv;
-    in_range = in_range && fabsf(q[i]) <= 448.0f;
-  }
-  uint32_t hi[(V + 3) / 4] = {}, lo[(V + 3) / 4] = {};
-  if (in_range) {
-    // Every |q| <= 448 is on the E4M3 range, where the hardware conversion
-    // (OCP E4M3, round to nearest even) is encode_e4m3; the residual
-    // |q - hi| <= 16 makes 16 (q - hi) lie within +-256.
-#pragma unroll
-    for (int w = 0; w < (V + 3) / 4; ++w) {
-      encode_pair_e4m3<false>(q[4 * w], q[4 * w + 1], hi[w], lo[w]);
-      if constexpr (V >= 4) encode_pair_e4m3<true>(q[4 * w + 2], q[4 * w + 3], hi[w], lo[w]);
-    }
-  } else {  // a non-finite or saturating value in this lane
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      const uint32_t h = encode_e4m3(q[i]);
-      const uint32_t l = encode_e4m3((q[i] - e4m3_value(h)) * 16.0f);
-      hi[i >> 2] |= h << (8 * (i & 3));
-      lo[i >> 2] |= l << (8 * (i & 3));
-    }
-  }
+  const float s = split_scale(amax);
+  uint32_t hi[(V + 3) / 4], lo[(V + 3) / 4];
+  split_encode<V>(x, 1.0f / s, hi, lo);
   if (!valid) return;
-  const int64_t off = row * a.cols + col;
   if constexpr (V == 8) {
+    static_assert(!OPERAND, "split_operand_kernel");
+    const int64_t off = row * a.cols + col;
     *reinterpret_cast<uint2*>(a.hi + off) = make_uint2(hi[0], hi[1]);
     *reinterpret_cast<uint2*>(a.lo + off) = make_uint2(lo[0], lo[1]);
   } else {
     static_assert(V == 2, "narrow split handles two columns per lane");
+    const int64_t off = OPERAND ? operand_order_offset(row, col, a.rows, a.cols) : row * a.cols + col;
     *reinterpret_cast<uint16_t*>(a.hi + off) = static_cast<uint16_t>(hi[0]);
     *reinterpret_cast<uint16_t*>(a.lo + off) = static_cast<uint16_t>(lo[0]);
   }
   if (lane % kLanesPerBlock == 0) a.scale[row * blocks_per_row + blk] = s;
 }
 
-template <int V>
+// The split into planes in operand order, 16-byte aligned rows: wavefront = 8
+// rows x one 128-column block, lane l the 16 columns from 16 (l % 8) of row l
+// / 8, which are one 16-byte piece of the operand, so that the 8 lanes of a
+// piece write 128 consecutive bytes (one row per wavefront, as above, writes
+// 8 bytes here and there, which cost the 300-row linear more than its kernel
+// gained).
+__global__ __launch_bounds__(256) void split_operand_kernel(SplitArgs a) {
+  const int lane = threadIdx.x & 63, piece = lane & 7;
+  const int64_t unit = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
+  const int64_t blocks_per_row = a.cols / kBlock;
+  if (unit >= (a.rows + 7) / 8 * blocks_per_row) return;
+  const int64_t blk = unit % blocks_per_row;
+  const int64_t row = unit / blocks_per_row * 8 + (lane >> 3);
+  const bool valid = row < a.rows;
+  Bf16Run<8> x[2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) {
+    x[j].clear();
+    if (valid) x[j].load(a.x + row * a.x_row_stride + blk * kBlock + 16 * piece + 8 * j);
+  }
+  float amax = 0.0f;
+#pragma unroll
+  for (int j = 0; j < 2; ++j)
+#pragma unroll
+    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[j].get(i)));
+  amax = fmaxf(amax, dpp_f32<0xB1>(amax));
+  amax = fmaxf(amax, dpp_f32<0x4E>(amax));
+  amax = fmaxf(amax, dpp_f32<0x141>(amax));  // the row's amax in its 8 lanes
+  const float s = split_scale(amax);
+  uint32_t hi[2][2], lo[2][2];
+#pragma unroll
+  for (int j = 0; j < 2; ++j) split_encode<8>(x[j], 1.0f / s, hi[j], lo[j]);
+  if (!valid) return;
+  const int64_t off = operand_order_offset(row, blk * kBlock + 16 * piece, a.rows, a.cols);
+  *reinterpret_cast<u32x4*>(a.hi + off) = (u32x4){hi[0][0], hi[0][1], hi[1][0], hi[1][1]};
+  *reinterpret_cast<u32x4*>(a.lo + off) = (u32x4){lo[0][0], lo[0][1], lo[1][0], lo[1][1]};
+  if (piece == 0) a.scale[row * blocks_per_row + blk] = s;
+}
+
+template <int V, bool OPERAND>
 __global__ __launch_bounds__(256) void split_activations_kernel(SplitArgs a) {
-  split_unit<V>(a, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
+  split_unit<V, OPERAND>(a, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
 }
 
 // The whole route plan of up to kPlanOneLaunchRoutes routes in one workgroup
@@ -438,7 +493,7 @@ __global__ __launch_bounds__(1024) void route_plan_one_kernel(RoutePlanArgs a, i
   __shared__ unsigned tile_cum[kPlanMaxExperts];
   __shared__ unsigned invalid_total;
   if (blockIdx.x > 0) {
-    split_unit<V>(s, static_cast<int64_t>(blockIdx.x - 1) * kPlanWaves + (threadIdx.x >> 6), threadIdx.x & 63);
+    split_unit<V, false>(s, static_cast<int64_t>(blockIdx.x - 1) * kPlanWaves + (threadIdx.x >> 6), threadIdx.x & 63);
     return;
   }
   static_assert(kPlanOneLaunchRoutes <= 2 * 64 * kPlanWaves, "two batches per wavefront at most");
@@ -1636,7 +1691,7 @@ hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hip
   if (a.routes <= kPlanOneLaunchRoutes) {
     SplitArgs s{};
     if (split != nullptr) s = *split;
-    if (s.cols % kBlock != 0) return hipErrorInvalidValue;
+    if (s.cols % kBlock != 0 || s.operand_order) return hipErrorInvalidValue;
     int id_bits = 0;
     while ((1 << id_bits) < a.experts) ++id_bits;
     const int64_t split_blocks = s.rows > 0 ? (split_units(s) + kPlanWaves - 1) / kPlanWaves : 0;
@@ -1659,9 +1714,13 @@ hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hip
 hipError_t launch_split_activations(const SplitArgs& a, hipStream_t st) {
   if (a.rows == 0) return hipSuccess;
   if (a.cols % kBlock != 0) return hipErrorInvalidValue;
-  const dim3 grid(static_cast<unsigned>((split_units(a) + 3) / 4));
-  if (split_wide(a)) hipLaunchKernelGGL(split_activations_kernel<8>, grid, dim3(256), 0, st, a);
-  else hipLaunchKernelGGL(split_activations_kernel<2>, grid, dim3(256), 0, st, a);
+  const bool wide = split_wide(a);
+  const int64_t units = wide && a.operand_order ? (a.rows + 7) / 8 * (a.cols / kBlock) : split_units(a);
+  const dim3 grid(static_cast<unsigned>((units + 3) / 4));
+  if (wide && a.operand_order) hipLaunchKernelGGL(split_operand_kernel, grid, dim3(256), 0, st, a);
+  else if (wide) hipLaunchKernelGGL((split_activations_kernel<8, false>), grid, dim3(256), 0, st, a);
+  else if (a.operand_order) hipLaunchKernelGGL((split_activations_kernel<2, true>), grid, dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((split_activations_kernel<2, false>), grid, dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
