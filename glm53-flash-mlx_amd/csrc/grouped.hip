@@ -265,29 +265,47 @@ __device__ __forceinline__ void store_bf16_run(uint16_t* p, const float* v) {
   }
 }
 
-// A block's scale s = 2^ceil(log2(amax / 448)): amax / s lies in (224, 448].
-__device__ __forceinline__ float split_scale(float amax) {
-  float s = 1.0f;
-  if (amax > 0.0f && isfinite(amax)) {
-    int e = ilogbf(amax / 448.0f);
-    if (e < -126) e = -126;
-    s = ldexpf(1.0f, e);
-    if (amax / s > 448.0f) s = ldexpf(1.0f, e + 1);
+// The largest |x| of a lane's values, NaNs left out; has_nan: there are some.
+// On the BF16 bits, two values per instruction.
+template <int V>
+__device__ __forceinline__ float lane_amax(const Bf16Run<V>& x, bool& has_nan) {
+  uint32_t m = 0;
+#pragma unroll
+  for (int i = 0; i < (V + 1) / 2; ++i) m = max_u16x2(m, x.w[i] & 0x7FFF7FFFu);
+  const uint32_t u = max(m & 0xFFFFu, m >> 16);
+  has_nan = u > 0x7F80u;
+  float amax = __uint_as_float(u << 16);
+  if (has_nan) {
+    amax = 0.0f;
+#pragma unroll
+    for (int i = 0; i < V; ++i) amax = fmaxf(amax, fabsf(x.get(i)));
   }
-  return s;
+  return amax;
 }
 
-// V values of a block, times inv = 1 / s, as hi and lo codes packed four to a word.
+// A block's scale s = 2^ceil(log2(amax / 448)), so that amax / s lies in (224,
+// 448], and 1 / s; both 1 for an all-zero or non-finite block.  448 = 1.75
+// 2^8: the exponent is amax's less 8, plus one where its significand is over
+// 1.75, and not below -126.
+struct SplitScale {
+  float s, inv;
+};
+__device__ __forceinline__ SplitScale split_scale(float amax) {
+  const uint32_t u = __float_as_uint(amax);
+  int code = static_cast<int>(u >> 23) + ((u & 0x7FFFFFu) > 0x600000u ? 1 : 0) - 8;
+  code = max(code, 1);
+  if (u == 0u || u >= 0x7F800000u) code = 127;
+  return {__uint_as_float(static_cast<uint32_t>(code) << 23), __uint_as_float(static_cast<uint32_t>(254 - code) << 23)};
+}
+
+// V values of a block, times inv = 1 / s, as hi and lo codes packed four to a
+// word; in_range: all of them finite, in a block of finite amax.
 template <int V>
-__device__ __forceinline__ void split_encode(const Bf16Run<V>& x, float inv, uint32_t (&hi)[(V + 3) / 4],
-                                             uint32_t (&lo)[(V + 3) / 4]) {
+__device__ __forceinline__ void split_encode(const Bf16Run<V>& x, float inv, bool in_range,
+                                             uint32_t (&hi)[(V + 3) / 4], uint32_t (&lo)[(V + 3) / 4]) {
   float q[V];
-  bool in_range = true;
 #pragma unroll
-  for (int i = 0; i < V; ++i) {
-    q[i] = x.get(i) * inv;
-    in_range = in_range && fabsf(q[i]) <= 448.0f;
-  }
+  for (int i = 0; i < V; ++i) q[i] = x.get(i) * inv;
 #pragma unroll
   for (int w = 0; w < (V + 3) / 4; ++w) hi[w] = lo[w] = 0;
   if (in_range) {
@@ -299,7 +317,7 @@ __device__ __forceinline__ void split_encode(const Bf16Run<V>& x, float inv, uin
       encode_pair_e4m3<false>(q[4 * w], q[4 * w + 1], hi[w], lo[w]);
       if constexpr (V >= 4) encode_pair_e4m3<true>(q[4 * w + 2], q[4 * w + 3], hi[w], lo[w]);
     }
-  } else {  // a non-finite or saturating value in this lane
+  } else {  // non-finite values in the lane or its block
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       const uint32_t h = encode_e4m3(q[i]);
@@ -329,9 +347,8 @@ __device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int
   Bf16Run<V> x;
   x.clear();
   if (valid) x.load(a.x + row * a.x_row_stride + col);
-  float amax = 0.0f;
-#pragma unroll
-  for (int i = 0; i < V; ++i) amax = fmaxf(amax, fabsf(x.get(i)));
+  bool has_nan;
+  float amax = lane_amax<V>(x, has_nan);
   if constexpr (kLanesPerBlock == 64) {
     amax = wave_max(amax);
   } else {
@@ -341,9 +358,9 @@ __device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int
     amax = fmaxf(amax, dpp_f32<0x141>(amax));  // row_half_mirror
     amax = fmaxf(amax, dpp_f32<0x140>(amax));  // row_mirror: the block's amax in all 16 lanes
   }
-  const float s = split_scale(amax);
+  const SplitScale s = split_scale(amax);
   uint32_t hi[(V + 3) / 4], lo[(V + 3) / 4];
-  split_encode<V>(x, 1.0f / s, hi, lo);
+  split_encode<V>(x, s.inv, isfinite(amax) && !has_nan, hi, lo);
   if (!valid) return;
   if constexpr (V == 8) {
     static_assert(!OPERAND, "split_operand_kernel");
@@ -356,7 +373,7 @@ __device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int
     *reinterpret_cast<uint16_t*>(a.hi + off) = static_cast<uint16_t>(hi[0]);
     *reinterpret_cast<uint16_t*>(a.lo + off) = static_cast<uint16_t>(lo[0]);
   }
-  if (lane % kLanesPerBlock == 0) a.scale[row * blocks_per_row + blk] = s;
+  if (lane % kLanesPerBlock == 0) a.scale[row * blocks_per_row + blk] = s.s;
 }
 
 // The split into planes in operand order, 16-byte aligned rows: wavefront = 8
@@ -379,23 +396,21 @@ __global__ __launch_bounds__(256) void split_operand_kernel(SplitArgs a) {
     x[j].clear();
     if (valid) x[j].load(a.x + row * a.x_row_stride + blk * kBlock + 16 * piece + 8 * j);
   }
-  float amax = 0.0f;
-#pragma unroll
-  for (int j = 0; j < 2; ++j)
-#pragma unroll
-    for (int i = 0; i < 8; ++i) amax = fmaxf(amax, fabsf(x[j].get(i)));
+  bool has_nan[2];
+  float amax = lane_amax<8>(x[0], has_nan[0]);
+  amax = fmaxf(amax, lane_amax<8>(x[1], has_nan[1]));
   amax = fmaxf(amax, dpp_f32<0xB1>(amax));
   amax = fmaxf(amax, dpp_f32<0x4E>(amax));
   amax = fmaxf(amax, dpp_f32<0x141>(amax));  // the row's amax in its 8 lanes
-  const float s = split_scale(amax);
+  const SplitScale s = split_scale(amax);
   uint32_t hi[2][2], lo[2][2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) split_encode<8>(x[j], 1.0f / s, hi[j], lo[j]);
+  for (int j = 0; j < 2; ++j) split_encode<8>(x[j], s.inv, isfinite(amax) && !has_nan[j], hi[j], lo[j]);
   if (!valid) return;
   const int64_t off = operand_order_offset(row, blk * kBlock + 16 * piece, a.rows, a.cols);
   *reinterpret_cast<u32x4*>(a.hi + off) = (u32x4){hi[0][0], hi[0][1], hi[1][0], hi[1][1]};
   *reinterpret_cast<u32x4*>(a.lo + off) = (u32x4){lo[0][0], lo[0][1], lo[1][0], lo[1][1]};
-  if (piece == 0) a.scale[row * blocks_per_row + blk] = s;
+  if (piece == 0) a.scale[row * blocks_per_row + blk] = s.s;
 }
 
 template <int V, bool OPERAND>
