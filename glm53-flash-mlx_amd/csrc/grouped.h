@@ -98,6 +98,7 @@ struct GroupedGemmArgs {
   const int32_t* fixup_up;    // SwiGLU mode: the up weights' flag when kept apart (or null)
   int tile_rows;                 // routes per descriptor: kGemmMinTileRows, kGemmTileRows (also 0) or kGemmWideRows
   int64_t n_tiles, descriptors;  // set by the launcher
+  int64_t deal;                  // likewise (launch_grouped_linear): descriptors per XCD and turn
   // device count of the routed descriptors in use (the route plan's
   // status[1]), or null: all `descriptors`.  Work items are dealt over
   // the descriptors in use only, so unused capacity costs no XCD share.

@@ -1132,13 +1132,18 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedGemmArgs a) {
 // bytes once more.
 __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
-  const int64_t items = a.n_tiles * a.descriptors;
-  const int64_t per_xcd = (items + 7) / 8;
-  const int64_t w = static_cast<int64_t>(blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-  if (w >= items) return;
-  int64_t ntile, d;
+  // A caller's descriptors end in unused ones (a tile plan over 288 experts
+  // and 4,096 routes holds 416, ~300 of them used) whose number only the
+  // device knows: workgroup i runs on XCD i % 8, and descriptors go to the
+  // XCDs in turn, a.deal at a time (one expert's neighbours share an L2),
+  // each with all its column tiles.  In contiguous runs the last XCDs held
+  // the unused ones: the chain above 1,569 us, 1,355 dealt in turn (1, 2 or 4 at
+  // a time alike).
+  const int64_t j = blockIdx.x / 8, turn = j / (a.deal * a.n_tiles), in_turn = j % (a.deal * a.n_tiles);
+  int64_t ntile = in_turn % a.n_tiles, d = (8 * turn + blockIdx.x % 8) * a.deal + in_turn / a.n_tiles;
+  if (d >= a.descriptors) return;
   bool fix;
-  const ItemSource src = item_source(a, a.descriptors, w, true, ntile, d, fix);
+  const ItemSource src = item_source(a, a.descriptors, d * a.n_tiles + ntile, true, ntile, d, fix);
   int32_t expert, start, len;
   if (!item_routes<kGemmTileRows>(src, d, expert, start, len)) return;
   for (int32_t done = 0; done < len; done += kGemmMinTileRows) {
@@ -1808,7 +1813,9 @@ hipError_t launch_grouped_linear(const GroupedGemmArgs& a, int64_t descriptors, 
   GroupedGemmArgs g = a;
   g.n_tiles = (a.N + kTileRows - 1) / kTileRows;
   g.descriptors = descriptors;
-  const unsigned grid = static_cast<unsigned>(8 * ((g.n_tiles * descriptors + 7) / 8));
+  g.deal = descriptors >= 256 ? 4 : 1;  // a few turns at least
+  const int64_t turns = (descriptors + 8 * g.deal - 1) / (8 * g.deal);
+  const unsigned grid = static_cast<unsigned>(8 * turns * g.deal * g.n_tiles);
   const size_t lds = gemm_lds_bytes<1>(a.K);
   if (a.K % kBlock != 0 || a.K <= 0 || lds > 160 * 1024) return hipErrorInvalidValue;
   hipLaunchKernelGGL(grouped_linear_kernel, dim3(grid), dim3(256), lds, st, g);
