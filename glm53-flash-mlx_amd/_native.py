@@ -94,6 +94,7 @@ _SIGNATURES = {
     "glm53_bank_destroy": (None, [P]),
     "glm53_relayout_weights": (ctypes.c_int, [P, P, I64, I64, I64, I32, I32, P]),
     "glm53_fp8_linear_workspace_bytes": (SZ, [I64, I64, I64]),
+    "glm53_fp8_linear_workspace_needed": (SZ, [P, I64, I64, I64]),
     "glm53_fp8_linear": (ctypes.c_int, [P, I64, I64, P, I64, P, P, P, P, SZ, P]),
     "glm53_mlp_workspace_bytes": (SZ, [I64, I64, I64]),
     "glm53_mlp": (ctypes.c_int, [P, F32, P, I64, P, P, SZ, P]),

@@ -94,12 +94,22 @@ hipError_t split(const void* x, int64_t rows, int64_t cols, const SplitBuf& b, h
   return launch_split_activations(split_args(x, rows, cols, b), st);
 }
 
+// Whether the shape splits these activations itself.
+bool takes_raw(const void* x, int64_t rows, int64_t K, DenseTile tile, bool swiglu) {
+  return dense_splits_x(tile, K, swiglu) && aligned(x, 16) && rows * K < (int64_t{1} << 31);
+}
+
 // One dense problem, plain or SwiGLU, in the shape that dense_tile names: x
 // bf16 [d.rows, d.K] is split into `space` (d's planes) and multiplied.
 // `flags`: device int32 [1] (SwiGLU: [2]) for the weights that come without a
 // code flag where the shape does not look for the codes itself.
 int dense(DenseArgs d, const void* x, const SplitBuf& space, bool swiglu, int32_t* flags, hipStream_t st) {
   const DenseTile tile = dense_tile(d.rows, d.K, d.N, swiglu);
+  if (takes_raw(x, d.rows, d.K, tile, swiglu)) {
+    d.x = static_cast<const uint16_t*>(x);
+    HIP_TRY(launch_dense_linear(d, tile, swiglu, st), "dense linear launch");
+    return GLM53_OK;
+  }
   SplitArgs sp = split_args(x, d.rows, d.K, space);
   sp.operand_order = dense_ksplit(tile, swiglu);
   HIP_TRY(launch_split_activations(sp, st), "split launch");
@@ -402,6 +412,11 @@ void glm53_bank_destroy(glm53_bank* bank) {
   delete b;
 }
 
+size_t glm53_fp8_linear_workspace_needed(const void* x, int64_t M, int64_t N, int64_t K) {
+  const size_t need = glm53_fp8_linear_workspace_bytes(M, N, K);
+  return need > 0 && takes_raw(x, M, K, dense_tile(M, K, N, false), false) ? 0 : need;
+}
+
 int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight, int64_t N, const float* scale_inv,
                      const int32_t* code_flags, void* y, void* workspace, size_t workspace_bytes, void* stream) {
   CHECK_ARG(M >= 0 && K > 0 && N > 0, "invalid shape M=%lld K=%lld N=%lld", (long long)M, (long long)K, (long long)N);
@@ -435,8 +450,9 @@ int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight,
     return GLM53_OK;
   }
   const size_t need = glm53_fp8_linear_workspace_bytes(M, N, K);
-  if (need > 0 && aligned(weight, 16) && workspace != nullptr && workspace_bytes >= need) {
-    SplitBuf b = carve_split(workspace, M, K);
+  const bool raw = need > 0 && glm53_fp8_linear_workspace_needed(x, M, N, K) == 0;
+  if (need > 0 && aligned(weight, 16) && (raw || (workspace != nullptr && workspace_bytes >= need))) {
+    SplitBuf b = carve_split(workspace, M, K);  // raw: not used
     DenseArgs d{};
     d.weight = weight;
     d.scale = scale_inv;

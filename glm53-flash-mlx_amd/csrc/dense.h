@@ -7,7 +7,8 @@
 namespace glm53 {
 
 struct DenseArgs {
-  const uint8_t* a_hi;     // [rows, K] split activations; for launch_dense_linear in MFMA operand order
+  const uint16_t* x;       // [rows, K] bf16 activations, 16-byte aligned, or null: a_hi, a_lo, a_scale hold their split
+  const uint8_t* a_hi;     // [rows, K]; for launch_dense_linear in MFMA operand order
   const uint8_t* a_lo;
   const float* a_scale;    // [rows, K / 128]
   const uint8_t* weight;   // [N, K], 16-byte aligned
@@ -34,6 +35,9 @@ struct DenseTile {
 DenseTile dense_tile(int64_t rows, int64_t K, int64_t N, bool swiglu);
 // Whether launch_dense_linear runs the tile.
 inline bool dense_ksplit(DenseTile t, bool swiglu) { return t.rows <= 32 && (swiglu ? 2 : 1) * t.cols <= 64; }
+// Whether launch_dense_linear takes the tile's bf16 activations as they are
+// (DenseArgs.x) and splits them itself.
+bool dense_splits_x(DenseTile t, int64_t K, bool swiglu);
 hipError_t launch_dense_linear(const DenseArgs& a, DenseTile tile, bool swiglu, hipStream_t st);
 
 }  // namespace glm53

@@ -5,6 +5,7 @@
 #include "dense.h"
 #include "grouped.h"
 #include "mfma_fp8.h"
+#include "split_fp8.h"
 
 namespace glm53 {
 
@@ -29,9 +30,16 @@ template <int P, int C>
 constexpr int load_depth() {
   return P * C <= 2 ? 4 : 2;
 }
-template <int P, int C>
+// Operand tiles a wavefront passes through its own LDS buffer: its weight
+// tiles, and (RAW) the hi and lo tile it makes of its activations
+template <int C, bool RAW>
+constexpr int turn_tiles() {
+  return C + (RAW ? 2 : 0);
+}
+
+template <int P, int C, bool RAW>
 size_t dense_lds_bytes(int64_t K) {
-  return static_cast<size_t>(kDenseWaves) * (fold_steps<P, C>() * P * C * 1024 + C * kOperand) +
+  return static_cast<size_t>(kDenseWaves) * (fold_steps<P, C>() * P * C * 1024 + turn_tiles<C, RAW>() * kOperand) +
          2 * sizeof(float) * static_cast<size_t>(K / kBlock);
 }
 
@@ -52,7 +60,12 @@ size_t dense_lds_bytes(int64_t K) {
 // to LDS, and wavefront t < P C adds tile t's results in block order, so
 // every output goes through the operations of the grouped GEMM and has its
 // bits.  Returns codes_480 of the weight bytes (DETECT).
-template <int P, int C, bool SWIGLU, bool FIX, bool DETECT>
+//
+// RAW (P = 1): the activations come as bf16 (a.x) and the wavefront splits
+// each of its blocks itself on the way to LDS -- lanes 16 j .. 16 j + 15 hold
+// 8 columns each of rows j, 4 + j, 8 + j and 12 + j -- instead of a launch of
+// its own that writes planes and scales first.
+template <int P, int C, bool SWIGLU, bool RAW, bool FIX, bool DETECT>
 __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_t row0, int64_t col0, uint8_t* lds) {
   constexpr int D = FIX ? 1 : load_depth<P, C>(), F = FIX ? 1 : fold_steps<P, C>();
   constexpr int H = SWIGLU ? C / 2 : C;  // tiles of one matrix
@@ -64,13 +77,21 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   const int steps = (KB + kDenseWaves - 1) / kDenseWaves;
   constexpr int kFold = kDenseWaves * fold_steps<P, C>() * P * C * 1024;
   f32x4* lds_c = reinterpret_cast<f32x4*>(lds);                                          // [8 F][P C][64]
-  uint8_t* turn = lds + kFold + wave * C * kOperand;                    // this wavefront's
-  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * C * kOperand);  // [2][KB]
+  constexpr int kTurn = turn_tiles<C, RAW>() * kOperand;
+  uint8_t* turn = lds + kFold + wave * kTurn;                                            // this wavefront's
+  float* lds_sw = reinterpret_cast<float*>(lds + kFold + kDenseWaves * kTurn);           // [2][KB]
   const OperandSlots slots = operand_slots(lane);
 
   // rows past the last repeat it, columns past the matrix its last row: valid
   // bytes whose results are never stored (offsets from wave-uniform bases;
   // the launcher keeps them below 2^32)
+  static_assert(!RAW || P == 1, "a raw item holds one pair");
+  uint32_t xoff[4];  // RAW: byte offsets of the lane's columns of row 4 i + lane / 16
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    const int64_t m = row0 + 4 * i + kq;
+    xoff[i] = static_cast<uint32_t>(2 * ((m < a.rows ? m : a.rows - 1) * K + 8 * r));
+  }
   uint32_t aoff[P], srow[P], wrow[C][2];
   int64_t apair[P];  // the pair's bytes in the planes
   int arows[P];      // and rows
@@ -102,9 +123,14 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
     kb = kb < KB ? kb : KB - 1;  // past the end: loaded, never folded
     const int64_t ko = static_cast<int64_t>(kb) * kBlock;  // wave-uniform
     const uint8_t *w = a.weight + ko, *up = SWIGLU ? a.weight_up + ko : w;
+    if constexpr (RAW) {
+      const uint8_t* x = reinterpret_cast<const uint8_t*>(a.x + ko);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) (i < 2 ? v.h : v.l)[0][i & 1] = *reinterpret_cast<const u32x4*>(x + xoff[i]);
+    }
     const float* se = a.a_scale + kb;
 #pragma unroll
-    for (int p = 0; p < P; ++p) {
+    for (int p = 0; p < (RAW ? 0 : P); ++p) {
       const int64_t block = apair[p] + ko * arows[p];
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
@@ -141,12 +167,64 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
   uint32_t found = 0;
   float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
   auto multiply = [&](int slot, const Step& v) {  // the step's results into slot (block slot of the fold)
-    i32x8 b[C], bc[1];
+    i32x8 b[C], bc[1], ah[P], al[P];
+    int se[P];
 #pragma unroll
     for (int c = 0; c < C; ++c) put(c, v.b[c]);
+    if constexpr (RAW) {
+      // byte (row, k) of a tile at 128 row + 16 (k / 16 ^ row % 8 ^ row / 8) + k % 16 (operand_slots)
+      // The four rows side by side (one branch for all of them): each is a
+      // chain of ~60 dependent instructions.
+      Bf16Run<8> x[4];
+      SplitScale sc[4];
+      uint32_t hi[4][2], lo[4][2];
+      bool plain = true;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) x[i].w[j] = (i < 2 ? v.h : v.l)[0][i & 1][j];
+        // a lane with a NaN counts as infinite: no plain block
+        sc[i] = split_scale(row16_amax(__uint_as_float(min(lane_amax_bits<8>(x[i]), 0x7F80u) << 16)));
+        plain = plain && sc[i].plain;
+      }
+      if (__builtin_expect(__builtin_amdgcn_ballot_w64(!plain) == 0, 1)) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) split_encode_plain<8>(x[i], sc[i], hi[i], lo[i]);
+      } else {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          bool has_nan;
+          sc[i] = split_scale(row16_amax(lane_amax<8>(x[i], has_nan)));
+          split_encode_any<8>(x[i], sc[i], hi[i], lo[i]);
+        }
+      }
+      uint32_t codes = 0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        codes |= scale_e8m0(sc[i].s) << (8 * i);
+        const int row = 4 * i + kq;
+        uint8_t* at = turn + C * kOperand + 128 * row + 16 * ((r >> 1) ^ (row & 7) ^ (row >> 3)) + 8 * (r & 1);
+        *reinterpret_cast<uint2*>(at) = make_uint2(hi[i][0], hi[i][1]);
+        *reinterpret_cast<uint2*>(at + kOperand) = make_uint2(lo[i][0], lo[i][1]);
+      }
+      // row r's scale code: byte r / 4 of the codes of lanes 16 (r % 4) ..
+      codes = static_cast<uint32_t>(__builtin_amdgcn_ds_bpermute(4 * 16 * (r & 3), static_cast<int>(codes)));
+      se[0] = static_cast<int>((codes >> (8 * (r >> 2))) & 0xFFu);
+    } else {
+#pragma unroll
+      for (int p = 0; p < P; ++p) {
+        ah[p] = vec(v.h[p]);
+        al[p] = vec(v.l[p]);
+        se[p] = static_cast<int>(scale_e8m0(v.s[p]));
+      }
+    }
     turned();
 #pragma unroll
     for (int c = 0; c < C; ++c) b[c] = lds_operand(turn + c * kOperand, slots);
+    if constexpr (RAW) {
+      ah[0] = lds_operand(turn + C * kOperand, slots);
+      al[0] = lds_operand(turn + (C + 1) * kOperand, slots);
+    }
     turned();
     if constexpr (DETECT) {
 #pragma unroll
@@ -162,9 +240,8 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
         weight_operand<FIX>(b[c], bc[0]);
 #pragma unroll
         for (int p = 0; p < P; ++p) {
-          const int e = static_cast<int>(scale_e8m0(v.s[p]));
-          const f32x4 x = pair_pass<FIX, 0, 127>(vec(v.h[p]), b[c], bc[0], kZero, e);
-          lds_c[(slot * P * C + p * C + c) * 64 + lane] = pair_pass<FIX, 0, 123>(vec(v.l[p]), b[c], bc[0], x, e);
+          const f32x4 x = pair_pass<FIX, 0, 127>(ah[p], b[c], bc[0], kZero, se[p]);
+          lds_c[(slot * P * C + p * C + c) * 64 + lane] = pair_pass<FIX, 0, 123>(al[p], b[c], bc[0], x, se[p]);
         }
       }
     } else {
@@ -173,13 +250,13 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
       for (int p = 0; p < P; ++p)
 #pragma unroll
         for (int c = 0; c < C; ++c)
-          x[p][c] = pair_pass<FIX, 0, 127>(vec(v.h[p]), b[c], b[c], kZero, static_cast<int>(scale_e8m0(v.s[p])));
+          x[p][c] = pair_pass<FIX, 0, 127>(ah[p], b[c], b[c], kZero, se[p]);
 #pragma unroll
       for (int p = 0; p < P; ++p)
 #pragma unroll
         for (int c = 0; c < C; ++c)
           lds_c[(slot * P * C + p * C + c) * 64 + lane] =
-              pair_pass<FIX, 0, 123>(vec(v.l[p]), b[c], b[c], x[p][c], static_cast<int>(scale_e8m0(v.s[p])));
+              pair_pass<FIX, 0, 123>(al[p], b[c], b[c], x[p][c], se[p]);
     }
   };
   // adds the results of the K blocks of steps s0 .. s0 + F - 1, in block order
@@ -270,7 +347,7 @@ __device__ __forceinline__ uint32_t dense_ksplit_item(const DenseArgs& a, int64_
 
 // Workgroup i runs on XCD i % 8; each XCD takes a contiguous run of items,
 // row groups fastest, so the items that share weight columns meet in one L2.
-template <int P, int C, bool SWIGLU>
+template <int P, int C, bool SWIGLU, bool RAW>
 __global__ __launch_bounds__(64 * kDenseWaves) void dense_ksplit_kernel(DenseArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
   constexpr int kCols = SWIGLU ? 8 * C : 16 * C;
@@ -283,21 +360,29 @@ __global__ __launch_bounds__(64 * kDenseWaves) void dense_ksplit_kernel(DenseArg
   const bool look = a.flag == nullptr || (SWIGLU && a.flag_up == nullptr);
   bool fix = (a.flag != nullptr && *a.flag != 0) || (SWIGLU && a.flag_up != nullptr && *a.flag_up != 0);
   if (!fix) {
-    const uint32_t found = dense_ksplit_item<P, C, SWIGLU, false, true>(a, row0, col0, lds_dyn);
+    const uint32_t found = dense_ksplit_item<P, C, SWIGLU, RAW, false, true>(a, row0, col0, lds_dyn);
     if (look) fix = workgroup_any((found & 0x80808080u) != 0, lds_dyn);
   }
-  if (fix) dense_ksplit_item<P, C, SWIGLU, true, false>(a, row0, col0, lds_dyn);
+  if (fix) dense_ksplit_item<P, C, SWIGLU, RAW, true, false>(a, row0, col0, lds_dyn);
+}
+
+template <int P, int C, bool SWIGLU, bool RAW>
+hipError_t launch_ksplit_t(const DenseArgs& a, hipStream_t st) {
+  constexpr int kCols = SWIGLU ? 8 * C : 16 * C;
+  const int64_t items = ((a.rows + 16 * P - 1) / (16 * P)) * ((a.N + kCols - 1) / kCols);
+  const size_t lds = dense_lds_bytes<P, C, RAW>(a.K);
+  if (a.K > kDenseMaxK || lds > 160 * 1024) return hipErrorInvalidValue;
+  hipLaunchKernelGGL((dense_ksplit_kernel<P, C, SWIGLU, RAW>), dim3(static_cast<unsigned>(8 * ((items + 7) / 8))),
+                     dim3(64 * kDenseWaves), lds, st, a);
+  return hipGetLastError();
 }
 
 template <int P, int C, bool SWIGLU>
 hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
-  constexpr int kCols = SWIGLU ? 8 * C : 16 * C;
-  const int64_t items = ((a.rows + 16 * P - 1) / (16 * P)) * ((a.N + kCols - 1) / kCols);
-  const size_t lds = dense_lds_bytes<P, C>(a.K);
-  if (a.K > kDenseMaxK || lds > 160 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL((dense_ksplit_kernel<P, C, SWIGLU>), dim3(static_cast<unsigned>(8 * ((items + 7) / 8))),
-                     dim3(64 * kDenseWaves), lds, st, a);
-  return hipGetLastError();
+  if constexpr (P == 1) {
+    if (a.x != nullptr) return launch_ksplit_t<P, C, SWIGLU, true>(a, st);
+  }
+  return a.x != nullptr ? hipErrorInvalidValue : launch_ksplit_t<P, C, SWIGLU, false>(a, st);
 }
 
 }  // namespace
@@ -338,7 +423,21 @@ DenseTile dense_tile(int64_t rows, int64_t K, int64_t N, bool swiglu) {
   return of(wide ? DenseTile{128, 512} : DenseTile{64, 128});
 }
 
+// One-pair tiles split their own blocks: the conversion (~55 instructions per
+// 8 columns, every workgroup for its 16 rows, the four rows of a lane side by
+// side: one after the other they took 13.3 us) makes the kernel 11.6 us at 16
+// x 4096 x 4096 where split and product take 3.7 + 7.0 and a launch between,
+// and saves that launch and the workspace: 11.9 us a call instead of 16.0.
+// The conversion grows with K where the split's launch does not, so long rows
+// keep the launch.
+bool dense_splits_x(DenseTile t, int64_t K, bool swiglu) {
+  return t.rows == 16 && dense_ksplit(t, swiglu) && K <= 8192;
+}
+
 hipError_t launch_dense_linear(const DenseArgs& a, DenseTile t, bool swiglu, hipStream_t st) {
+  if (a.x != nullptr && (!dense_splits_x(t, a.K, swiglu) || reinterpret_cast<uintptr_t>(a.x) % 16 != 0 ||
+                         a.rows * a.K >= (int64_t{1} << 31)))
+    return hipErrorInvalidValue;
   if (a.rows <= 0 || a.K <= 0 || a.K % kBlock != 0 || a.N <= 0 || a.N % 16 != 0) return hipErrorInvalidValue;
   if (a.N * a.K >= (int64_t{1} << 32) || a.rows * a.K >= (int64_t{1} << 32)) return hipErrorInvalidValue;
   const int cols = swiglu ? 2 * t.cols : t.cols;

@@ -28,6 +28,7 @@
 #include "common.h"
 #include "grouped.h"
 #include "mfma_fp8.h"
+#include "split_fp8.h"
 
 namespace glm53 {
 
@@ -190,66 +191,6 @@ __global__ __launch_bounds__(256) void route_scatter_kernel(RoutePlanArgs a) {
 
 // ------------------------------------------------ activation hi/lo split --
 
-// RNE to the E4M3 grid, saturating at +-448 (never the 0x7F/0xFF codes).
-__device__ __forceinline__ uint32_t encode_e4m3(float v) {
-  uint32_t sign = (__float_as_uint(v) >> 24) & 0x80u;
-  float a = fabsf(v);
-  if (!(a < 448.0f)) return sign | 0x7Eu;
-  if (a < 0.015625f) {  // below 2^-6: subnormal grid of 2^-9
-    return sign | static_cast<uint32_t>(rintf(a * 512.0f));
-  }
-  int e = ilogbf(a);
-  float m = rintf(ldexpf(a, 3 - e));  // in [8, 16]
-  if (m >= 16.0f) {
-    e += 1;
-    m = 8.0f;
-  }
-  if (e > 8 || (e == 8 && m > 14.0f)) return sign | 0x7Eu;
-  return sign | (static_cast<uint32_t>(e + 7) << 3) | (static_cast<uint32_t>(m) - 8u);
-}
-
-__device__ __forceinline__ float e4m3_value(uint32_t code) {
-  uint16_t h = static_cast<uint16_t>(((code & 0x7Fu) << 7) | ((code & 0x80u) << 8));
-  return static_cast<float>(__builtin_bit_cast(_Float16, h)) * 256.0f;
-}
-
-// Hardware E4M3 conversion of a pair (q0, q1), both |q| <= 448, into bytes
-// 0-1 (kUpper false) or 2-3 of hi_word, and of their residuals 16 (q - hi)
-// into the same bytes of lo_word; the other bytes are kept.
-template <bool kUpper>
-__device__ __forceinline__ void encode_pair_e4m3(float q0, float q1, uint32_t& hi_word, uint32_t& lo_word) {
-  const int h = __builtin_amdgcn_cvt_pk_fp8_f32(q0, q1, static_cast<int>(hi_word), kUpper);
-  hi_word = static_cast<uint32_t>(h);
-  const float r0 = (q0 - __builtin_amdgcn_cvt_f32_fp8(h, kUpper ? 2 : 0)) * 16.0f;
-  const float r1 = (q1 - __builtin_amdgcn_cvt_f32_fp8(h, kUpper ? 3 : 1)) * 16.0f;
-  lo_word = static_cast<uint32_t>(__builtin_amdgcn_cvt_pk_fp8_f32(r0, r1, static_cast<int>(lo_word), kUpper));
-}
-
-// V consecutive BF16 values as raw words: V = 8 is one 16-byte load (the
-// pointer 16-byte aligned), V = 1 or 2 are 2-byte loads.
-template <int V>
-struct Bf16Run {
-  uint32_t w[(V + 1) / 2];
-  __device__ __forceinline__ void load(const uint16_t* p) {
-    if constexpr (V == 8) {
-      const uint4 r = *reinterpret_cast<const uint4*>(p);
-      w[0] = r.x, w[1] = r.y, w[2] = r.z, w[3] = r.w;
-    } else {
-#pragma unroll
-      for (int i = 0; i < (V + 1) / 2; ++i) w[i] = 0u;
-#pragma unroll
-      for (int i = 0; i < V; ++i) w[i >> 1] |= static_cast<uint32_t>(p[i]) << (16 * (i & 1));
-    }
-  }
-  __device__ __forceinline__ void clear() {
-#pragma unroll
-    for (int i = 0; i < (V + 1) / 2; ++i) w[i] = 0u;
-  }
-  __device__ __forceinline__ float get(int i) const {
-    return __uint_as_float(i & 1 ? (w[i >> 1] & 0xffff0000u) : (w[i >> 1] << 16));
-  }
-};
-
 // Rounds V floats to BF16 and stores them (one 16-byte store for V = 8).
 template <int V>
 __device__ __forceinline__ void store_bf16_run(uint16_t* p, const float* v) {
@@ -262,69 +203,6 @@ __device__ __forceinline__ void store_bf16_run(uint16_t* p, const float* v) {
   } else {
 #pragma unroll
     for (int i = 0; i < V; ++i) p[i] = f32_to_bf16(v[i]);
-  }
-}
-
-// The largest |x| of a lane's values, NaNs left out; has_nan: there are some.
-// On the BF16 bits, two values per instruction.
-template <int V>
-__device__ __forceinline__ float lane_amax(const Bf16Run<V>& x, bool& has_nan) {
-  uint32_t m = 0;
-#pragma unroll
-  for (int i = 0; i < (V + 1) / 2; ++i) m = max_u16x2(m, x.w[i] & 0x7FFF7FFFu);
-  const uint32_t u = max(m & 0xFFFFu, m >> 16);
-  has_nan = u > 0x7F80u;
-  float amax = __uint_as_float(u << 16);
-  if (has_nan) {
-    amax = 0.0f;
-#pragma unroll
-    for (int i = 0; i < V; ++i) amax = fmaxf(amax, fabsf(x.get(i)));
-  }
-  return amax;
-}
-
-// A block's scale s = 2^ceil(log2(amax / 448)), so that amax / s lies in (224,
-// 448], and 1 / s; both 1 for an all-zero or non-finite block.  448 = 1.75
-// 2^8: the exponent is amax's less 8, plus one where its significand is over
-// 1.75, and not below -126.
-struct SplitScale {
-  float s, inv;
-};
-__device__ __forceinline__ SplitScale split_scale(float amax) {
-  const uint32_t u = __float_as_uint(amax);
-  int code = static_cast<int>(u >> 23) + ((u & 0x7FFFFFu) > 0x600000u ? 1 : 0) - 8;
-  code = max(code, 1);
-  if (u == 0u || u >= 0x7F800000u) code = 127;
-  return {__uint_as_float(static_cast<uint32_t>(code) << 23), __uint_as_float(static_cast<uint32_t>(254 - code) << 23)};
-}
-
-// V values of a block, times inv = 1 / s, as hi and lo codes packed four to a
-// word; in_range: all of them finite, in a block of finite amax.
-template <int V>
-__device__ __forceinline__ void split_encode(const Bf16Run<V>& x, float inv, bool in_range,
-                                             uint32_t (&hi)[(V + 3) / 4], uint32_t (&lo)[(V + 3) / 4]) {
-  float q[V];
-#pragma unroll
-  for (int i = 0; i < V; ++i) q[i] = x.get(i) * inv;
-#pragma unroll
-  for (int w = 0; w < (V + 3) / 4; ++w) hi[w] = lo[w] = 0;
-  if (in_range) {
-    // Every |q| <= 448 is on the E4M3 range, where the hardware conversion
-    // (OCP E4M3, round to nearest even) is encode_e4m3; the residual
-    // |q - hi| <= 16 makes 16 (q - hi) lie within +-256.
-#pragma unroll
-    for (int w = 0; w < (V + 3) / 4; ++w) {
-      encode_pair_e4m3<false>(q[4 * w], q[4 * w + 1], hi[w], lo[w]);
-      if constexpr (V >= 4) encode_pair_e4m3<true>(q[4 * w + 2], q[4 * w + 3], hi[w], lo[w]);
-    }
-  } else {  // non-finite values in the lane or its block
-#pragma unroll
-    for (int i = 0; i < V; ++i) {
-      const uint32_t h = encode_e4m3(q[i]);
-      const uint32_t l = encode_e4m3((q[i] - e4m3_value(h)) * 16.0f);
-      hi[i >> 2] |= h << (8 * (i & 3));
-      lo[i >> 2] |= l << (8 * (i & 3));
-    }
   }
 }
 
@@ -353,14 +231,11 @@ __device__ __forceinline__ void split_unit(const SplitArgs& a, int64_t unit, int
     amax = wave_max(amax);
   } else {
     static_assert(kLanesPerBlock == 16, "a block spans one DPP row or the whole wavefront");
-    amax = fmaxf(amax, dpp_f32<0xB1>(amax));   // quad_perm [1,0,3,2]
-    amax = fmaxf(amax, dpp_f32<0x4E>(amax));   // quad_perm [2,3,0,1]
-    amax = fmaxf(amax, dpp_f32<0x141>(amax));  // row_half_mirror
-    amax = fmaxf(amax, dpp_f32<0x140>(amax));  // row_mirror: the block's amax in all 16 lanes
+    amax = row16_amax(amax);
   }
   const SplitScale s = split_scale(amax);
   uint32_t hi[(V + 3) / 4], lo[(V + 3) / 4];
-  split_encode<V>(x, s.inv, isfinite(amax) && !has_nan, hi, lo);
+  split_encode<V>(x, s, has_nan, hi, lo);
   if (!valid) return;
   if constexpr (V == 8) {
     static_assert(!OPERAND, "split_operand_kernel");
@@ -405,7 +280,7 @@ __global__ __launch_bounds__(256) void split_operand_kernel(SplitArgs a) {
   const SplitScale s = split_scale(amax);
   uint32_t hi[2][2], lo[2][2];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) split_encode<8>(x[j], s.inv, isfinite(amax) && !has_nan[j], hi[j], lo[j]);
+  for (int j = 0; j < 2; ++j) split_encode<8>(x[j], s, has_nan[j], hi[j], lo[j]);
   if (!valid) return;
   const int64_t off = operand_order_offset(row, blk * kBlock + 16 * piece, a.rows, a.cols);
   *reinterpret_cast<u32x4*>(a.hi + off) = (u32x4){hi[0][0], hi[0][1], hi[1][0], hi[1][1]};

@@ -72,7 +72,9 @@ def native_block_fp8_linear(x, weight, scale_inv, code_flags):
     rows = flat.shape[0]
     y = torch.empty((rows, out_features), dtype=torch.bfloat16, device=x.device)
     lib = N.lib()
-    ws_bytes = lib.glm53_fp8_linear_workspace_bytes(rows, out_features, in_features) if rows > 1 else 0
+    ws_bytes = 0
+    if rows > 1:
+        ws_bytes = lib.glm53_fp8_linear_workspace_needed(flat.data_ptr(), rows, out_features, in_features)
     ws = N.workspace(ws_bytes, x.device)
     N.check(lib.glm53_fp8_linear(flat.data_ptr(), rows, in_features, weight.data_ptr(), out_features,
                                  scale_inv.data_ptr(), None if code_flags is None else code_flags.data_ptr(),

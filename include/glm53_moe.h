@@ -177,6 +177,9 @@ int glm53_e4m3_scan_codes(const uint8_t* codes, int64_t n, int32_t* flag, void* 
  * or scans the weight first (M > 1).
  * ---------------------------------------------------------------------- */
 size_t glm53_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
+/* The same for this x: 0 where the call splits the activations inside the
+ * product (few rows, x 16-byte aligned) and takes a NULL workspace. */
+size_t glm53_fp8_linear_workspace_needed(const void* x, int64_t M, int64_t N, int64_t K);
 int glm53_fp8_linear(const void* x, int64_t M, int64_t K, const uint8_t* weight, int64_t N,
                      const float* scale_inv, const int32_t* code_flags, void* y, void* workspace,
                      size_t workspace_bytes, void* stream);

@@ -115,6 +115,32 @@ def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
     assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
 
 
+@pytest.mark.parametrize("rows,n,k", [(3, 128, 128), (16, 272, 1152), (40, 2064, 8192), (250, 272, 640), (3, 64, 8320)])
+def test_few_rows_split_in_the_kernel_equals_the_split_launch(M, O, dev, rows, n, k):
+    """Rows that are 16-byte aligned are split inside the few-row product (K
+    up to 8192), others by a launch of their own: the same bytes, with zero
+    blocks, subnormal and huge blocks, NaN and infinities among them."""
+    import torch
+
+    rng = np.random.default_rng(rows + n + k)
+    codes = rng.integers(0, 0x7F, size=(n, k), dtype=np.int64).astype(np.uint8)
+    scale = (rng.uniform(size=(-(-n // 128), k // 128)) * 0.002).astype(np.float32)
+    w, s = torch.from_numpy(codes).to(dev), torch.from_numpy(scale).to(dev)
+    x = rng.normal(size=(rows, k)) * 2.0 ** rng.integers(-20, 20, size=(rows, 1))
+    bits = O.f32_to_bf16(x.astype(np.float32)).reshape(rows, k)
+    bits[0, :128] = 0
+    bits[1, :128] = rng.integers(0, 0x80, size=128)  # subnormal
+    bits[2, 5], bits[2, k - 3], bits[2, 40], bits[rows - 1, k - 1] = 0x7F80, 0xFFC1, 0x7F01, 0xFF80
+    aligned = from_bits(bits, dev)
+    shifted = torch.empty(rows * k + 1, dtype=torch.bfloat16, device=dev)[1:].view(rows, k)
+    shifted.copy_(aligned)
+    assert aligned.data_ptr() % 16 == 0 and shifted.data_ptr() % 16 == 2
+    needed = submodule("_native").lib().glm53_fp8_linear_workspace_needed
+    assert (needed(aligned.data_ptr(), rows, n, k) == 0) == (k <= 8192) and needed(shifted.data_ptr(), rows, n, k) > 0
+    got, want = (M.block_fp8_linear(v, w, s) for v in (aligned, shifted))
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
 @pytest.mark.parametrize("with_480", [False, True])
 @pytest.mark.parametrize("rows", [2, 33, 150, 300, 700, 1300, 6000, 12000])
 def test_mlp_in_one_call_equals_its_parts(M, dev, rows, with_480):

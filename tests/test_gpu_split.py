@@ -71,6 +71,13 @@ def test_split_every_bf16_value_in_range(dev, shift, offset):
     _check(_exhaustive_rows(shift), dev, offset=offset)
 
 
+@pytest.mark.parametrize("shift", [-96, -95, -94, -7, 60, 119])
+def test_split_every_bf16_value_at_the_scaled_conversions_ends(dev, shift):
+    """The scaled hardware conversions serve blocks of scale 2^-95 and up to
+    the largest finite block; 2^-96 takes the encoder in code."""
+    _check(_exhaustive_rows(shift), dev)
+
+
 @pytest.mark.parametrize("cols,offset,stride_pad", [(512, 0, 0), (384, 0, 8), (384, 1, 3), (128, 0, 0)])
 def test_split_random_block_magnitudes(dev, cols, offset, stride_pad):
     rng = np.random.default_rng(cols + offset)
