@@ -1334,7 +1334,7 @@ int glm53_routed_diagnostic_counters(const glm53_routed_diagnostic* d, uint64_t*
 // ---------------------------------------------------- prefill pieces ------
 
 size_t glm53_route_plan_workspace_bytes(int64_t routes, int64_t experts) {
-  const int64_t blocks = std::max<int64_t>(cdiv(routes, 256), 1);
+  const int64_t blocks = std::max<int64_t>(cdiv(routes, kPlanBlockRoutes), 1);
   return round_up(sizeof(unsigned) * blocks * experts) + round_up(sizeof(unsigned) * blocks);
 }
 
@@ -1352,7 +1352,7 @@ int route_plan_impl(const int32_t* expert_ids, const float* scores, int64_t rout
   a.top_k = static_cast<int>(top_k);
   a.experts = static_cast<int>(experts);
   a.tile_rows = static_cast<int>(tile_rows);
-  a.blocks = cdiv(routes, 256);
+  a.blocks = cdiv(routes, kPlanBlockRoutes);
   a.capacity = capacity;
   a.block_counts = static_cast<unsigned*>(workspace);
   a.block_invalid = reinterpret_cast<unsigned*>(static_cast<uint8_t*>(workspace) +

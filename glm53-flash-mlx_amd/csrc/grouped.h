@@ -8,6 +8,7 @@ namespace glm53 {
 
 constexpr int kPlanMaxExperts = 1024;
 constexpr int64_t kPlanOneLaunchRoutes = 2048;  // route plans up to here run as one workgroup
+constexpr int64_t kPlanBlockRoutes = 1024;  // larger ones count and rank blocks of this many
 constexpr int kGroupedTileRows = 32;   // routes per descriptor of the reference (grouped_fp8.py:20)
 constexpr int kGemmTileRows = 64;      // routes per descriptor of the MFMA grouped GEMM (many routes per expert)
 constexpr int kGemmMinTileRows = 32;   // its narrow form (one group per wavefront, deeper ring)
@@ -32,7 +33,7 @@ struct RoutePlanArgs {
   int top_k;
   int experts;
   int tile_rows;
-  int64_t blocks;             // ceil(routes / 256)
+  int64_t blocks;             // ceil(routes / kPlanBlockRoutes)
   int64_t capacity;           // ceil(routes / tile_rows) + experts
   unsigned* block_counts;     // [blocks, experts] scratch
   unsigned* block_invalid;    // [blocks] scratch

@@ -34,21 +34,85 @@ namespace glm53 {
 
 // ------------------------------------------------------------ route plan --
 
-__global__ __launch_bounds__(256) void route_count_kernel(RoutePlanArgs a) {
-  __shared__ unsigned hist[kPlanMaxExperts];
-  __shared__ unsigned bad;
-  for (int e = threadIdx.x; e < a.experts; e += 256) hist[e] = 0;
-  if (threadIdx.x == 0) bad = 0;
+constexpr int kPlanWaves = 16;
+static_assert(kPlanBlockRoutes == 64 * kPlanWaves, "a counted block is one batch of every wavefront");
+
+// Ranks routes first + 64 B w + 64 b + lane (wavefront w of a workgroup of
+// kPlanWaves, batch b < B) among the same expert's earlier routes of its
+// wavefront; a lane's peers (same id in its batch) come from one ballot per
+// id bit, so a batch costs ~12 ballots and one LDS counter round trip
+// instead of a loop over the routes before it.  The wavefronts' counts then
+// turn into their bases: hist[w][e] = routes of expert e in the wavefronts
+// before w.  Returns the workgroup's routes of expert threadIdx.x (0 past the
+// last).  id is -1 past the last route.
+template <int B>
+__device__ __forceinline__ unsigned rank_routes(const RoutePlanArgs& a, int64_t first, int id_bits, unsigned* hist,
+                                                unsigned* invalid_total, int32_t (&id)[B], unsigned (&rank)[B]) {
+  const int t = threadIdx.x, lane = t & 63, w = t >> 6, E = a.experts;
+  unsigned* mine = hist + w * E;
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const int64_t i = first + (static_cast<int64_t>(w) * B + b) * 64 + lane;
+    id[b] = i < a.routes ? a.expert_ids[i] : -1;
+  }
+  for (int e = lane; e < E; e += 64) mine[e] = 0;
+  if (t == 0) *invalid_total = 0;
   __syncthreads();
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
-  if (i < a.routes) {
-    int32_t e = a.expert_ids[i];
-    if (e >= 0 && e < a.experts) atomicAdd(&hist[e], 1u);
-    else atomicAdd(&bad, 1u);
+#pragma unroll
+  for (int b = 0; b < B; ++b) {
+    const int64_t i = first + (static_cast<int64_t>(w) * B + b) * 64 + lane;
+    const bool valid = id[b] >= 0 && id[b] < E;
+    const unsigned long long bad = __ballot(i < a.routes && !valid);
+    if (lane == 0 && bad != 0) atomicAdd(invalid_total, static_cast<unsigned>(__popcll(bad)));
+    unsigned long long peers = __ballot(valid);
+    for (int bit = 0; bit < id_bits; ++bit) {
+      const bool one = (id[b] >> bit) & 1;
+      const unsigned long long ones = __ballot(one);
+      peers &= one ? ones : ~ones;
+    }
+    const unsigned before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers >> 32),
+                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers), 0u));
+    rank[b] = valid ? mine[id[b]] + before : 0u;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every peer has read the counter
+    if (valid && before == 0) mine[id[b]] = rank[b] + static_cast<unsigned>(__popcll(peers));
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next batch reads it
   }
   __syncthreads();
-  for (int e = threadIdx.x; e < a.experts; e += 256) a.block_counts[static_cast<int64_t>(blockIdx.x) * a.experts + e] = hist[e];
-  if (threadIdx.x == 0) a.block_invalid[blockIdx.x] = bad;
+  unsigned run = 0;
+  if (t < E) {
+    unsigned c[kPlanWaves];
+#pragma unroll
+    for (int j = 0; j < kPlanWaves; ++j) c[j] = hist[j * E + t];
+#pragma unroll
+    for (int j = 0; j < kPlanWaves; ++j) {
+      hist[j * E + t] = run;
+      run += c[j];
+    }
+  }
+  __syncthreads();
+  return run;
+}
+
+// Per block of kPlanBlockRoutes routes: the routes per expert, and each
+// route's rank among its expert's routes of the block (inverse holds it until
+// route_scatter_kernel; -1: id out of range), so that the scatter needs no
+// look at other routes.  All three launches are bound by latency: blocks of
+// 1,024 leave the scan a quarter of the rows that blocks of 256 did, and the
+// scatter no loop over up to 255 routes.  Count / scan / scatter at 65,536
+// routes over 288 experts 5.2 / 15.9 / 10.0 -> 5.2 / 10.2 / 6.7 us.
+__global__ __launch_bounds__(64 * kPlanWaves) void route_count_kernel(RoutePlanArgs a, int id_bits) {
+  extern __shared__ unsigned plan_hist[];  // [kPlanWaves][experts]
+  __shared__ unsigned invalid;
+  const int t = threadIdx.x, w = t >> 6;
+  const int64_t first = static_cast<int64_t>(blockIdx.x) * kPlanBlockRoutes;
+  int32_t id[1];
+  unsigned rank[1];
+  const unsigned count = rank_routes<1>(a, first, id_bits, plan_hist, &invalid, id, rank);
+  if (t < a.experts) a.block_counts[static_cast<int64_t>(blockIdx.x) * a.experts + t] = count;
+  if (t == 0) a.block_invalid[blockIdx.x] = invalid;
+  if (first + t >= a.routes) return;
+  const bool valid = id[0] >= 0 && id[0] < a.experts;
+  a.inverse[first + t] = valid ? static_cast<int32_t>(plan_hist[w * a.experts + id[0]] + rank[0]) : -1;
 }
 
 // Inclusive scans of a[0..n) and b[0..n) in LDS (n <= 1024, 1024 threads,
@@ -167,25 +231,16 @@ __global__ __launch_bounds__(1024) void route_scan_kernel(RoutePlanArgs a) {
 }
 
 __global__ __launch_bounds__(256) void route_scatter_kernel(RoutePlanArgs a) {
-  __shared__ int32_t ids[256];
-  const int t = threadIdx.x;
-  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + t;
-  ids[t] = i < a.routes ? a.expert_ids[i] : -1;
-  __syncthreads();
+  const int64_t i = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x;
   if (i >= a.routes) return;
-  const int32_t e = ids[t];
-  if (e < 0 || e >= a.experts) {
-    a.inverse[i] = -1;
-    return;
-  }
-  int rank = 0;
-  for (int j = 0; j < t; ++j) rank += ids[j] == e;
+  const int32_t e = a.expert_ids[i], rank = a.inverse[i];
+  if (rank < 0) return;  // an id out of range
   const int64_t pos = static_cast<int64_t>(a.route_offsets[e]) +
-                      a.block_counts[static_cast<int64_t>(blockIdx.x) * a.experts + e] + rank;
+                      a.block_counts[i / kPlanBlockRoutes * a.experts + e] + rank;
   a.sorted_route[pos] = static_cast<int32_t>(i);
   a.inverse[i] = static_cast<int32_t>(pos);
   a.sorted_expert[pos] = e;
-  a.sorted_token[pos] = static_cast<int32_t>(i / a.top_k);
+  a.sorted_token[pos] = static_cast<int32_t>(static_cast<uint32_t>(i) / static_cast<uint32_t>(a.top_k));
   if (a.scores != nullptr) a.sorted_score[pos] = a.scores[i];
 }
 
@@ -293,64 +348,22 @@ __global__ __launch_bounds__(256) void split_activations_kernel(SplitArgs a) {
   split_unit<V, OPERAND>(a, static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6), threadIdx.x & 63);
 }
 
-// The whole route plan of up to kPlanOneLaunchRoutes routes in one workgroup
-// of 16 wavefronts; wavefront w ranks the routes of its own run of B
-// batches of 64, held in registers from one round of loads.  A lane's peers
-// (same id in its batch) come from one ballot per id bit, so a batch costs
-// ~12 ballots and one LDS counter round trip instead of a loop over the
-// routes before it; the wavefront's counters per expert then turn into its
-// bases by one pass over the 16 rows.  Bound by latency: 5.4 us at 512
-// routes and 8.4 at 2,048 over 288 experts, where the three launches take
-// 11.7 and 12.3; at 3,072 and 4,096 (11.7 and 13.7 with four batches against
-// 13.3 and 13.0) one workgroup's batches cost what the launches do, so
-// larger plans keep those.
-constexpr int kPlanWaves = 16;
+// The whole route plan of up to kPlanOneLaunchRoutes routes in one workgroup,
+// wavefront w's run of B batches held in registers from one round of loads.
+// Bound by latency: 5.4 us at 512 routes and 8.4 at 2,048 over 288 experts,
+// where the three launches of 256-route blocks took 11.7 and 12.3; at 3,072
+// and 4,096 (11.7 and 13.7 with four batches against 13.3 and 13.0) one
+// workgroup's batches cost what the launches do, so larger plans keep those.
 template <int B>
 __device__ __forceinline__ void route_plan_one(const RoutePlanArgs& a, int id_bits, unsigned* hist,
                                                unsigned* route_cum, unsigned* tile_cum, unsigned* invalid_total) {
   const int t = threadIdx.x, lane = t & 63, w = t >> 6, E = a.experts;
-  unsigned* mine = hist + w * E;
   int32_t id[B];
   unsigned rank[B];
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
-    const int64_t i = (static_cast<int64_t>(w) * B + b) * 64 + lane;
-    id[b] = i < a.routes ? a.expert_ids[i] : -1;
-  }
-  for (int e = lane; e < E; e += 64) mine[e] = 0;
-  if (t == 0) *invalid_total = 0;
-  __syncthreads();
-#pragma unroll
-  for (int b = 0; b < B; ++b) {
-    const int64_t i = (static_cast<int64_t>(w) * B + b) * 64 + lane;
-    const bool valid = id[b] >= 0 && id[b] < E;
-    const unsigned long long bad = __ballot(i < a.routes && !valid);
-    if (lane == 0 && bad != 0) atomicAdd(invalid_total, static_cast<unsigned>(__popcll(bad)));
-    unsigned long long peers = __ballot(valid);
-    for (int bit = 0; bit < id_bits; ++bit) {
-      const bool one = (id[b] >> bit) & 1;
-      const unsigned long long ones = __ballot(one);
-      peers &= one ? ones : ~ones;
-    }
-    const unsigned before = __builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(peers >> 32),
-                                                      __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(peers), 0u));
-    rank[b] = valid ? mine[id[b]] + before : 0u;
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // every peer has read the counter
-    if (valid && before == 0) mine[id[b]] = rank[b] + static_cast<unsigned>(__popcll(peers));
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // before the next batch reads it
-  }
-  __syncthreads();
+  const unsigned count = rank_routes<B>(a, 0, id_bits, hist, invalid_total, id, rank);
   if (t < E) {
-    unsigned c[kPlanWaves], run = 0;
-#pragma unroll
-    for (int j = 0; j < kPlanWaves; ++j) c[j] = hist[j * E + t];
-#pragma unroll
-    for (int j = 0; j < kPlanWaves; ++j) {
-      hist[j * E + t] = run;
-      run += c[j];
-    }
-    route_cum[t] = run;
-    tile_cum[t] = (run + a.tile_rows - 1) / a.tile_rows;
+    route_cum[t] = count;
+    tile_cum[t] = (count + a.tile_rows - 1) / a.tile_rows;
   }
   __syncthreads();
   block_scan2_inclusive(route_cum, tile_cum, E);
@@ -363,7 +376,7 @@ __device__ __forceinline__ void route_plan_one(const RoutePlanArgs& a, int id_bi
       a.inverse[i] = -1;
       continue;
     }
-    const int64_t pos = static_cast<int64_t>((e == 0 ? 0u : route_cum[e - 1]) + mine[e] + rank[b]);
+    const int64_t pos = static_cast<int64_t>((e == 0 ? 0u : route_cum[e - 1]) + hist[w * E + e] + rank[b]);
     a.sorted_route[pos] = static_cast<int32_t>(i);
     a.inverse[i] = static_cast<int32_t>(pos);
     a.sorted_expert[pos] = e;
@@ -1583,15 +1596,15 @@ int64_t split_units(const SplitArgs& a) {  // wavefronts
 }  // namespace
 
 hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hipStream_t st) {
+  int id_bits = 0;
+  while ((1 << id_bits) < a.experts) ++id_bits;
+  const size_t lds = sizeof(unsigned) * static_cast<size_t>(kPlanWaves * a.experts);
   if (a.routes <= kPlanOneLaunchRoutes) {
     SplitArgs s{};
     if (split != nullptr) s = *split;
     if (s.cols % kBlock != 0 || s.operand_order) return hipErrorInvalidValue;
-    int id_bits = 0;
-    while ((1 << id_bits) < a.experts) ++id_bits;
     const int64_t split_blocks = s.rows > 0 ? (split_units(s) + kPlanWaves - 1) / kPlanWaves : 0;
     const dim3 grid(static_cast<unsigned>(1 + split_blocks));
-    const size_t lds = sizeof(unsigned) * static_cast<size_t>(kPlanWaves * a.experts);
     if (split_wide(s)) hipLaunchKernelGGL(route_plan_one_kernel<8>, grid, dim3(64 * kPlanWaves), lds, st, a, id_bits, s);
     else hipLaunchKernelGGL(route_plan_one_kernel<2>, grid, dim3(64 * kPlanWaves), lds, st, a, id_bits, s);
     return hipGetLastError();
@@ -1600,9 +1613,9 @@ hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hip
     const hipError_t e = launch_split_activations(*split, st);
     if (e != hipSuccess) return e;
   }
-  hipLaunchKernelGGL(route_count_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(route_count_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(64 * kPlanWaves), lds, st, a, id_bits);
   hipLaunchKernelGGL(route_scan_kernel, dim3(1), dim3(1024), 0, st, a);
-  hipLaunchKernelGGL(route_scatter_kernel, dim3(static_cast<unsigned>(a.blocks)), dim3(256), 0, st, a);
+  hipLaunchKernelGGL(route_scatter_kernel, dim3(static_cast<unsigned>((a.routes + 255) / 256)), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

@@ -57,12 +57,13 @@ def test_tile_plan_kat_sparse_edge_buckets(M, dev):
 @pytest.mark.parametrize("tokens,experts,skew", [(2048, 288, False), (2049, 288, False), (2048, 16, True),
                                                  (2300, 16, True), (130, 1024, False), (1, 9, False),
                                                  (8, 1, True), (9, 64, True), (127, 288, False), (128, 288, True),
-                                                 (129, 8, False), (256, 1024, True), (257, 1024, False)])
+                                                 (129, 8, False), (256, 1024, True), (257, 1024, False),
+                                                 (4096, 288, True), (4097, 1024, False)])
 def test_route_plan_with_invalid_ids(dev, tokens, experts, skew):
     """The route plan (one workgroup up to 2,048 routes, count / scan / scatter
     above) on ids with ~1% out of range
     (negative or >= experts), uniform or skewed (long runs of one expert in
-    every 256-route block), up to 1,024 experts: valid routes in stable
+    every 1,024-route block), up to 1,024 experts, 32 and 33 blocks: valid routes in stable
     expert order (numpy's stable argsort), invalid ones with inverse -1 and
     counted in status[0]."""
     import torch
