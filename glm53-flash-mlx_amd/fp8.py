@@ -173,7 +173,7 @@ class ClampedMLP(torch.nn.Module):
                 and _ops.direct(x, gate, up, down, *scales))
 
     def forward(self, x):
-        # One call of five launches where the four calls took nine: x split
+        # One call of four launches where the four calls took nine: x split
         # once, the SwiGLU in the gate/up product's epilogue (96 tokens,
         # H = 4096, I = 1536: 64 -> 37 us).
         if not self._one_call(x):
