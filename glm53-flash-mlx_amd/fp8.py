@@ -167,9 +167,9 @@ class ClampedMLP(torch.nn.Module):
             return False
         table = _scale_shape(inter, hidden)
         return (tuple(s.shape for s in scales) == (table, table, table[::-1])
-                and all(s.dtype == torch.float32 and s.is_contiguous() for s in scales)
-                and all(w.dtype == torch.uint8 and w.is_contiguous() and w.data_ptr() % 16 == 0
-                        and w.device == x.device for w in (gate, up, down))
+                and all(s.dtype == torch.float32 for s in scales)
+                and all(w.dtype == torch.uint8 and w.data_ptr() % 16 == 0 for w in (gate, up, down))
+                and all(t.is_contiguous() and t.device == x.device for t in (gate, up, down, *scales))
                 and _ops.direct(x, gate, up, down, *scales))
 
     def forward(self, x):

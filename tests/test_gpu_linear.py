@@ -174,6 +174,22 @@ def test_mlp_in_one_call_equals_its_parts(M, dev, rows, with_480):
         mlp(x[..., :128])
 
 
+@pytest.mark.parametrize("name", ["gate_proj", "up_proj", "down_proj"])
+def test_mlp_with_a_scale_table_on_the_host_is_refused(M, dev, name):
+    """A projection whose scale table stayed on the host raises, whatever the
+    number of rows."""
+    import torch
+
+    mlp = M.ClampedMLP(256, 128, 2.0, device=dev)
+    proj = getattr(mlp, name)
+    proj.weight_scale_inv = proj.weight_scale_inv.cpu()
+    for rows in (1, 5):
+        x = torch.zeros((rows, 256), dtype=torch.bfloat16, device=dev)
+        assert not mlp._one_call(x)
+        with pytest.raises(ValueError, match="ROCm device"):
+            mlp(x)
+
+
 @pytest.mark.parametrize("rows", [1, 5, 64])
 def test_both_480_codes_gemv_and_mfma(M, O, dev, rows):
     """Codes over the whole byte range, so 0x7F (+480) and 0xFF (-480) both

@@ -7,7 +7,7 @@ from __future__ import annotations
 
 import pytest
 
-from conftest import submodule
+from conftest import pkg, submodule
 
 torch = pytest.importorskip("torch")
 
@@ -83,3 +83,26 @@ def test_direct_calls_only_where_the_op_would_reach_its_kernel_alone():
     assert seen and not any(seen)
     assert torch.equal(torch.compile(lambda v: v + 1 if ops.direct(v) else v - 1, backend="eager")(x), x - 1)
     assert ops.direct(x)
+
+
+@pytest.fixture
+def mlp_and_rows(monkeypatch):
+    """A ClampedMLP and rows for it whose device addresses are never used."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    monkeypatch.setattr(submodule("ops"), "direct", lambda *tensors: True)
+    with FakeTensorMode():
+        yield pkg().ClampedMLP(256, 384, 2.0, device="cuda"), torch.empty((4, 256), dtype=torch.bfloat16, device="cuda")
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor")
+@pytest.mark.parametrize("name", ["gate_proj", "up_proj", "down_proj"])
+@pytest.mark.parametrize("buffer", ["weight", "weight_scale_inv"])
+def test_mlp_in_one_call_only_with_every_buffer_on_the_rows_device(mlp_and_rows, name, buffer):
+    """glm53_mlp takes the buffers by their addresses; one on the host must
+    reach the projections, which refuse it."""
+    mlp, x = mlp_and_rows
+    assert mlp._one_call(x)
+    proj = getattr(mlp, name)
+    setattr(proj, buffer, torch.empty_like(getattr(proj, buffer), device="cpu"))
+    assert not mlp._one_call(x)
