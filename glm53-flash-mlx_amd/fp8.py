@@ -124,6 +124,12 @@ class BlockFP8Linear(torch.nn.Module):
             self._code_flags = (stamp, N.scan_codes(self.weight))
         return self._code_flags[1]
 
+    def widths_hold(self) -> bool:
+        """Whether in_features and out_features, which as_c_struct passes on,
+        are the weight's: a call on the tensors goes by the weight's shape
+        alone, also after a weight of another size took its place."""
+        return self.weight.shape == (self.out_features, self.in_features)
+
     def as_c_struct(self) -> N.Linear:
         return N.Linear(self.weight.data_ptr(), self.weight_scale_inv.data_ptr(), self.out_features, self.in_features,
                         self.code_flags().data_ptr())
@@ -156,7 +162,8 @@ class ClampedMLP(torch.nn.Module):
         if type(self) is not ClampedMLP or rows < 2 or x.dtype != torch.bfloat16 or not x.is_cuda:
             return False
         projections = (self.gate_proj, self.up_proj, self.down_proj)
-        if any(type(p) is not BlockFP8Linear or p.bias is not None or _hooked(p) for p in projections):
+        if any(type(p) is not BlockFP8Linear or p.bias is not None or _hooked(p) or not p.widths_hold()
+               for p in projections):
             return False
         gate, up, down = (p.weight for p in projections)
         scales = tuple(p.weight_scale_inv for p in projections)

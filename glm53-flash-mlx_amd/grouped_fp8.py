@@ -336,7 +336,7 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
             for proj, shape in ((shared.gate_proj, (width, bank.hidden_size)),
                                 (shared.up_proj, (width, bank.hidden_size)),
                                 (shared.down_proj, (bank.hidden_size, width))):
-                if type(proj) is not BlockFP8Linear or _hooked(proj) or proj.bias is not None:
+                if type(proj) is not BlockFP8Linear or _hooked(proj) or proj.bias is not None or not proj.widths_hold():
                     return False
                 weights.append(proj.weight)
                 tables.append(proj.weight_scale_inv)

@@ -106,3 +106,47 @@ def test_mlp_in_one_call_only_with_every_buffer_on_the_rows_device(mlp_and_rows,
     proj = getattr(mlp, name)
     setattr(proj, buffer, torch.empty_like(getattr(proj, buffer), device="cpu"))
     assert not mlp._one_call(x)
+
+
+def _empty_linear(out_features, in_features):
+    """A BlockFP8Linear of an earlier size with buffers of the sizes given."""
+    proj = pkg().BlockFP8Linear(128, 128, device="cuda")
+    proj.weight = torch.empty((out_features, in_features), dtype=torch.uint8, device="cuda")
+    proj.weight_scale_inv = torch.empty((-(-out_features // 128), -(-in_features // 128)), device="cuda")
+    return proj
+
+
+@pytest.fixture
+def moe_and_rows(mlp_and_rows):
+    """A SortedGroupedFP8MoE with a shared expert, and a few rows for it, of
+    which no device address is ever used."""
+    from types import SimpleNamespace
+
+    M = pkg()
+    shared, x = mlp_and_rows
+    cfg = SimpleNamespace(hidden_size=256, moe_intermediate_size=128, swiglu_limit=2.0, n_routed_experts=4,
+                          num_experts_per_tok=2, n_shared_experts=1)
+    put = lambda *shape, dtype=torch.uint8: M.owned_tensor(  # noqa: E731
+        torch.empty(shape, dtype=dtype, device="cuda"), layout=M.TensorLayout.ROW_MAJOR_CONTIGUOUS)
+    bank = M.PackedFP8ExpertBank(put(4, 256, 256), put(4, 2, 2, dtype=torch.float32), put(4, 256, 128),
+                                 put(4, 2, 1, dtype=torch.float32), intermediate_size=128)
+    gate = M.Float32Gate(torch.empty((4, 256), device="cuda"), torch.empty(4, device="cuda"), top_k=2)
+    return M.SortedGroupedFP8MoE(bank, cfg, gate, shared), x
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor")
+def test_projections_of_another_width_than_their_attributes_run_by_their_tensors(moe_and_rows):
+    """The projections go by their tensors' shapes, the C structs by
+    in_features and out_features: where these differ (buffers of another size
+    were assigned), neither the one-call MLP nor the few-token prefill is
+    taken."""
+    moe, x = moe_and_rows
+    mlp = moe.shared_experts
+    assert mlp._one_call(x) and moe._few_routes_on_device(x, 4)
+    sizes = {"gate_proj": (384, 256), "up_proj": (384, 256), "down_proj": (256, 384)}
+    for name, size in sizes.items():
+        kept = getattr(mlp, name)
+        setattr(mlp, name, _empty_linear(*size))
+        assert not mlp._one_call(x) and not moe._few_routes_on_device(x, 4), name
+        setattr(mlp, name, kept)
+    assert mlp._one_call(x) and moe._few_routes_on_device(x, 4)
