@@ -306,8 +306,8 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
         """Whether a call below min_routes can run as one grouped prefill in
         the Direct order, which gives the Direct loop's bytes (every route and
         the shared expert on the same MFMA tree, the same accumulation order):
-        the plan's widths, a plain Float32Gate over the bank's experts, a
-        shared expert whose forward is the plan's (plain block-FP8
+        the plan's widths, expert views as the bank gave them, a plain
+        Float32Gate over the bank's experts, a shared expert whose forward is the plan's (plain block-FP8
         projections without bias, the layer's limit, no hooks), and buffers
         that the native call can take by their addresses.  Anything else,
         traced calls, and batches of over 4,096 routes stay with the loop."""
@@ -321,7 +321,7 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
             return False
         if bank.hidden_size % BLOCK_SIZE or bank.intermediate_size % BLOCK_SIZE or bank.expert_count > PLAN_MAX_EXPERTS:
             return False
-        if self._expert_views[0].limit != limit or self._expert_views[0].gate_proj._bank is not bank:
+        if self._expert_views[0].limit != limit or not self._views_are_the_banks():
             return False
         weights = [bank.gate_up_weight, bank.down_weight]
         tables = [bank.gate_up_scale_inv, bank.down_scale_inv, gate.weight, gate.e_score_correction_bias]

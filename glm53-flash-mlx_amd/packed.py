@@ -25,7 +25,21 @@ from .ownership import (ResidentTensor, TensorLayout, borrowed_stable_tensor, ow
 from .router import Float32Gate
 
 
-class _PackedLinearView:
+class _Watched:
+    """Notes in the set given to `watch` the names of attributes set from then on."""
+
+    _edits = None
+
+    def __setattr__(self, name, value):
+        object.__setattr__(self, name, value)
+        if self._edits is not None:
+            self._edits.add(name)
+
+    def watch(self, edits: set) -> None:
+        object.__setattr__(self, "_edits", edits)
+
+
+class _PackedLinearView(_Watched):
     """One projection of one bank expert.  In a row-major bank its rows are a
     contiguous slice (no copy); in a row-group bank `weight` returns the
     expert's rows re-laid into the reference row-major layout (a copy)."""
@@ -57,7 +71,7 @@ class _PackedLinearView:
         return block_fp8_linear(x, self.weight, self.weight_scale_inv, flags)
 
 
-class _PackedExpertView:
+class _PackedExpertView(_Watched):
     def __init__(self, bank: "PackedFP8ExpertBank", expert_id: int, limit: float):
         inter = bank.intermediate_size
         scale_rows = bank.intermediate_scale_rows
@@ -674,11 +688,25 @@ class PackedFP8MoE(DirectFP8MoE):
         self.gate = gate
         self.shared_experts = shared_experts
         self._expert_views = tuple(bank.expert(i, limit=config.swiglu_limit) for i in range(bank.expert_count))
+        self._view_edits: set = set()  # non-empty: some view is no longer as the bank gave it
+        for view in self._expert_views:
+            for part in (view, view.gate_proj, view.up_proj, view.down_proj):
+                part.watch(self._view_edits)
         self._plans: dict = {}
         self._op_key = ops.register_owner(self)
 
     def _expert(self, expert_id: int):
         return self._expert_views[expert_id]
+
+    def _views_are_the_banks(self) -> bool:
+        """Whether every expert view still stands for its matrices of
+        self.bank under the limit of construction.  The views were made
+        together, so the tensors of one speak for all while none was edited."""
+        bank, view = self.bank, self._expert_views[0]
+        gate_up, down = view.gate_proj, view.down_proj
+        return (not self._view_edits and "_expert" not in self.__dict__ and gate_up._bank is bank
+                and gate_up._bank_weight is bank.gate_up_weight and down._bank_weight is bank.down_weight
+                and gate_up._bank_scale_inv is bank.gate_up_scale_inv and down._bank_scale_inv is bank.down_scale_inv)
 
     def _plan(self, device) -> DecodePlan:
         key = (device.index, torch.cuda.current_stream(device).cuda_stream)

@@ -150,3 +150,25 @@ def test_projections_of_another_width_than_their_attributes_run_by_their_tensors
         assert not mlp._one_call(x) and not moe._few_routes_on_device(x, 4), name
         setattr(mlp, name, kept)
     assert mlp._one_call(x) and moe._few_routes_on_device(x, 4)
+
+
+@pytest.mark.filterwarnings("ignore:Accessing the data pointer of FakeTensor")
+@pytest.mark.parametrize("expert", [0, 1, 3])
+def test_few_token_prefill_only_over_expert_views_as_the_bank_gave_them(moe_and_rows, expert):
+    """The loop that the prefill stands for runs every touched expert's own
+    view: an edit of any of them keeps the loop, and so do tensors of the bank
+    that are no longer the views'."""
+    moe, x = moe_and_rows
+    view = moe._expert(expert)
+    edits = [(view, "limit", 3.0), (view, "down_proj", lambda rows: rows), (view.up_proj, "row_offset", 0),
+             (moe.bank, "down_scale_inv", torch.empty_like(moe.bank.down_scale_inv)), (moe, "_expert", lambda e: view)]
+    for part, name, value in edits:
+        moe._view_edits.clear()
+        assert moe._few_routes_on_device(x, 4)
+        kept = getattr(part, name)
+        setattr(part, name, value)
+        assert not moe._few_routes_on_device(x, 4), name
+        if part is moe:
+            del part._expert
+        else:
+            setattr(part, name, kept)
