@@ -120,14 +120,17 @@ int dense(DenseArgs d, const void* x, const SplitBuf& space, bool swiglu, int32_
     HIP_TRY(launch_dense_linear(d, tile, swiglu, st), "dense linear launch");
     return GLM53_OK;
   }
-  auto flag_of = [&](const int32_t* flag, const uint8_t* weight, int32_t* space) -> const int32_t* {
-    if (flag != nullptr) return flag;
-    return launch_scan_480(weight, d.N * d.K, space, true, st) == hipSuccess ? space : nullptr;
-  };
   GroupedGemmArgs g{};
-  g.fixup = flag_of(d.flag, d.weight, flags);
-  if (swiglu) g.fixup_up = flag_of(d.flag_up, d.weight_up, flags + 1);
-  if (g.fixup == nullptr || (swiglu && g.fixup_up == nullptr)) return hip_fail(hipGetLastError(), "scan launch");
+  g.fixup = d.flag;
+  g.fixup_up = d.flag_up;
+  if (g.fixup == nullptr) {
+    HIP_TRY(launch_scan_480(d.weight, d.N * d.K, flags, true, st), "scan launch");
+    g.fixup = flags;
+  }
+  if (swiglu && g.fixup_up == nullptr) {
+    HIP_TRY(launch_scan_480(d.weight_up, d.N * d.K, flags + 1, true, st), "scan launch");
+    g.fixup_up = flags + 1;
+  }
   g.a_hi = d.a_hi;
   g.a_lo = d.a_lo;
   g.a_scale = d.a_scale;
