@@ -181,11 +181,17 @@ def check(status: int) -> None:
     raise RuntimeError(message)
 
 
+# a private name, ~2 us a call below torch.cuda.current_stream's Stream object
+_raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+
+
 def stream_handle(device: torch.device | None = None) -> int:
     """The hipStream_t of torch's current stream on `device` (the current
     device when None or without an index)."""
     index = device.index if device is not None else None
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)
+    if _raw_stream is None:
+        return torch.cuda.current_stream(index).cuda_stream
+    return _raw_stream(torch.cuda.current_device() if index is None else index)
 
 
 def require_device(*tensors: torch.Tensor) -> None:

@@ -45,6 +45,28 @@ def register_owner(module) -> int:
 _PLAIN_TENSORS = (torch.Tensor, torch.nn.Parameter, torch.nn.Buffer)
 
 
+def _dispatch_probe():
+    """A function that tells whether anything acts between an eager call and
+    its kernel.  It asks torch's private state; where this torch lacks one of
+    the names, the function says yes and every call goes through the op."""
+    try:
+        c, forward_ad, profiling = torch._C, torch.autograd.forward_ad, torch.autograd._profiler_enabled
+        tracing, transforms = c._get_tracing_state, c._functorch.peek_interpreter_stack
+        dispatch_modes, function_modes = c._len_torch_dispatch_stack, c._len_torch_function_stack
+        forward_ad._current_level
+    except AttributeError:
+        return lambda: True
+
+    def acts() -> bool:
+        return bool(torch.compiler.is_compiling() or tracing() is not None or dispatch_modes() or function_modes()
+                    or transforms() is not None or forward_ad._current_level >= 0 or profiling())
+
+    return acts
+
+
+_dispatch_acts = _dispatch_probe()
+
+
 def direct(*tensors) -> bool:
     """True when dispatching an op on `tensors` could only reach its device
     kernel, so that an eager call may run the native call itself: the custom
@@ -55,10 +77,7 @@ def direct(*tensors) -> bool:
     compilation, dispatch and function modes, functorch transforms, forward-
     and reverse-mode differentiation, a recording profiler, tensor
     subclasses."""
-    if (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None
-            or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
-            or torch._C._functorch.peek_interpreter_stack() is not None
-            or torch.autograd.forward_ad._current_level >= 0 or torch.autograd._profiler_enabled()):
+    if _dispatch_acts():
         return False
     grad = torch.is_grad_enabled()
     for t in tensors:

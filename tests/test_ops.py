@@ -85,6 +85,33 @@ def test_direct_calls_only_where_the_op_would_reach_its_kernel_alone():
     assert ops.direct(x)
 
 
+@pytest.mark.parametrize("place,name", [("_C", "_get_tracing_state"), ("_C", "_len_torch_dispatch_stack"),
+                                        ("_C", "_len_torch_function_stack"),
+                                        ("_C._functorch", "peek_interpreter_stack"),
+                                        ("autograd.forward_ad", "_current_level"),
+                                        ("autograd", "_profiler_enabled")])
+def test_no_direct_calls_with_a_torch_that_lacks_a_name(monkeypatch, place, name):
+    """ops.direct asks private state of torch; without it every call goes
+    through the op."""
+    from functools import reduce
+
+    ops, x = submodule("ops"), torch.zeros(4)
+    with monkeypatch.context() as m:
+        m.delattr(reduce(getattr, place.split("."), torch), name)
+        probe = ops._dispatch_probe()
+    monkeypatch.setattr(ops, "_dispatch_acts", probe)
+    assert not ops.direct(x)
+
+
+def test_stream_handle_without_the_raw_stream_name(monkeypatch):
+    from types import SimpleNamespace
+
+    N = submodule("_native")
+    monkeypatch.setattr(N, "_raw_stream", None)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda device=None: SimpleNamespace(cuda_stream=(device, 7)))
+    assert N.stream_handle() == (None, 7) and N.stream_handle(torch.device("cuda", 3)) == (3, 7)
+
+
 @pytest.fixture
 def mlp_and_rows(monkeypatch):
     """A ClampedMLP and rows for it whose device addresses are never used."""
