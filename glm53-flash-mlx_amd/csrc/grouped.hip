@@ -1518,51 +1518,49 @@ __global__ __launch_bounds__(256) void restore_reduce_kernel(ReduceArgs a) {
 // Thread = V consecutive columns; loads are issued as above, in sorted order.
 // The order comes from ranks (slots of a smaller id, and earlier slots of the
 // same one, before it) and selects: every array index is static, and the
-// ids, positions and scores are uniform.  (A sort that indexed its arrays at
-// run time kept them in scratch memory: 64 tokens x 4096 columns 10.6 us,
-// 6.4 with the ranks.)
+// ids, positions and scores are uniform.  K is top_k itself: a form for any
+// top_k with all kMaxReduceTopK slots unrolled spends their ranks and loads
+// on slots that are not there.  Measured (us; a sort in scratch memory / the
+// form for any top_k / this): 64 tokens x 4096 columns 4.5 / 10.8 / 2.7 at
+// top_k 2, 9.6 / 4.9 (as this) at 8, 20.8 / 15.3 / 12.8 at 16; 4,096 tokens
+// 30.8 / 143 / 17.2 at top_k 2, 148 / 164 / 97 at 12; 64 x 1023 columns, one
+// per thread, 8.9 / 12.1 / 3.9 at 8.
 template <int V, int K>
 __global__ __launch_bounds__(256) void direct_order_reduce_kernel(ReduceArgs a) {
-  constexpr int kSlots = K > 0 ? K : kMaxReduceTopK;  // K = 0: top_k known only at run time
-  const int k = K > 0 ? K : a.top_k;
   const int64_t t = blockIdx.y;
   const int64_t h0 = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * V;
   if (h0 >= a.H) return;
-  int32_t id[kSlots], slot_pos[kSlots];
-  float slot_score[kSlots];
+  int32_t id[K], slot_pos[K];
+  float slot_score[K];
 #pragma unroll
-  for (int s = 0; s < kSlots; ++s) {
-    const int64_t i = t * k + (s < k ? s : 0);
+  for (int s = 0; s < K; ++s) {
+    const int64_t i = t * K + s;
     id[s] = a.expert_ids[i];
     slot_pos[s] = a.inverse[i];
     slot_score[s] = a.route_score[i];
   }
-  int32_t pos[kSlots];
-  float score[kSlots];
+  int32_t pos[K];
+  float score[K];
 #pragma unroll
-  for (int r = 0; r < kSlots; ++r) {
+  for (int r = 0; r < K; ++r) {
     pos[r] = 0;
     score[r] = 0.0f;
   }
 #pragma unroll
-  for (int s = 0; s < kSlots; ++s) {
+  for (int s = 0; s < K; ++s) {
     int rank = 0;
 #pragma unroll
-    for (int o = 0; o < kSlots; ++o)
-      if (o < k) rank += o < s ? id[o] <= id[s] : id[o] < id[s];
+    for (int o = 0; o < K; ++o) rank += o < s ? id[o] <= id[s] : id[o] < id[s];
 #pragma unroll
-    for (int r = 0; r < kSlots; ++r) {
-      const bool here = s < k && rank == r;
+    for (int r = 0; r < K; ++r) {
+      const bool here = rank == r;
       pos[r] = here ? slot_pos[s] : pos[r];
       score[r] = here ? slot_score[s] : score[r];
     }
   }
-  Bf16Run<V> row[kSlots];
+  Bf16Run<V> row[K];
 #pragma unroll
-  for (int r = 0; r < kSlots; ++r) {
-    row[r].clear();
-    if (r < k) row[r].load(a.route_out + static_cast<int64_t>(pos[r] < 0 ? 0 : pos[r]) * a.H + h0);
-  }
+  for (int r = 0; r < K; ++r) row[r].load(a.route_out + static_cast<int64_t>(pos[r] < 0 ? 0 : pos[r]) * a.H + h0);
   Bf16Run<V> sh;
   sh.clear();
   if (a.shared != nullptr) sh.load(a.shared + t * a.H + h0);
@@ -1570,8 +1568,7 @@ __global__ __launch_bounds__(256) void direct_order_reduce_kernel(ReduceArgs a) 
 #pragma unroll
   for (int i = 0; i < V; ++i) total[i] = 0.0f;
 #pragma unroll
-  for (int r = 0; r < kSlots; ++r) {
-    if (r >= k) continue;
+  for (int r = 0; r < K; ++r) {
 #pragma unroll
     for (int i = 0; i < V; ++i) {
       const float v = pos[r] < 0 ? __builtin_nanf("") : row[r].get(i);
@@ -1721,21 +1718,31 @@ hipError_t launch_scan_480(const uint8_t* codes, int64_t n, int32_t* flag, bool 
   return hipGetLastError();
 }
 
+namespace {
+// direct_order_reduce_kernel for a.top_k, 1 .. K
+template <int V, int K = kMaxReduceTopK>
+void launch_direct_order(const ReduceArgs& a, dim3 grid, hipStream_t st) {
+  if constexpr (K > 1) {
+    if (a.top_k < K) return launch_direct_order<V, K - 1>(a, grid, st);
+  }
+  hipLaunchKernelGGL((direct_order_reduce_kernel<V, K>), grid, dim3(256), 0, st, a);
+}
+}  // namespace
+
 hipError_t launch_reduce(const ReduceArgs& a, bool direct_order, hipStream_t st) {
   if (a.tokens == 0) return hipSuccess;
-  if (a.top_k > kMaxReduceTopK) return hipErrorInvalidValue;
+  if (a.top_k < 1 || a.top_k > kMaxReduceTopK) return hipErrorInvalidValue;
   auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
   const bool wide = a.H % 8 == 0 && a16(a.route_out) && a16(a.out) && a16(a.shared) && a16(a.hc_residual) &&
                     a16(a.hc_out);
   const int64_t per_thread = wide ? 8 : 1;
   const dim3 grid(static_cast<unsigned>((a.H / per_thread + 255) / 256), static_cast<unsigned>(a.tokens));
   if (wide) {
-    if (direct_order && a.top_k == 8) hipLaunchKernelGGL((direct_order_reduce_kernel<8, 8>), grid, dim3(256), 0, st, a);
-    else if (direct_order) hipLaunchKernelGGL((direct_order_reduce_kernel<8, 0>), grid, dim3(256), 0, st, a);
+    if (direct_order) launch_direct_order<8>(a, grid, st);
     else if (a.top_k == 8) hipLaunchKernelGGL((restore_reduce_kernel<8, 8>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((restore_reduce_kernel<8, 0>), grid, dim3(256), 0, st, a);
   } else {
-    if (direct_order) hipLaunchKernelGGL((direct_order_reduce_kernel<1, 0>), grid, dim3(256), 0, st, a);
+    if (direct_order) launch_direct_order<1>(a, grid, st);
     else hipLaunchKernelGGL((restore_reduce_kernel<1, 0>), grid, dim3(256), 0, st, a);
   }
   return hipGetLastError();

@@ -222,10 +222,11 @@ def test_reductions_at_any_width_and_alignment_match_oracle(M, O, dev, hidden, o
     assert np.array_equal(to_bits(out), want)
 
 
-@pytest.mark.parametrize("k,hidden", [(1, 64), (5, 72), (8, 2056), (8, 63), (16, 64)])
+@pytest.mark.parametrize("k,hidden", [(1, 64), (5, 72), (8, 2056), (8, 63), (16, 64)]
+                         + [(k, h) for k in range(1, 17) for h in (80, 33)])
 def test_direct_reduction_order_with_equal_and_missing_experts(O, dev, k, hidden):
     """Ascending expert id, equal ids in slot order, a route without a sorted
-    position NaN: top_k 8 (its own form) and others, 8 columns and 1 column
+    position NaN: every top_k (each has its own form), 8 columns and 1 column
     per thread, against the accumulation written out in BF16 steps."""
     import torch
 
