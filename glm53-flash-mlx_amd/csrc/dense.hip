@@ -13,7 +13,7 @@ namespace {
 
 constexpr int kDenseWaves = 8;
 constexpr int64_t kWideDenseMaxK = 1 << 14;  // 128 x 512 items: 128 K blocks of scales beside their stages
-constexpr int64_t kDenseMaxK = 1 << 18;  // its weight scales take 8 KB of LDS
+constexpr int64_t kDenseMaxK = 1 << 18;  // its weight scales take 16 KB of LDS (gate and up)
 template <int V>
 struct Int {
   static constexpr int value = V;
@@ -389,47 +389,77 @@ hipError_t launch_ksplit(const DenseArgs& a, hipStream_t st) {
 
 // The smallest tile whose items fit one round of a workgroup per CU: a
 // larger tile brings fewer bytes per output but takes longer per round, and
-// a second round costs more than the larger tile does.  Measured (us, N =
-// 4096, K = 4096, each tile at its last one-round row count and just past
-// it): 16 x 16 6.6 at 16 rows, 12 at 32, where 16 x 32 takes 7.6; 32 x 32
-// 10.0 at 64 rows, 17.2 at 96, where 32 x 64 takes 12.7; 32 x 64 13.0 at
-// 128, 22.7 at 200; 32 x 128 (grouped GEMM) 26.8 at 200, 40.5 at 300; 64 x
-// 128 29.2 at 300 rows, 34.8 at 512 (256 items, where 128 x 128 takes 32.2:
-// its two workgroups per CU share the load path from about 224 items on);
-// 128 x 128 (wide shape) 37.6 at 1,024, 66.2 at 1,500; 128 x 256 49.0 at
-// 1,500, 58.0 at 2,048, 118 at 4,096; 128 x 512 74.6 at 2,048 and 97.3 at
-// 4,096, one round of the matrix pipes at 2.8 PFLOP/s counting both passes.
-// (64 x 128 took every row count before: 22.2 at 16 rows, 28.1 at 128, 77.3
-// at 2,048, 156 at 4,096.)  The narrow tiles' offsets fit 32 bits, the wide
-// shape's 31.
+// a second round mostly costs more than the larger tile does.  All figures
+// are us per call, split included, of replayed graphs over weights that no
+// cache holds.  N = 4096, K = 4096, each tile at its last one-round row count
+// and just past it: 16 x 16 11.6 at 16 rows, 19.5 at 24, where 16 x 32 takes
+// 12.4; 16 x 32 12.6 at 32, 21.7 at 48, where 32 x 32 takes 13.0; 32 x 32 14.2
+// at 64, 21.5 at 96, where 32 x 64 takes 17.0; 32 x 64 17.7 at 128, 28.8 at
+// 200 (32 x 128 32.0); 64 x 128 34.5 at 400 and 39.5 at 512 (256 items, where
+// 128 x 128 takes 38.9: two workgroups per CU share the load path); 128 x 128
+// 46.5 at 1,024; 128 x 256 57.4 at 1,500; 128 x 512 74.6 at 2,048 and 97.3 at
+// 4,096 (kernel alone), one round of the matrix pipes at 2.8 PFLOP/s counting
+// both passes.  (64 x 128 takes 25.6 at 16 rows, 32.5 at 128, 85.2 at 2,048.)
+// Where a tile's items are not the whole of it:
+// * 32 x 128 streams the weights past the caches, so row groups that read the
+//   same columns again pay for it unless the matrix is small or the K loop
+//   long: 32 x 128 / 64 x 128 at 256 x 4096 x 1536 18.6 / 17.3, 288 x 3072 x
+//   3072 27.7 / 26.6; but 160 x 6144 x 2048 0.95 of it, 2,048 x 512 x 7168
+//   50.7 / 58.3, 200 x 4096 x 8192 52.9 / 59.6.
+// * 64 x 128 has two workgroups per CU.  Over few columns (activations are
+//   most of the bytes) it beats the 128-row tiles up to 512 items: 4,096 x 512
+//   x 512 13.3 / 15.5 (128 x 128), 2,048 x 1536 x 4096 42.3 / 44.1; and where
+//   128 x 128 no longer fits, 128 x 256: 320 x 12288 x 4096 46.2 / 54.5.  Over
+//   a matrix of more than 16 MB it wins up to 256 items (twice the CUs that
+//   128 x 128 has busy: 256 x 8192 x 7168 63.0 / 67.5, 128 x 16384 x 4096 39.5 /
+//   43.0; 256 x 8192 x 512 12.4 / 11.1), and from 32 MB on at 257 to 384 rows,
+//   where 128 x 128 has three row groups (384 x 8192 x 7168 65.9 / 69.6).
+// * Few rows over more columns than one round of 128 x 256 holds are a
+//   stream of the weights: 32 x 128 (16 x 131072 x 4096 106 us, 128 x 512 133,
+//   64 x 128 131; not for a few K blocks: 2 x 131072 x 512 21.8 / 18.1), and
+//   128 x 256 for up to 64 rows where 128 x 512 needs a second round (48 x
+//   151936 x 7168 231 / 253).
+// The narrow tiles' offsets fit 32 bits, the wide shape's 31.
 // A SwiGLU tile holds half as many output columns in the same time (gate and
-// up tile side by side), so 16 x 16 has no SwiGLU form of its own.
+// up tile side by side), so 16 x 16 and 128 x 128 have no SwiGLU form.
 DenseTile dense_tile(int64_t rows, int64_t K, int64_t N, bool swiglu) {
-  struct Candidate {
-    DenseTile tile;  // weight columns
-    int64_t items;   // at most
-  };
-  constexpr Candidate kTiles[] = {{{16, 16}, 256},  {{16, 32}, 256},  {{32, 32}, 256},   {{32, 64}, 256},
-                                  {{32, 128}, 256}, {{64, 128}, 224}, {{128, 128}, 256}, {{128, 256}, 256}};
+  constexpr DenseTile kNarrow[] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}};  // weight columns
   const bool narrow = K <= kDenseMaxK && N * K < (int64_t{1} << 32) && rows * K < (int64_t{1} << 32);
   const bool wide = K <= kWideDenseMaxK && wide_offsets_fit(N, K, rows);
   auto of = [&](DenseTile t) { return DenseTile{t.rows, swiglu ? t.cols / 2 : t.cols}; };
-  for (const Candidate& c : kTiles) {
-    if (c.tile.cols < 128 ? !narrow : c.tile.rows == 128 && !wide) continue;
-    if (swiglu && (c.tile.cols == 16 || (c.tile.rows == 128 && c.tile.cols == 128))) continue;
-    const DenseTile t = of(c.tile);
-    if (((rows + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols) <= c.items) return t;
+  auto items = [&](DenseTile t) {
+    t = of(t);
+    return ((rows + t.rows - 1) / t.rows) * ((N + t.cols - 1) / t.cols);
+  };
+  for (const DenseTile& t : kNarrow)
+    if (narrow && !(swiglu && t.cols == 16) && items(t) <= 256) return of(t);
+  if (items({32, 128}) <= 256 && (swiglu || rows <= 192 || N <= 2048 || K >= 4096)) return of({32, 128});
+  if (!wide) return of({64, 128});
+  int64_t most = 224;
+  if (!swiglu) {
+    if (N <= 2048 || (N <= 3072 && K >= 2048) || (rows > 128 && items({128, 128}) > 256)) most = 512;
+    else if (rows > 256 && rows <= 384 && N * K >= (int64_t{1} << 25)) most = 384;
+    else if (N * K > (int64_t{1} << 24)) most = 256;
   }
-  return of(wide ? DenseTile{128, 512} : DenseTile{64, 128});
+  if (items({64, 128}) <= most) return of({64, 128});
+  if (!swiglu && items({128, 128}) <= 256) return of({128, 128});
+  if (items({128, 256}) <= 256) return of({128, 256});
+  if (!swiglu && rows <= 32 && K >= 1024) return of({32, 128});
+  if (!swiglu && rows <= 64 && items({128, 512}) > 256) return of({128, 256});
+  return of({128, 512});
 }
 
 // One-pair tiles split their own blocks: the conversion (~55 instructions per
 // 8 columns, every workgroup for its 16 rows, the four rows of a lane side by
 // side: one after the other they took 13.3 us) makes the kernel 11.6 us at 16
 // x 4096 x 4096 where split and product take 3.7 + 7.0 and a launch between,
-// and saves that launch and the workspace: 11.9 us a call instead of 16.0.
-// The conversion grows with K where the split's launch does not, so long rows
-// keep the launch.
+// and saves that launch and the workspace.  The conversion grows with K where
+// the split's launch does not.  Eager calls of 16 rows over 4096 columns (us,
+// in the kernel / by a launch): 11.4 / 15.4 at K = 4096, 14.5 / 15.4 at 6144,
+// 16.0 / 15.5 at 7168, 18.1 / 15.5 at 8192: past ~6,700 it keeps the workspace
+// away but no longer saves time, and longer rows keep the launch.  In a
+// replayed graph, where a launch costs little, the launch is the quicker one:
+// 11.6 / 9.4 at K = 4096, 19.4 / 15.2 at 8192.
 bool dense_splits_x(DenseTile t, int64_t K, bool swiglu) {
   return t.rows == 16 && dense_ksplit(t, swiglu) && K <= 8192;
 }

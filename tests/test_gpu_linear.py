@@ -100,10 +100,9 @@ def test_multi_row_mfma_path_matches_oracle(M, O, dev, rows):
 @pytest.mark.parametrize("rows,k", [(2, 128), (17, 4224), (250, 1152), (499, 1152), (999, 1152), (1999, 640),
                                     (2800, 256), (4801, 384), (11000, 128), (16500, 256)])
 def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
-    """Row counts that take each output tile of the several-row linear in turn
-    (16 x 16 twice, 16 x 32, 32 x 32, 32 x 64, 32 x 128, 64 x 128, 128 x 128, 128 x 256
-    and 128 x 512 at 272 columns), the last row and
-    column tiles ragged, K of 1 to 33 blocks.
+    """Row counts that take one output tile of the several-row linear after
+    the other at 272 columns (16 x 16 to 64 x 128, then 128 x 256 and 128 x 512),
+    the last row and column tiles ragged, K of 1 to 33 blocks.
     Without a code flag a few 0x7F / 0xFF in one tile must be found."""
     rng = np.random.default_rng(rows + k)
     n = 272
@@ -113,6 +112,34 @@ def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
     scale = (rng.uniform(size=(-(-n // 128), k // 128)) * 0.002).astype(np.float32)
     x = O.f32_to_bf16(rng.normal(size=(rows, k)).astype(np.float32))
     assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
+
+
+@pytest.mark.parametrize("with_480", [False, True])
+@pytest.mark.parametrize("rows,n,k", [(450, 4112, 256), (1100, 4112, 256), (2100, 4112, 128), (190, 4112, 1664),
+                                      (195, 4112, 1664), (1500, 3088, 256), (600, 2064, 384), (230, 8208, 2176),
+                                      (300, 8208, 4224), (33, 16400, 2176), (2, 65552, 1024), (32, 65552, 896),
+                                      (33, 65552, 1024), (3, 131088, 128), (40, 131088, 128)])
+def test_dense_tile_rule_on_wide_outputs_matches_oracle(M, O, dev, rows, n, k, with_480):
+    """Both sides of the tile rule's lines: 128 x 128 and wider over many
+    columns, 32 x 128 by its rows, 64 x 128 by columns, matrix size and row
+    groups, few rows over more columns than a round of 128 x 256 holds; the
+    last row and column tiles ragged.  Checked on 64 of the rows and a run of
+    columns at either end and in the middle (columns do not mix), taken
+    together: about 1.2% of the outputs lie one BF16 step off, and over the
+    544 outputs of the smallest case 5% is more than five deviations away."""
+    rng = np.random.default_rng(rows + n + k)
+    codes = rng.integers(0, 0x7F, size=(n, k), dtype=np.uint8)
+    if with_480:
+        codes[0, 0], codes[n - 1, k - 1], codes[n // 2, k // 2] = 0x7F, 0xFF, 0xFF
+    scale = (rng.uniform(size=(-(-n // 128), k // 128)) * 0.002).astype(np.float32)
+    x = O.f32_to_bf16(rng.normal(size=(rows, k)).astype(np.float32))
+    got = _linear(M, dev, x, codes, scale)
+    keep = np.unique(np.concatenate([np.arange(min(rows, 8)), np.linspace(0, rows - 1, 48, dtype=int),
+                                     np.arange(max(rows - 8, 0), rows)]))
+    runs = [slice(c0, min(c0 + 128, n)) for c0 in (0, n // 256 * 128, (n - 1) // 128 * 128)]
+    want = [O.fp8_linear(x[keep], codes[c], scale[c.start // 128:c.start // 128 + 1]) for c in runs]
+    assert_parity(np.concatenate([got[keep, c] for c in runs], axis=1), np.concatenate(want, axis=1), O,
+                  exact_fraction=0.95)
 
 
 @pytest.mark.parametrize("rows,n,k", [(3, 128, 128), (16, 272, 1152), (40, 2064, 8192), (250, 272, 640), (3, 64, 8320)])
