@@ -1442,7 +1442,14 @@ int glm53_grouped_linear(const void* x, int64_t act_rows, const int32_t* row_ind
   SplitBuf b = carve_split(workspace, act_rows, K);
   HIP_TRY(split(x, act_rows, K, b, st), "split launch");
   GroupedGemmArgs g{};
-  g.fixup = code_flags;  // null: the kernel looks for 0x7F / 0xFF itself
+  g.fixup = code_flags;  // null: the 32-route shape looks for 0x7F / 0xFF itself
+  g.tile_rows = grouped_linear_narrow(routes, descriptors, experts, code_flags != nullptr) ? kGemmMinTileRows
+                                                                                           : kGemmTileRows;
+  if (g.tile_rows == kGemmTileRows && code_flags == nullptr) {
+    int32_t* flag = reinterpret_cast<int32_t*>(static_cast<uint8_t*>(workspace) + split_bytes(act_rows, K));
+    HIP_TRY(launch_scan_480(weight, experts * N * K, flag, true, st), "scan launch");
+    g.fixup = flag;
+  }
   g.a_hi = b.hi;
   g.a_lo = b.lo;
   g.a_scale = b.scale;

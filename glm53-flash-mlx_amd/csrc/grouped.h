@@ -148,8 +148,11 @@ constexpr int kHcBranches = 4;
 hipError_t launch_route_plan(const RoutePlanArgs& a, const SplitArgs* split, hipStream_t st);
 hipError_t launch_split_activations(const SplitArgs& a, hipStream_t st);
 hipError_t launch_grouped_gemm(const GroupedGemmArgs& a, int mode, int64_t descriptors, hipStream_t st);
-// tile_expert / tile_start / tile_len set by the caller; descriptors of up to
-// kGemmTileRows routes; fixup null: the items look for 0x7F / 0xFF themselves
+// tile_expert / tile_start / tile_len set by the caller, descriptors of up to
+// kGemmTileRows routes; tile_rows the shape (kGemmMinTileRows where
+// grouped_linear_narrow, else kGemmTileRows); fixup null (32-route shape
+// only): the items look for 0x7F / 0xFF themselves
+bool grouped_linear_narrow(int64_t routes, int64_t descriptors, int64_t experts, bool flagged);
 hipError_t launch_grouped_linear(const GroupedGemmArgs& a, int64_t descriptors, hipStream_t st);
 // A dense problem (implicit descriptors, expert 0) on the wide shape with
 // `tiles` weight tiles per wavefront: 128 rows x 128 tiles weight rows per item

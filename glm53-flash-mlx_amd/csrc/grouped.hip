@@ -1006,18 +1006,20 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedGemmArgs a) {
   else grouped_gemm_body<MODE, false, GPW>(a, src, ntile, d, lds_dyn);
 }
 
-// The 32-route shape over a caller's own descriptors (glm53_grouped_linear):
-// a descriptor of up to kGemmTileRows routes runs in 32-route parts (one for
-// the tile plan's descriptors, which hold at most 32, so the 64-route shape
-// would carry half its activation rows empty and stream the weights through
-// shallower direct loads).  Bound by the weight stream: 4,096 routes over
-// 288 experts, [4096 x 4096] and [4096 x 2048] in one chain of building
-// blocks, 2,800 -> 2,612 us for the whole chain against the 64-route shape.
+// A caller's own descriptors of up to kGemmTileRows routes
+// (glm53_grouped_linear), on the 32-route shape (GPW = 1: a larger descriptor
+// runs in 32-route parts, each streaming its weights again) or the 64-route
+// one (GPW = 2); grouped_linear_narrow says which.  Bound by the weight
+// stream at few routes per expert, where the 32-route shape streams deeper
+// and past the caches (4,096 routes over 288 experts, [4096 x 4096] and [4096
+// x 2048] in one chain of building blocks, 2,800 -> 2,612 us for the whole
+// chain against the 64-route shape).
 // Weights that come without a code flag (a.fixup null) are looked at as they
-// stream through the registers, 40 VALU instructions per wavefront and stage
-// beside a stage's 8 MFMAs and loads, and an item that met 0x7F / 0xFF runs
-// again in the FIX form; a scan of the bank beforehand read every expert's
-// bytes once more.
+// stream through the 32-route shape's registers, 40 VALU instructions per
+// wavefront and stage beside a stage's 8 MFMAs and loads, and an item that met
+// 0x7F / 0xFF runs again in the FIX form; a scan of the bank beforehand, which
+// the 64-route shape needs, reads every expert's bytes once more.
+template <int GPW>
 __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t lds_dyn[];
   // A caller's descriptors end in unused ones (a tile plan over 288 experts
@@ -1025,8 +1027,7 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) 
   // device knows: workgroup i runs on XCD i % 8, and descriptors go to the
   // XCDs in turn, a.deal at a time (one expert's neighbours share an L2),
   // each with all its column tiles.  In contiguous runs the last XCDs held
-  // the unused ones: the chain above 1,569 us, 1,355 dealt in turn (1, 2 or 4 at
-  // a time alike).
+  // the unused ones: the chain above 1,569 us, 1,355 dealt in turn.
   const int64_t j = blockIdx.x / 8, turn = j / (a.deal * a.n_tiles), in_turn = j % (a.deal * a.n_tiles);
   int64_t ntile = in_turn % a.n_tiles, d = (8 * turn + blockIdx.x % 8) * a.deal + in_turn / a.n_tiles;
   if (d >= a.descriptors) return;
@@ -1034,6 +1035,11 @@ __global__ __launch_bounds__(256) void grouped_linear_kernel(GroupedGemmArgs a) 
   const ItemSource src = item_source(a, a.descriptors, d * a.n_tiles + ntile, true, ntile, d, fix);
   int32_t expert, start, len;
   if (!item_routes<kGemmTileRows>(src, d, expert, start, len)) return;
+  if constexpr (GPW == 2) {
+    if (fix) grouped_gemm_part<GEMM_PLAIN, true, 2, false>(a, src, ntile, expert, start, len, lds_dyn);
+    else grouped_gemm_part<GEMM_PLAIN, false, 2, false>(a, src, ntile, expert, start, len, lds_dyn);
+    return;
+  }
   for (int32_t done = 0; done < len; done += kGemmMinTileRows) {
     if (done > 0) __syncthreads();  // every wavefront has read the part before out of LDS
     const int32_t part = len - done < kGemmMinTileRows ? len - done : kGemmMinTileRows;
@@ -1692,18 +1698,55 @@ hipError_t launch_wide_dense(const GroupedGemmArgs& a, int mode, int tiles, hipS
   return hipGetLastError();
 }
 
+// Whether the descriptors are as many as a tile plan of `rows` routes has
+// (ceil(routes / rows) + experts, the last ones unused).
+static bool plan_of(int64_t rows, int64_t routes, int64_t descriptors, int64_t experts) {
+  return (descriptors - experts) * rows >= routes;
+}
+
+// Whether glm53_grouped_linear takes the 32-route shape: up to `most` routes
+// per expert, beyond which experts fill the 64-route shape's items or have
+// several descriptors, whose weights the 32-route shape streams again for each
+// of them.  A code flag, which spares the 64-route shape its scan of the bank,
+// brings the line down; so do descriptors too few for the plan of 32 routes,
+// which may hold up to 64 routes, two parts of the 32-route shape, and a list
+// without unused ones, which the 64-route shape takes in contiguous runs.
+// Measured (us, 32-route / 64-route shape, 288 experts [3072 x 4096], uniform
+// routing): flagged, plan of 32: 16 routes per expert 644 / 718, 24 738 / 763, 32
+// 1,011 / 902, 96 2,393 / 1,668; plan of 64: 8 592 / 682, 16 644 / 717 (Zipf 774 /
+// 704), 24 724 / 746 (Zipf 919 / 780), 192 4,546 / 2,076; none unused: 2 492 / 520,
+// 8 596 / 634 (Zipf 611 / 598), 12 619 / 653 (Zipf 745 / 654); without a flag,
+// plan of 32: 48 1,382 / 1,611, 64 1,725 / 1,784, 96 2,393 / 2,194; plan of 64: 40
+// 1,281 / 1,317, 48 1,462 / 1,370, 192 4,545 / 2,498.
+bool grouped_linear_narrow(int64_t routes, int64_t descriptors, int64_t experts, bool flagged) {
+  const bool plan32 = plan_of(kGroupedTileRows, routes, descriptors, experts);
+  const bool plan64 = plan_of(kGemmTileRows, routes, descriptors, experts);
+  const int64_t most = flagged ? (plan32 ? 24 : plan64 ? 12 : 6) : plan32 ? 80 : 40;
+  return routes <= most * experts;
+}
+
 hipError_t launch_grouped_linear(const GroupedGemmArgs& a, int64_t descriptors, hipStream_t st) {
   if (descriptors == 0) return hipSuccess;
   if (a.out_row_stride < a.N || a.out_row_stride >= (int64_t{1} << 22)) return hipErrorInvalidValue;
   GroupedGemmArgs g = a;
   g.n_tiles = (a.N + kTileRows - 1) / kTileRows;
   g.descriptors = descriptors;
-  g.deal = descriptors >= 256 ? 4 : 1;  // a few turns at least
+  // Four at a time from 256 descriptors on (us, 4 / 1, 288 experts [3072 x
+  // 4096]: 4 routes per expert 562 / 578, 8 590 / 609, 16 644 / 656); fewer leave
+  // too few turns to even out (64-route shape, 64 experts [4096 x 2048], 24
+  // routes per expert: 146 / 126).
+  // The 64-route shape over a list without unused ones: contiguous runs (288
+  // experts of 16 routes 665, four at a time 724; 64 routes 827 / 880).
+  const bool narrow = a.tile_rows == kGemmMinTileRows;
+  g.deal = descriptors >= 256 ? 4 : 1;
+  if (!narrow && !plan_of(kGemmTileRows, a.routes, descriptors, a.experts)) g.deal = (descriptors + 7) / 8;
   const int64_t turns = (descriptors + 8 * g.deal - 1) / (8 * g.deal);
   const unsigned grid = static_cast<unsigned>(8 * turns * g.deal * g.n_tiles);
-  const size_t lds = gemm_lds_bytes<1>(a.K);
+  const size_t lds = narrow ? gemm_lds_bytes<1>(a.K) : gemm_lds_bytes<2>(a.K);
   if (a.K % kBlock != 0 || a.K <= 0 || lds > 160 * 1024) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(grouped_linear_kernel, dim3(grid), dim3(256), lds, st, g);
+  if (!narrow && (a.tile_rows != kGemmTileRows || a.fixup == nullptr)) return hipErrorInvalidValue;
+  if (narrow) hipLaunchKernelGGL(grouped_linear_kernel<1>, dim3(grid), dim3(256), lds, st, g);
+  else hipLaunchKernelGGL(grouped_linear_kernel<2>, dim3(grid), dim3(256), lds, st, g);
   return hipGetLastError();
 }
 

@@ -415,8 +415,8 @@ int glm53_split_activations(const void* x, int64_t rows, int64_t cols, int64_t x
  * identity) and e(r) comes from the 32-route descriptors.  x bf16
  * [act_rows, K], weight u8 [E, N, K], scale f32 [E, ceil(N/128), K/128],
  * y bf16 [routes, N].  Requires K % 128 == 0 and N % 16 == 0.  code_flags
- * (device int32) as in glm53_bank; NULL has every work item look for 0x7F /
- * 0xFF in the weight rows it reads. */
+ * (device int32) as in glm53_bank; NULL has the call look for 0x7F / 0xFF
+ * itself, as the weights stream by or (many routes per expert) beforehand. */
 size_t glm53_grouped_linear_workspace_bytes(int64_t act_rows, int64_t K);
 int glm53_grouped_linear(const void* x, int64_t act_rows, const int32_t* row_index, int64_t routes,
                          int64_t K, const int32_t* tile_expert, const int32_t* tile_start,

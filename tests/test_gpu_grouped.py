@@ -180,6 +180,46 @@ def test_grouped_linear_callers_descriptors_of_up_to_64_routes(M, O, dev, tile_r
     assert_parity(to_bits(y), O.grouped_linear(x, sorted_e, codes, scale), O, exact_fraction=0.95)
 
 
+@pytest.mark.parametrize("past", [False, True])
+@pytest.mark.parametrize("rows,spare", [(32, True), (64, True), (64, False)])
+@pytest.mark.parametrize("flagged", [False, True])
+@pytest.mark.parametrize("k", [256, 4224])
+def test_grouped_linear_shapes_on_both_sides_of_their_line(O, dev, flagged, rows, spare, past, k):
+    """glm53_grouped_linear takes the 32-route shape up to a number of routes
+    per expert, the 64-route one beyond: with a code flag 24, 12 or 6, without
+    80 or 40, for a tile plan of 32 routes, one of 64, and a list without
+    unused descriptors.  Skewed experts, one without routes, codes 0x7F / 0xFF
+    in a middle and in the last K block, K of 2 and of 33 blocks."""
+    import torch
+
+    experts, n = 5, 144
+    most = {(32, True): (80, 24), (64, True): (40, 12), (64, False): (40, 6)}[rows, spare][flagged]
+    routes = experts * most + past
+    rng = np.random.default_rng(routes + k)
+    counts = [routes // 2, 3, 0, routes // 4]
+    counts.append(routes - sum(counts))
+    sorted_e = np.repeat(np.arange(experts), counts).astype(np.int32)
+    tiles = [(e, sum(counts[:e]) + d, min(rows, c - d)) for e, c in enumerate(counts) for d in range(0, c, rows)]
+    if spare:
+        tiles += [(0, routes, 0)] * (-(-routes // rows) + experts - len(tiles))
+    assert ((len(tiles) - experts) * 32 >= routes, (len(tiles) - experts) * 64 >= routes) == (rows == 32, spare)
+    plan = [torch.tensor(v, dtype=torch.int32, device=dev) for v in zip(*tiles)]
+    codes = rng.integers(0, 127, size=(experts, n, k), dtype=np.int64).astype(np.uint8)
+    codes[0, 17, k // 2], codes[0, n - 1, k - 1], codes[3, 130, k - 128] = 0x7F, 0xFF, 0xFF
+    scale = (rng.uniform(size=(experts, -(-n // 128), k // 128)) * 0.002).astype(np.float32)
+    x = O.f32_to_bf16(rng.normal(size=(routes, k)).astype(np.float32))
+    N = submodule("_native")
+    lib = N.lib()
+    w, s, xd = torch.from_numpy(codes).to(dev), torch.from_numpy(scale).to(dev), from_bits(x, dev)
+    y = torch.zeros((routes, n), dtype=torch.bfloat16, device=dev)
+    flag = N.scan_codes(w) if flagged else None
+    size = lib.glm53_grouped_linear_workspace_bytes(routes, k)
+    ws = N.workspace(size, dev)
+    N.check(lib.glm53_grouped_linear(N.ptr(xd), routes, None, routes, k, *(N.ptr(t) for t in plan), len(tiles), N.ptr(w),
+                                     N.ptr(s), N.ptr(flag), experts, n, N.ptr(y), N.ptr(ws), size, N.stream_handle(dev)))
+    assert_parity(to_bits(y), O.grouped_linear(x, sorted_e, codes, scale), O, exact_fraction=0.95)
+
+
 def _place(bits, offset, dev):
     """Device BF16 copy of `bits` starting `offset` elements into its buffer
     (offset 1 leaves the rows 2-byte aligned only)."""
