@@ -814,6 +814,44 @@ def test_few_tokens_equal_the_direct_loop_bit_for_bit(M, dev, shared_experts, re
         assert torch.equal(moe(x).view(torch.int16), loop(x).view(torch.int16))
 
 
+def test_few_tokens_through_the_op_equal_the_eager_call(M, dev):
+    """Where something acts on the call -- a dispatch mode, a recording
+    profiler, an input that requires a gradient -- the few-token prefill runs
+    as glm53::moe_direct: the eager call's bytes, without a gradient as from
+    the loop.  FakeTensor gets the shape; opcheck validates the op."""
+    import torch
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    seen = []
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            seen.append(func._schema.name)
+            return func(*args, **(kwargs or {}))
+
+    syn = submodule("synthetic")
+    cfg = syn.layer_config(hidden=512, intermediate=256, experts=40, top_k=8, limit=7.0)
+    bank, shared, gate = syn.synth_layer(cfg, seed=91, device=dev)
+    moe = M.SortedGroupedFP8MoE(bank, cfg, gate, shared)
+    x = syn.normal_bf16((1, 9, 512), syn.key(91, "x"), device=dev)
+    want = moe(x)
+    with Mode():
+        got = [moe(x)]
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CPU]) as prof:
+        got.append(moe(x))
+    leaf = x.clone().requires_grad_()
+    with Mode():
+        got.append(moe(leaf))
+    for y in got:
+        assert not y.requires_grad and torch.equal(y.view(torch.int16), want.view(torch.int16))
+    assert seen.count("glm53::moe_direct") == 2
+    assert any(e.name == "glm53::moe_direct" for e in prof.events())
+    with FakeTensorMode(allow_non_fake_inputs=True) as fake:
+        assert moe(fake.from_tensor(x)).shape == x.shape
+    torch.library.opcheck(torch.ops.glm53.moe_direct, (x, moe._op_key), test_utils=("test_schema", "test_faketensor"))
+
+
 def test_custom_ops_compile_without_graph_breaks(M, dev):
     """The MoE modules call the glm53 custom ops: torch.compile with
     fullgraph=True (no graph break allowed) traces decode and prefill, and

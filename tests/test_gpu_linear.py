@@ -2,6 +2,7 @@
 
 from __future__ import annotations
 
+import ctypes
 import hashlib
 import json
 from pathlib import Path
@@ -112,6 +113,69 @@ def test_dense_tiles_ragged_edges_match_oracle(M, O, dev, rows, k, with_480):
     scale = (rng.uniform(size=(-(-n // 128), k // 128)) * 0.002).astype(np.float32)
     x = O.f32_to_bf16(rng.normal(size=(rows, k)).astype(np.float32))
     assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
+
+
+@pytest.mark.parametrize("rows,k", [(17, 3712), (17, 9344), (250, 4224), (250, 9344), (499, 4224), (499, 3712),
+                                    (999, 4224), (999, 3712)])
+def test_few_row_tiles_over_long_k_match_oracle(M, O, dev, rows, k):
+    """16 x 16, 16 x 32, 32 x 32 and 32 x 64 tiles through more than one turn
+    of their K loop and several folds, the last step of K whole or ragged over
+    the wavefronts; 0x7F / 0xFF in a middle and in the last K block, found
+    without a code flag."""
+    rng = np.random.default_rng(rows + k)
+    n = 272
+    codes = (rng.integers(0, 0x7F, size=(n, k)) | (rng.integers(0, 2, size=(n, k)) << 7)).astype(np.uint8)
+    scale = (rng.uniform(size=(-(-n // 128), k // 128)) * 0.002).astype(np.float32)
+    x = O.f32_to_bf16(rng.normal(size=(rows, k)).astype(np.float32))
+    assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
+    codes[3, k // 2], codes[100, k - 1], codes[n - 1, k - 128] = 0x7F, 0xFF, 0x7F
+    assert_parity(_linear(M, dev, x, codes, scale), O.fp8_linear(x, codes, scale), O, exact_fraction=0.95)
+
+
+@pytest.mark.parametrize("marked", ["none", "gate_proj", "up_proj"])
+@pytest.mark.parametrize("rows", [33, 150, 300])
+def test_mlp_over_long_k_equals_its_parts_and_the_oracle(M, O, dev, rows, marked):
+    """The 16 x 32, 32 x 32 and 32 x 64 SwiGLU tiles through 33 K blocks: the
+    bytes of the projections called in turn, with the code flags and without
+    (0x7F / 0xFF in a middle and in the last K block, looked for), and the
+    oracle's chain."""
+    import torch
+
+    hidden, inter, limit = 4224, 640, 2.0
+    gen = torch.Generator().manual_seed(rows)
+    mlp = M.ClampedMLP(hidden, inter, limit, device=dev)
+    for name in ("gate_proj", "up_proj", "down_proj"):
+        proj = getattr(mlp, name)
+        codes = torch.randint(0, 0x7F, tuple(proj.weight.shape), generator=gen, dtype=torch.uint8)
+        codes |= torch.randint(0, 2, tuple(codes.shape), generator=gen, dtype=torch.uint8) << 7
+        if name == marked:
+            codes[7, hidden // 2], codes[-1, -1], codes[200, -128] = 0x7F, 0xFF, 0x7F
+        proj.weight.copy_(codes)
+        proj.weight_scale_inv.copy_(torch.rand(tuple(proj.weight_scale_inv.shape), generator=gen) * 0.002)
+    x = torch.randn((rows, hidden), generator=gen).to(dev, torch.bfloat16)
+    y = mlp(x)
+    parts = mlp.down_proj(M.swiglu(mlp.gate_proj(x), mlp.up_proj(x), limit))
+    assert mlp._one_call(x) and torch.equal(y.view(torch.int16), parts.view(torch.int16))
+    N = submodule("_native")
+    plain = mlp.as_c_struct()
+    for linear in (plain.gate, plain.up, plain.down):
+        linear.code_flags = None
+    size = N.lib().glm53_mlp_workspace_bytes(rows, hidden, inter)
+    ws, looked = N.workspace(size, dev), torch.empty_like(y)
+    N.check(N.lib().glm53_mlp(ctypes.byref(plain), limit, N.ptr(x), rows, N.ptr(looked), N.ptr(ws), size,
+                              N.stream_handle(dev)))
+    assert torch.equal(looked.view(torch.int16), y.view(torch.int16))
+    at = [(p.weight.cpu().numpy(), p.weight_scale_inv.cpu().numpy()) for p in (mlp.gate_proj, mlp.up_proj, mlp.down_proj)]
+    bits = to_bits(x)
+    h = O.swiglu(O.fp8_linear(bits, *at[0]), O.fp8_linear(bits, *at[1]), limit)
+    want = O.fp8_linear(h, *at[2])
+    assert_parity(to_bits(y), want, O, elementwise=False)
+    # An output of one step (2^-7) apart, plus what the hidden values bring:
+    # about 2.4% of them are a step off (1.2% of gate and of up each), so the
+    # sum is off by sqrt(0.024) 2^-7 = 1.2e-3 of the outputs' RMS (one
+    # deviation); six of them.
+    got, want = O.bf16_to_f32(to_bits(y)).astype(np.float64), O.bf16_to_f32(want).astype(np.float64)
+    assert (np.abs(got - want) <= 2.0 ** -7 * np.abs(want) + 7.3e-3 * np.sqrt(np.mean(want ** 2))).all()
 
 
 @pytest.mark.parametrize("with_480", [False, True])

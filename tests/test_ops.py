@@ -38,6 +38,16 @@ def test_fake_shapes_and_dtypes():
         assert torch.ops.glm53.moe_prefill(x, 7, ids, sc).shape == x.shape
 
 
+def test_moe_direct_is_registered_with_its_shape():
+    from torch._subclasses.fake_tensor import FakeTensorMode
+
+    submodule("ops")
+    with FakeTensorMode():
+        x = torch.empty((2, 5, 256), dtype=torch.bfloat16)
+        y = torch.ops.glm53.moe_direct(x, 7)
+        assert y.shape == x.shape and y.dtype == x.dtype
+
+
 def test_unknown_owner_raises():
     ops = submodule("ops")
     with pytest.raises(RuntimeError, match="no longer exists"):
