@@ -24,14 +24,17 @@ DECODE_TOP_K = 8
 PREFILL_TILE_ROWS = 8
 
 
-def _hooked(module) -> bool:
-    """Whether calling `module` would run more than its class's forward."""
-    return bool(module._forward_hooks or module._forward_pre_hooks or module._backward_hooks
-                or module._backward_pre_hooks or "forward" in module.__dict__
-                or torch.nn.modules.module._global_forward_hooks
-                or torch.nn.modules.module._global_forward_pre_hooks
-                or torch.nn.modules.module._global_backward_hooks
-                or torch.nn.modules.module._global_backward_pre_hooks)
+def _hooked(*modules) -> bool:
+    """Whether calling one of `modules` would run more than its class's forward."""
+    every = torch.nn.modules.module
+    if (every._global_forward_hooks or every._global_forward_pre_hooks or every._global_backward_hooks
+            or every._global_backward_pre_hooks):
+        return True
+    for m in modules:
+        if (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks
+                or "forward" in m.__dict__):
+            return True
+    return False
 
 
 def _scale_shape(out_features: int, in_features: int) -> tuple[int, int]:
@@ -124,12 +127,6 @@ class BlockFP8Linear(torch.nn.Module):
             self._code_flags = (stamp, N.scan_codes(self.weight))
         return self._code_flags[1]
 
-    def widths_hold(self) -> bool:
-        """Whether in_features and out_features, which as_c_struct passes on,
-        are the weight's: a call on the tensors goes by the weight's shape
-        alone, also after a weight of another size took its place."""
-        return self.weight.shape == (self.out_features, self.in_features)
-
     def as_c_struct(self) -> N.Linear:
         return N.Linear(self.weight.data_ptr(), self.weight_scale_inv.data_ptr(), self.out_features, self.in_features,
                         self.code_flags().data_ptr())
@@ -155,29 +152,34 @@ class ClampedMLP(torch.nn.Module):
     def _one_call(self, x) -> bool:
         """Whether glm53_mlp stands for gate_proj, up_proj, swiglu and
         down_proj called in turn on x: two or more bf16 rows, plain
-        projections (no bias, no hooks) of widths the MFMA path takes, in
-        buffers it can take by their addresses, and nothing acting on the
+        projections (no bias, no hooks) of widths the MFMA path takes and
+        that their attributes, which as_c_struct passes on, state, in buffers
+        it can take by their addresses, and nothing acting on the
         projections' ops."""
-        rows = x.numel() // max(x.shape[-1], 1)
-        if type(self) is not ClampedMLP or rows < 2 or x.dtype != torch.bfloat16 or not x.is_cuda:
+        hidden = x.shape[-1]
+        if type(self) is not ClampedMLP or x.dtype != torch.bfloat16 or not x.is_cuda:
             return False
-        projections = (self.gate_proj, self.up_proj, self.down_proj)
-        if any(type(p) is not BlockFP8Linear or p.bias is not None or _hooked(p) or not p.widths_hold()
-               for p in projections):
+        if hidden == 0 or hidden % BLOCK_SIZE or x.numel() < 2 * hidden:
             return False
-        gate, up, down = (p.weight for p in projections)
-        scales = tuple(p.weight_scale_inv for p in projections)
-        inter, hidden = gate.shape
-        if x.shape[-1] != hidden or hidden % BLOCK_SIZE or inter % BLOCK_SIZE:
+        gate, up, down = self.gate_proj, self.up_proj, self.down_proj
+        if type(gate) is not BlockFP8Linear or type(up) is not BlockFP8Linear or type(down) is not BlockFP8Linear:
             return False
-        if up.shape != (inter, hidden) or down.shape != (hidden, inter):
+        inter = gate.out_features
+        if inter == 0 or inter % BLOCK_SIZE or _hooked(gate, up, down):
             return False
-        table = _scale_shape(inter, hidden)
-        return (tuple(s.shape for s in scales) == (table, table, table[::-1])
-                and all(s.dtype == torch.float32 for s in scales)
-                and all(w.dtype == torch.uint8 and w.data_ptr() % 16 == 0 for w in (gate, up, down))
-                and all(t.is_contiguous() and t.device == x.device for t in (gate, up, down, *scales))
-                and _ops.direct(x, gate, up, down, *scales))
+        device, tensors = x.device, [x]
+        for p, rows, cols in ((gate, inter, hidden), (up, inter, hidden), (down, hidden, inter)):
+            w, s = p.weight, p.weight_scale_inv
+            if p.bias is not None or p.out_features != rows or p.in_features != cols or w.shape != (rows, cols):
+                return False
+            if s.shape != (rows // BLOCK_SIZE, cols // BLOCK_SIZE) or w.dtype != torch.uint8 or s.dtype != torch.float32:
+                return False
+            if w.device != device or s.device != device or not (w.is_contiguous() and s.is_contiguous()):
+                return False
+            if w.data_ptr() % 16:
+                return False
+            tensors += (w, s)
+        return _ops.direct(*tensors)
 
     def forward(self, x):
         # One call of four launches where the four calls took nine: x split

@@ -315,34 +315,41 @@ class SortedGroupedFP8MoE(PackedFP8MoE):
         limit = float(cfg.swiglu_limit)
         if type(self) is not SortedGroupedFP8MoE or type(gate) is not Float32Gate or _hooked(gate):
             return False
-        if x.dtype != torch.bfloat16 or x.shape[-1] != bank.hidden_size or torch.compiler.is_compiling():
+        hidden, inter, experts = bank.hidden_size, bank.intermediate_size, bank.expert_count
+        if x.dtype != torch.bfloat16 or x.shape[-1] != hidden or torch.compiler.is_compiling():
             return False
         if gate.top_k != cfg.num_experts_per_tok or tokens * gate.top_k > _DIRECT_PLAN_ROUTES:
             return False
-        if bank.hidden_size % BLOCK_SIZE or bank.intermediate_size % BLOCK_SIZE or bank.expert_count > PLAN_MAX_EXPERTS:
+        if hidden % BLOCK_SIZE or inter % BLOCK_SIZE or experts > PLAN_MAX_EXPERTS:
             return False
         if self._expert_views[0].limit != limit or not self._views_are_the_banks():
             return False
         weights = [bank.gate_up_weight, bank.down_weight]
-        tables = [bank.gate_up_scale_inv, bank.down_scale_inv, gate.weight, gate.e_score_correction_bias]
-        shapes = [(gate.weight, (bank.expert_count, bank.hidden_size)),
-                  (gate.e_score_correction_bias, (bank.expert_count,))]
+        router, bias = gate.weight, gate.e_score_correction_bias
+        tables = [bank.gate_up_scale_inv, bank.down_scale_inv, router, bias]
+        if router.shape != (experts, hidden) or bias.shape != (experts,):
+            return False
         if shared is not None:
-            if type(shared) is not ClampedMLP or _hooked(shared) or shared.limit != limit:
+            if type(shared) is not ClampedMLP or shared.limit != limit:
                 return False
-            width = shared.gate_proj.weight.shape[0]
-            if width % BLOCK_SIZE:
+            gate_proj, up_proj, down_proj = shared.gate_proj, shared.up_proj, shared.down_proj
+            if _hooked(shared, gate_proj, up_proj, down_proj):
                 return False
-            for proj, shape in ((shared.gate_proj, (width, bank.hidden_size)),
-                                (shared.up_proj, (width, bank.hidden_size)),
-                                (shared.down_proj, (bank.hidden_size, width))):
-                if type(proj) is not BlockFP8Linear or _hooked(proj) or proj.bias is not None or not proj.widths_hold():
+            if any(type(p) is not BlockFP8Linear for p in (gate_proj, up_proj, down_proj)):
+                return False
+            width = gate_proj.out_features
+            if width == 0 or width % BLOCK_SIZE:
+                return False
+            for proj, shape in ((gate_proj, (width, hidden)), (up_proj, (width, hidden)), (down_proj, (hidden, width))):
+                w, s = proj.weight, proj.weight_scale_inv
+                # as_c_struct passes the features on
+                if proj.bias is not None or (proj.out_features, proj.in_features) != shape:
                     return False
-                weights.append(proj.weight)
-                tables.append(proj.weight_scale_inv)
-                shapes += [(proj.weight, shape), (proj.weight_scale_inv, _scale_shape(*shape))]
-        return (all(t.shape == shape for t, shape in shapes)
-                and all(t.dtype == torch.uint8 and t.data_ptr() % 16 == 0 for t in weights)
+                if w.shape != shape or s.shape != _scale_shape(*shape):
+                    return False
+                weights.append(w)
+                tables.append(s)
+        return (all(t.dtype == torch.uint8 and t.data_ptr() % 16 == 0 for t in weights)
                 and all(t.dtype == torch.float32 for t in tables)
                 and all(t.is_contiguous() and t.device == x.device for t in weights + tables))
 
