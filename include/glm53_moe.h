@@ -169,12 +169,14 @@ int glm53_e4m3_scan_codes(const uint8_t* codes, int64_t n, int32_t* flag, void* 
  * block_fp8_linear -- replaces fp8.py:254-299 `block_fp8_linear`
  * (kernels fp8.py:41-116).  y[m, n] = T(sum_k x[m,k] * E4M3(w[n,k]) *
  * s[n/128, k/128]).  x bf16 [M, K], y bf16 [M, N].  M == 1 runs the
- * streaming GEMV; M > 1 with K % 128 == 0 runs the FP8 MFMA GEMM and needs
- * `workspace` of glm53_fp8_linear_workspace_bytes(M, N, K) bytes (may be
- * NULL when that is 0).  code_flags (device int32 from glm53_e4m3_scan_codes,
+ * streaming GEMV; M > 1 with K % 128 == 0 and N % 16 == 0 runs an FP8
+ * MFMA product with `workspace` of glm53_fp8_linear_workspace_bytes(M, N, K)
+ * bytes, NULL where glm53_fp8_linear_workspace_needed gives 0 (a NULL or
+ * smaller workspace elsewhere: the generic kernel).  code_flags (device int32 from glm53_e4m3_scan_codes,
  * may be NULL) lets both paths use the hardware E4M3 decode when the weight
- * holds no 0x7F / 0xFF code; NULL keeps the exact software decode (M == 1)
- * or scans the weight first (M > 1).
+ * holds no 0x7F / 0xFF code; NULL keeps the exact software decode (M == 1),
+ * and has M > 1 look for the codes as the weight streams by (few rows) or
+ * scan it first.
  * ---------------------------------------------------------------------- */
 size_t glm53_fp8_linear_workspace_bytes(int64_t M, int64_t N, int64_t K);
 /* The same for this x: 0 where the call splits the activations inside the
